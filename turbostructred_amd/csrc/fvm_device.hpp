@@ -27,39 +27,38 @@ struct BCDev {
 };
 
 // ---- fast reciprocal / square root ---------------------------------------------------------
-// Hardware estimates refined by Newton steps (double) or used directly (float).  Results are
-// within an ulp or two of the correctly rounded value; the parity tolerance is 1e-12.  Only for
-// operands well inside the normal range (densities, sound speeds, mass fluxes): the estimate
-// overflows for subnormal divisors.
+// Hardware estimates (good to about 2^-23 in double) refined by the shortest chain that reaches
+// working precision, or used directly (float).  Results are within an ulp or two of the correctly
+// rounded value; the parity tolerance is 1e-12.  Only for operands well inside the normal range
+// (densities, sound speeds, mass fluxes): the estimate overflows for subnormal divisors.
+//   reciprocal: one cubic step r (1 + e + e^2), e = 1 - x r, leaves e^3 ~ 2^-69 (4 instructions;
+//               two quadratic steps take 5 and a longer chain);
+//   quotient:   one quadratic step on the reciprocal (2^-46), then the residual correction of the
+//               quotient itself, whose error is the product of both (6 instructions against 8);
+//   root:       one Goldschmidt step (2^-45), then one residual correction.
 __device__ inline double frcp(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = __builtin_fma(-x, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-x, r, 1.0);
-    return __builtin_fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 __device__ inline float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ inline double fdiv(double a, double b) {
-    double r = frcp(b);
-    double q = a * r;
-    double e = __builtin_fma(-b, q, a);
-    return __builtin_fma(e, r, q);
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 __device__ inline float fdiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-// sqrt from the reciprocal-square-root estimate with two Newton-Raphson corrections (no
-// rescaling: for normal-range arguments; 0 maps to 0, negative arguments to NaN)
+// for normal-range arguments and zero; negative arguments give NaN.  The addend keeps the
+// estimate of a zero finite (its root comes out as 1e-150) and leaves every other argument as it is,
+// in one instruction where selecting the zero took three.
 __device__ inline double fsqrt(double x) {
-    double r = __builtin_amdgcn_rsq(x);
+    x += 1e-300;
+    const double r = __builtin_amdgcn_rsq(x);
     double y = x * r;
-    double h = 0.5 * r;
-    double e = __builtin_fma(-h, y, 0.5);
-    y = __builtin_fma(y, e, y);
-    h = __builtin_fma(h, e, h);
-    double d = __builtin_fma(-y, y, x);
-    y = __builtin_fma(d, h, y);
-    d = __builtin_fma(-y, y, x);
-    y = __builtin_fma(d, h, y);
-    return x == 0.0 ? 0.0 : y;
+    const double h = 0.5 * r;
+    y = __builtin_fma(y, __builtin_fma(-h, y, 0.5), y);
+    return __builtin_fma(__builtin_fma(-y, y, x), h, y);
 }
 __device__ inline float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
@@ -71,6 +70,22 @@ __device__ inline double vmin(double a, double b) { return __builtin_fmin(a, b);
 __device__ inline float vmin(float a, float b) { return __builtin_fminf(a, b); }
 __device__ inline double vabs(double a) { return __builtin_fabs(a); }
 __device__ inline float vabs(float a) { return __builtin_fabsf(a); }
+
+// The same on values that come straight from memory: the compiler would first pass each of them
+// through a maximum with itself, in case it is a signalling NaN (25 extra instructions per row of a
+// 2-D reconstruction); v_max_f64 and v_min_f64 quiet those by themselves.
+__device__ inline double vmax_mem(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline double vmin_mem(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline float vmax_mem(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ inline float vmin_mem(float a, float b) { return __builtin_fminf(a, b); }
 
 // smallest divisor the limiter uses: well inside the normal range, where the reciprocal
 // estimate and its Newton steps are accurate
@@ -191,7 +206,10 @@ __device__ inline void reconstruct(const R (&c)[NV], const R (&nb)[2 * ND][NV],
             // (c + g.p) - c: the two differ by an ulp of c, and so do the face values.  A
             // variable without spread has d_a = 0 and keeps its cell value, as the reference's
             // spread test (Limiters.h:50) gives.
-            R d[ND], dmax = R(0);
+            // The largest |d_a| starts at a floor, so that the divisor of a variable that is
+            // constant up to round-off stays in the reciprocal's range; its face values move by
+            // less than the floor.
+            R d[ND], dmax = tiny_divisor<R>();
 #pragma unroll
             for (int a = 0; a < ND; a++) {
                 d[a] = (nb[2 * a + 1][v] - nb[2 * a][v]) * (geo.rc[a] * geo.hh[a]);
@@ -200,16 +218,11 @@ __device__ inline void reconstruct(const R (&c)[NV], const R (&nb)[2 * ND][NV],
             R umax = c[v], umin = c[v];
 #pragma unroll
             for (int n = 0; n < 2 * ND; n++) {
-                umax = vmax(umax, nb[n][v]);
-                umin = vmin(umin, nb[n][v]);
+                umax = vmax_mem(umax, nb[n][v]);
+                umin = vmin_mem(umin, nb[n][v]);
             }
             const R hi = umax - c[v], lo = c[v] - umin;
-            const R m = vmin(hi, lo);
-            R lim = R(1);
-            // a divisor below the floor (a variable constant up to round-off) is raised to it:
-            // the reciprocal estimate stays in range, the quotient below 1, and the face values
-            // move by less than the floor
-            if (m < dmax) lim = fdiv(m, vmax(dmax, tiny_divisor<R>()));
+            const R lim = vmin(fdiv(vmin(hi, lo), dmax), R(1));
 #pragma unroll
             for (int a = 0; a < ND; a++) {
                 const R t = lim * d[a];
@@ -386,59 +399,49 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[NV], const R (&UR)
 
 // HLLC flux (Toro, Riemann Solvers and Numerical Methods for Fluid Dynamics, 3rd ed.,
 // sec. 10.4, eqs. 10.37-10.39) with Davis wave-speed bounds (eq. 10.48); lam = max(|SL|,|SR|).
-// Extension with no counterpart in the reference.  Branch-free: the upwind side of the contact
-// is selected first, then its flux and star state are evaluated once.
+// Extension with no counterpart in the reference.  Branch-free: the upwind side K of the contact is
+// selected first, then the flux of the state the face lies in is formed once.  With w = S_K - u_K
+// and r = 1 / (S_K - S*), the star state's density is rho_K w r, its tangential momentum m_t w r, its
+// pressure p* = p_K + rho_K w (S* - u_K) and its energy (w E_K - p_K u_K + p* S*) r (the jump
+// conditions across S_K), and its flux needs no more than that: (rho, m_t) S*, rho S*^2 + p*,
+// S* (E + p*).  A supersonic side takes its own velocity, pressure and energy in the places of
+// the star's.  (Against F_K + S_K (U* - U_K), which needs the whole flux of side K and
+// its velocities first: about 50 instructions fewer per face in double.)
 template <int D, typename R>
 __device__ inline void hllc_flux(R gamma, const R (&UL)[NV], const R (&UR)[NV], R (&F)[NV],
                                  R& lam) {
     const IdealGasEOS<R> eos(gamma);
-    R il = frcp(UL[0]), ir = frcp(UR[0]);
-    R vl[3] = {UL[1] * il, UL[2] * il, UL[3] * il};
-    R vr[3] = {UR[1] * ir, UR[2] * ir, UR[3] * ir};
-    R pl = eos.PressureOfEnergyDensity(internal_energy(UL[4], R(0.5) * UL[0] * (vl[0] * vl[0] + vl[1] * vl[1] + vl[2] * vl[2]), UL));
-    R pr = eos.PressureOfEnergyDensity(internal_energy(UR[4], R(0.5) * UR[0] * (vr[0] * vr[0] + vr[1] * vr[1] + vr[2] * vr[2]), UR));
-    R al = eos.SoundSpeedOfPressure(pl, il), ar = eos.SoundSpeedOfPressure(pr, ir);
-    R ul = vl[D], ur = vr[D];
-    R SL = __builtin_fmin(ul - al, ur - ar);
-    R SR = __builtin_fmax(ul + al, ur + ar);
-    R ml = UL[0] * (SL - ul), mr = UR[0] * (SR - ur);
-    R Ss = fdiv(pr - pl + ul * ml - ur * mr, ml - mr);
-    lam = __builtin_fmax(__builtin_fabs(SL), __builtin_fabs(SR));
-    bool left = Ss >= R(0);
-    R U[NV], vel[3];
-#pragma unroll
-    for (int i = 0; i < NV; i++) U[i] = left ? UL[i] : UR[i];
-#pragma unroll
-    for (int i = 0; i < 3; i++) vel[i] = left ? vl[i] : vr[i];
-    R S = left ? SL : SR;
-    R un = left ? ul : ur, p = left ? pl : pr, ik = left ? il : ir;
-    R m = left ? ml : mr;
-    R Fk[NV];
-    Fk[0] = U[0] * un;
-    Fk[1] = Fk[0] * vel[0];
-    Fk[2] = Fk[0] * vel[1];
-    Fk[3] = Fk[0] * vel[2];
-    Fk[1 + D] += p;
-    Fk[4] = un * (U[4] + p);
-    bool supersonic = left ? (S >= R(0)) : (S <= R(0));
-    // supersonic side: the star correction is multiplied by zero (and its operands made finite),
-    // which gives Fk exactly with two selects instead of five
-    // m / (S - Ss) and p / m from one reciprocal of m (S - Ss), which is positive on a
-    // subsonic side (S < 0 <= Ss with m = rho (S - u) < 0, or the mirror case)
-    const R dS = S - Ss;
-    const R rmd = frcp(supersonic ? R(1) : m * dS);
-    R coef = supersonic ? R(0) : m * m * rmd;
-    R Sc = supersonic ? R(0) : S;
-    R Us[NV];
-    Us[0] = coef;
-    Us[1] = coef * vel[0];
-    Us[2] = coef * vel[1];
-    Us[3] = coef * vel[2];
-    Us[1 + D] = coef * Ss;
-    R pm = supersonic ? R(0) : p * dS * rmd;
-    Us[4] = coef * (U[4] * ik + (Ss - un) * (Ss + pm));
-#pragma unroll
-    for (int i = 0; i < NV; i++) F[i] = Fk[i] + Sc * (Us[i] - U[i]);
+    constexpr int T1 = D == 0 ? 2 : 1, T2 = D == 2 ? 2 : 3;  // tangential momenta
+    const R il = frcp(UL[0]), ir = frcp(UR[0]);
+    const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
+    const R kl = R(0.5) * il * (UL[1] * UL[1] + UL[2] * UL[2] + UL[3] * UL[3]);
+    const R kr = R(0.5) * ir * (UR[1] * UR[1] + UR[2] * UR[2] + UR[3] * UR[3]);
+    const R pl = eos.PressureOfEnergyDensity(internal_energy(UL[4], kl, UL));
+    const R pr = eos.PressureOfEnergyDensity(internal_energy(UR[4], kr, UR));
+    const R al = eos.SoundSpeedOfPressure(pl, il), ar = eos.SoundSpeedOfPressure(pr, ir);
+    const R SL = vmin(ul - al, ur - ar);
+    const R SR = vmax(ul + al, ur + ar);
+    lam = vmax(vabs(SL), vabs(SR));
+    const R wl = SL - ul, wr = SR - ur;
+    const R ml = UL[0] * wl, mr = UR[0] * wr;
+    const R Ss = fdiv(pr - pl + ul * ml - ur * mr, ml - mr);
+    const bool left = Ss >= R(0);
+    const R S = left ? SL : SR, w = left ? wl : wr, m = left ? ml : mr;
+    const R rho = left ? UL[0] : UR[0], un = left ? ul : ur, p = left ? pl : pr, E = left ? UL[4] : UR[4];
+    const R t1 = left ? UL[T1] : UR[T1], t2 = left ? UL[T2] : UR[T2];
+    const bool supersonic = left ? (S >= R(0)) : (S <= R(0));
+    // on a subsonic side S - S* is not zero (S < 0 <= S*, or the mirror case)
+    const R r = frcp(supersonic ? R(1) : S - Ss);
+    const R ps = p + m * (Ss - un);
+    const R Es = (w * E - p * un + ps * Ss) * r;
+    const R c = supersonic ? R(1) : w * r;
+    const R uf = supersonic ? un : Ss, pf = supersonic ? p : ps, Ef = supersonic ? E : Es;
+    const R q = c * uf;
+    F[0] = rho * q;
+    F[T1] = t1 * q;
+    F[T2] = t2 * q;
+    F[1 + D] = F[0] * uf + pf;
+    F[4] = uf * (Ef + pf);
 }
 
 // ---- exact Riemann solver (always double) -----------------------------------------------------
@@ -767,16 +770,13 @@ __device__ inline R face_eigen(R gamma, const R (&UL)[NV], const R (&UR)[NV]) {
         return __builtin_fabs(v[D]) + fsqrt(gm1 * h - phi2);
     } else if constexpr (FLUX == FX_HLLC) {
         const IdealGasEOS<R> eos(gamma);
-        R il = frcp(UL[0]), ir = frcp(UR[0]);
-        R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-        R vl[3] = {UL[1] * il, UL[2] * il, UL[3] * il};
-        R vr[3] = {UR[1] * ir, UR[2] * ir, UR[3] * ir};
-        R pl = eos.PressureOfEnergyDensity(internal_energy(UL[4], R(0.5) * UL[0] * (vl[0] * vl[0] + vl[1] * vl[1] + vl[2] * vl[2]), UL));
-        R pr = eos.PressureOfEnergyDensity(internal_energy(UR[4], R(0.5) * UR[0] * (vr[0] * vr[0] + vr[1] * vr[1] + vr[2] * vr[2]), UR));
-        R al = eos.SoundSpeedOfPressure(pl, il), ar = eos.SoundSpeedOfPressure(pr, ir);
-        R SL = __builtin_fmin(ul - al, ur - ar);
-        R SR = __builtin_fmax(ul + al, ur + ar);
-        return __builtin_fmax(__builtin_fabs(SL), __builtin_fabs(SR));
+        const R il = frcp(UL[0]), ir = frcp(UR[0]);
+        const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
+        const R kl = R(0.5) * il * (UL[1] * UL[1] + UL[2] * UL[2] + UL[3] * UL[3]);
+        const R kr = R(0.5) * ir * (UR[1] * UR[1] + UR[2] * UR[2] + UR[3] * UR[3]);
+        const R al = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UL[4], kl, UL)), il);
+        const R ar = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UR[4], kr, UR)), ir);
+        return vmax(vabs(vmin(ul - al, ur - ar)), vabs(vmax(ul + al, ur + ar)));
     } else {
         R F[NV], lam;
         godunov_flux<D, R>(gamma, UL, UR, F, lam);

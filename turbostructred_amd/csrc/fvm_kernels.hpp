@@ -235,9 +235,10 @@ __device__ __forceinline__ T ld_geo_uniform(const T* p, int i) {
 
 
 // V/SR of one cell; a NaN or negative spectral radius (non-physical state) becomes 0 so that
-// the step fails with dt = 0 instead of silently skipping the cell in the minimum.
+// the step fails with dt = 0 instead of silently skipping the cell in the minimum.  A cell whose
+// spectral radius is zero (or below the reciprocal's range) bounds nothing.
 __device__ inline double dt_candidate(double vol, double sr) {
-    double q = vol / sr;
+    const double q = (sr >= 0.0 && sr < 1e-290) ? __builtin_inf() : fdiv(vol, sr);
     return (q > 0.0) ? q : 0.0;
 }
 
