@@ -32,7 +32,20 @@ Key key_of(const ts_config& c) {
 }  // namespace
 
 namespace tsr {
-int tuned_rows_per_tile(const ts_config& c, long long slots) {
+// Time of a march over `tiles` tiles of ty rows, in arbitrary units.  A tile is one wavefront's
+// (3-D: one workgroup's) march of ty rows plus two warm-up rows; `units` SIMDs (3-D: CUs) hold `occ`
+// of them each.  A row of one wavefront is a serial chain that leaves the SIMD idle most of
+// the time, so w wavefronts on a SIMD take w + 1.5 rows' issue time for a row each (2-D FP64 stage 1,
+// measured per row: 2.6 us alone, 3.4 us with two, 4.7 us with three).  Whole rounds run
+// full SIMDs; the last one runs as long as its fullest SIMD.
+double march_cost(long long tiles, int ty, long long units, int occ) {
+    const long long slots = units * occ, full = tiles / slots, rest = tiles % slots;
+    double c = full * (occ + 1.5);
+    if (rest) c += double((rest + units - 1) / units) + 1.5;
+    return c * (ty + 2);
+}
+
+int tuned_rows_per_tile(const ts_config& c, long long units, int occ) {
     if (c.ndims == 1) return 1;
     {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -41,23 +54,17 @@ int tuned_rows_per_tile(const ts_config& c, long long slots) {
     }
     const long long strips = (c.nx + 59) / 60;
     const long long zb = c.ndims == 3 ? (c.nz + 5) / 6 : 1;  // z blocks of a 3-D tile column
-    if (slots <= 0) {
+    if (units <= 0 || occ <= 0) {
         // no occupancy known: enough tiles to fill 256 CUs several times over, at most 32 rows
         long long rows = (long long)c.ny * zb;
         int ty = 32;
         while (ty > 4 && strips * ((rows + ty - 1) / ty) < 4096) ty /= 2;
         return ty;
     }
-    // A tile is one wavefront's (3-D: one workgroup's) march of ty rows plus two warm-up rows,
-    // and tiles run in rounds of `slots`.  The time goes as rounds * (ty + 2): pick the ty that
-    // minimises it, so that the last round is not a mostly empty one.
-    int best = 4;
+    int best = 1;
     double best_cost = 1e300;
-    const int hi = c.ny < 256 ? c.ny : 256;
-    for (int ty = 4; ty <= (hi > 4 ? hi : 4); ty++) {
-        long long tiles = strips * zb * ((c.ny + ty - 1) / ty);
-        long long rounds = (tiles + slots - 1) / slots;
-        double cost = double(rounds) * (ty + 2);
+    for (int ty = 1; ty <= std::min(c.ny, 256); ty++) {
+        const double cost = march_cost(strips * zb * ((c.ny + ty - 1) / ty), ty, units, occ);
         if (cost < best_cost) {
             best_cost = cost;
             best = ty;
@@ -90,13 +97,13 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
         ts_ctx* c = nullptr;
         if (ts_create(cfg, &c) == TS_OK) {
             const int m = c->ty;
-            cands = {m, m > 5 ? m - m / 4 : 4, m + m / 4 + 1};
+            cands = {m, m > 1 ? m - (m + 3) / 4 : 1, m + m / 4 + 1};
             const long long strips = c->nstrips, tiles_m = c->ntiles;
             const long long zb = cfg->ndims == 3 ? (cfg->nz + tsd::ZOUT - 1) / tsd::ZOUT : 1;
             // slots implied by the model's choice: its tile count rounded up to a whole round
             for (long long rounds = 1; rounds <= 2; rounds++) {
                 const long long target = tiles_m * rounds;
-                for (int ty = 4; ty <= 256; ty++)
+                for (int ty = 1; ty <= 256; ty++)
                     if (strips * zb * ((cfg->ny + ty - 1) / ty) <= target) {
                         cands.push_back(ty);
                         break;
@@ -105,11 +112,11 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
             ts_destroy(c);
         }
     }
-    for (int ty : {4, 8, 16, 24, 32, 48, 64}) cands.push_back(ty);
+    for (int ty : {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48, 64}) cands.push_back(ty);
     const int ymax = cfg->ny;
     std::vector<int> uniq;
     for (int ty : cands)
-        if (ty >= 1 && ty <= std::max(ymax, 4) && std::find(uniq.begin(), uniq.end(), ty) == uniq.end()) uniq.push_back(ty);
+        if (ty >= 1 && ty <= ymax && std::find(uniq.begin(), uniq.end(), ty) == uniq.end()) uniq.push_back(ty);
     const size_t nst = ts_state_size_cfg(cfg);
     std::vector<double> quiet;
     if (!aos) {

@@ -98,8 +98,11 @@ double venkat_eps2(int nd, double hx, double hy, double hz);
 void venkat_axis_factors(int nd, int n, const double* h, std::vector<double>& out);
 bool lookup_kernels(int dim, int flux, int rv, int precision, tsd::KernelSet* ks);
 void host_bc_image(const ts_bc_config& bc, double g, int axis, const double* u, double* o);
-// output rows per tile; `slots` = tiles the GPU holds at once (0: unknown)
-int tuned_rows_per_tile(const ts_config& c, long long slots = 0);
+// output rows per tile; the GPU holds `occ` tiles on each of `units` SIMDs (3-D: CUs) at once
+// (0: unknown)
+int tuned_rows_per_tile(const ts_config& c, long long units, int occ);
+// modelled time of marching `tiles` tiles of ty rows
+double march_cost(long long tiles, int ty, long long units, int occ);
 // the calling thread's error text for entry points without a context (ts_last_error(NULL))
 void set_thread_error(const std::string& m);
 // the reference AoS layout (5 values per cell, ghost layers on active axes) <-> SoA interior
