@@ -14,6 +14,23 @@ namespace tsd {
 
 constexpr int NV = 5;
 
+// A flow without momentum out of the grid's axes (a 1-D tube, a plane 2-D flow) keeps those
+// momenta at exactly zero: no flux, limiter or boundary image makes any.  The kernels are
+// templated on the number N of variables they carry (density, the first N - 2 momenta,
+// energy): N = 3 in 1-D and N = 4 in 2-D when the state and the boundary conditions have none, and
+// N = 5 otherwise.  The other variables' arithmetic is the same operation for operation.
+template <int N>
+__device__ __host__ constexpr int plane_of(int v) { return v == N - 1 ? NV - 1 : v; }
+
+// |momentum|^2
+template <typename R, int N>
+__device__ __forceinline__ R momentum2(const R (&u)[N]) {
+    R s = u[1] * u[1];
+#pragma unroll
+    for (int i = 2; i < N - 1; i++) s += u[i] * u[i];
+    return s;
+}
+
 // ---- boundary conditions -------------------------------------------------------------------
 // Values of BoundaryConditionType (src/BoundaryConditions/BoundaryConditionConfiguration.h:12-19)
 enum : int { BC_WALL = 0, BC_SYMMETRY = 1, BC_MOVING_WALL = 2, BC_SUBSONIC_INLET = 3,
@@ -131,36 +148,53 @@ struct IdealGasEOS {
 // BCGeneral.h:186-268).  Every condition in the reference is even in the normal's sign, so the
 // ghost fill (normal -e_axis on both sides, kernel.h:743,760) and the boundary-face states
 // (normal +e_axis, ExplicitRungeKuttaFVM.h:1202,1208) share this one function.
-template <typename R>
-__device__ __forceinline__ void bc_image(const BCDev& bc, R gamma, int axis, const R (&u)[NV], R (&o)[NV]) {
+template <typename R, int N>
+__device__ __forceinline__ void bc_image(const BCDev& bc, R gamma, int axis, const R (&u)[N], R (&o)[N]) {
     switch (bc.type) {
     case BC_SYMMETRY:
         // U - 2 (n.m) n: only the normal momentum changes sign
-        o[0] = u[0]; o[1] = u[1]; o[2] = u[2]; o[3] = u[3]; o[4] = u[4];
+#pragma unroll
+        for (int v = 0; v < N; v++) o[v] = u[v];
         o[1 + axis] = -u[1 + axis];
         break;
     case BC_WALL:
-        o[0] = u[0]; o[1] = -u[1]; o[2] = -u[2]; o[3] = -u[3]; o[4] = u[4];
+        o[0] = u[0];
+#pragma unroll
+        for (int v = 1; v < N - 1; v++) o[v] = -u[v];
+        o[N - 1] = u[N - 1];
         break;
     case BC_MOVING_WALL: {
-        R rho = u[0];
-        R ir = R(1) / rho;
-        R vx = u[1] * ir, vy = u[2] * ir, vz = u[3] * ir;
-        R rhoe = u[4] - R(0.5) * rho * (vx * vx + vy * vy + vz * vz);
-        R dx = R(2) * R(bc.vel[0]) - vx, dy = R(2) * R(bc.vel[1]) - vy, dz = R(2) * R(bc.vel[2]) - vz;
-        o[0] = rho; o[1] = rho * dx; o[2] = rho * dy; o[3] = rho * dz;
-        o[4] = rhoe + R(0.5) * rho * (dx * dx + dy * dy + dz * dz);
+        const R rho = u[0];
+        const R ir = R(1) / rho;
+        R in = R(0), out = R(0);
+        o[0] = rho;
+#pragma unroll
+        for (int v = 1; v < N - 1; v++) {
+            const R vel = u[v] * ir, img = R(2) * R(bc.vel[v - 1]) - vel;
+            in += vel * vel;
+            out += img * img;
+            o[v] = rho * img;
+        }
+        const R rhoe = u[N - 1] - R(0.5) * rho * in;
+        o[N - 1] = rhoe + R(0.5) * rho * out;
         break;
     }
     case BC_SUBSONIC_INLET: {
-        R r = R(bc.rho);
-        R vx = R(bc.vel[0]), vy = R(bc.vel[1]), vz = R(bc.vel[2]);
-        o[0] = r; o[1] = r * vx; o[2] = r * vy; o[3] = r * vz;
-        o[4] = IdealGasEOS<R>(gamma).EnergyDensityOfPressure(R(bc.p)) + R(0.5) * r * (vx * vx + vy * vy + vz * vz);
+        const R r = R(bc.rho);
+        R q = R(0);
+        o[0] = r;
+#pragma unroll
+        for (int v = 1; v < N - 1; v++) {
+            const R vel = R(bc.vel[v - 1]);
+            q += vel * vel;
+            o[v] = r * vel;
+        }
+        o[N - 1] = IdealGasEOS<R>(gamma).EnergyDensityOfPressure(R(bc.p)) + R(0.5) * r * q;
         break;
     }
     default:  // Natural, SubsonicOutlet: copy
-        o[0] = u[0]; o[1] = u[1]; o[2] = u[2]; o[3] = u[3]; o[4] = u[4];
+#pragma unroll
+        for (int v = 0; v < N; v++) o[v] = u[v];
     }
 }
 
@@ -188,11 +222,11 @@ struct CellGeo {
 // the stencil of ComputeSolutionReconstruction (ERK:897-916).
 // With POS set (the HLLC and exact-Godunov paths, which need a real sound speed), a face state
 // with rho <= 0 or 2 rho E <= |m|^2 falls back to the cell value.
-template <int ND, int RECON, int LIM, typename R, bool POS = false>
-__device__ inline void reconstruct(const R (&c)[NV], const R (&nb)[2 * ND][NV],
-                                   const CellGeo<ND, R>& geo, R (&face)[2 * ND][NV]) {
+template <int ND, int RECON, int LIM, typename R, bool POS = false, int N>
+__device__ inline void reconstruct(const R (&c)[N], const R (&nb)[2 * ND][N],
+                                   const CellGeo<ND, R>& geo, R (&face)[2 * ND][N]) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
+    for (int v = 0; v < N; v++) {
         if constexpr (RECON == RC_PWC) {  // PiecewiseConstant.h:15
 #pragma unroll
             for (int f = 0; f < 2 * ND; f++) face[f][v] = c[v];
@@ -300,8 +334,7 @@ __device__ inline void reconstruct(const R (&c)[NV], const R (&nb)[2 * ND][NV],
         bool any = false;
 #pragma unroll
         for (int f = 0; f < 2 * ND; f++) {
-            R q = R(2) * face[f][0] * face[f][4] -
-                  (face[f][1] * face[f][1] + face[f][2] * face[f][2] + face[f][3] * face[f][3]);
+            R q = R(2) * face[f][0] * face[f][N - 1] - momentum2(face[f]);
             bad[f] = !(face[f][0] > R(0) && q > R(0));
             any = any || bad[f];
         }
@@ -311,7 +344,7 @@ __device__ inline void reconstruct(const R (&c)[NV], const R (&nb)[2 * ND][NV],
             for (int f = 0; f < 2 * ND; f++)
                 if (bad[f]) {
 #pragma unroll
-                    for (int v = 0; v < NV; v++) face[f][v] = c[v];
+                    for (int v = 0; v < N; v++) face[f][v] = c[v];
                 }
         }
     }
@@ -324,41 +357,60 @@ enum : int { FX_GODUNOV = 0, FX_ROE = 1, FX_HLLC = 3 };
 // difference is redone in double when it is a small part of E (near vacuum, where the float
 // subtraction loses most of its digits).
 __device__ inline double internal_energy(double E, double rho_ke) { return E - rho_ke; }
-__device__ inline float internal_energy(float E, float rho_ke, const float (&U)[NV]) {
+template <int N>
+__device__ inline float internal_energy(float E, float rho_ke, const float (&U)[N]) {
     float e = E - rho_ke;
     if (e < 0.01f * E) {
-        double m2 = double(U[1]) * U[1] + double(U[2]) * U[2] + double(U[3]) * U[3];
-        e = float(double(U[4]) - 0.5 * m2 / double(U[0]));
+        double m2 = double(U[1]) * U[1];
+#pragma unroll
+        for (int i = 2; i < N - 1; i++) m2 += double(U[i]) * U[i];
+        e = float(double(U[N - 1]) - 0.5 * m2 / double(U[0]));
     }
     return e;
 }
-__device__ inline double internal_energy(double E, double rho_ke, const double (&)[NV]) {
+template <int N>
+__device__ inline double internal_energy(double E, double rho_ke, const double (&)[N]) {
     return E - rho_ke;
 }
 
 // Roe-Pike flux with Harten's entropy fix (RoeSolverPerfectGasEOS.h:48-134) across a face with
 // normal +e_D.  lam receives |u.n| + c of the Roe average (RoeSolverPerfectGasEOS.h:88,128).
-template <int D, typename R>
-__device__ inline void roe_flux(R gamma, R eps, const R (&UL)[NV], const R (&UR)[NV], R (&F)[NV],
+template <int D, typename R, int N>
+__device__ inline void roe_flux(R gamma, R eps, const R (&UL)[N], const R (&UR)[N], R (&F)[N],
                                 R& lam) {
+    constexpr int NM = N - 2;  // velocity components
     const R gm1 = gamma - R(1);
     R il = frcp(UL[0]), ir = frcp(UR[0]);
-    R vl[3] = {UL[1] * il, UL[2] * il, UL[3] * il};
-    R vr[3] = {UR[1] * ir, UR[2] * ir, UR[3] * ir};
-    R kl = R(0.5) * (vl[0] * vl[0] + vl[1] * vl[1] + vl[2] * vl[2]);
-    R kr = R(0.5) * (vr[0] * vr[0] + vr[1] * vr[1] + vr[2] * vr[2]);
-    R el = UL[4] * il, er = UR[4] * ir;
+    R vl[NM], vr[NM];
+    R kl = R(0), kr = R(0);
+#pragma unroll
+    for (int i = 0; i < NM; i++) {
+        vl[i] = UL[1 + i] * il;
+        vr[i] = UR[1 + i] * ir;
+        kl += vl[i] * vl[i];
+        kr += vr[i] * vr[i];
+    }
+    kl *= R(0.5);
+    kr *= R(0.5);
+    R el = UL[N - 1] * il, er = UR[N - 1] * ir;
     // physical fluxes (RoeSolverPerfectGasEOS.h:15-32)
-    R pl = gm1 * internal_energy(UL[4], UL[0] * kl, UL);
-    R pr = gm1 * internal_energy(UR[4], UR[0] * kr, UR);
+    R pl = gm1 * internal_energy(UL[N - 1], UL[0] * kl, UL);
+    R pr = gm1 * internal_energy(UR[N - 1], UR[0] * kr, UR);
     R hl = (el - kl) * gamma + kl;
     R hr = (er - kr) * gamma + kr;
     R sl = fsqrt(UL[0]), sr = fsqrt(UR[0]);
     R isum = frcp(sl + sr);
     R ql = sl * isum, qr = sr * isum;
-    R v[3] = {ql * vl[0] + qr * vr[0], ql * vl[1] + qr * vr[1], ql * vl[2] + qr * vr[2]};
+    R v[NM];
+    R vv = R(0), vvl = R(0), vvr = R(0);
+#pragma unroll
+    for (int i = 0; i < NM; i++) {
+        v[i] = ql * vl[i] + qr * vr[i];
+        vv += v[i] * v[i];
+        vvl += v[i] * vl[i];
+        vvr += v[i] * vr[i];
+    }
     R h = ql * hl + qr * hr;
-    R vv = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
     R phi2 = R(0.5) * gm1 * vv;
     R c = fsqrt(gm1 * h - phi2);
     R uw = v[D];
@@ -372,24 +424,28 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[NV], const R (&UR)
     R Eig1 = a1;
     R Eiga = (a3 - a4) * R(0.5) * ic;
     R Eigb = (a3 + a4) * R(0.5) - a1;
-    R R1 = phi2 * UR[0] - gm1 * UR[0] * ((v[0] * vr[0] + v[1] * vr[1] + v[2] * vr[2]) - er);
-    R R2 = phi2 * UL[0] - gm1 * UL[0] * ((v[0] * vl[0] + v[1] * vl[1] + v[2] * vl[2]) - el);
+    R R1 = phi2 * UR[0] - gm1 * UR[0] * (vvr - er);
+    R R2 = phi2 * UL[0] - gm1 * UL[0] * (vvl - el);
     R D1 = UR[0] * (vr[D] - v[D]);
     R D2 = UL[0] * (vl[D] - v[D]);
     R C2 = ic * ic;
     // dissipation (RoeSolverPerfectGasEOS.h:96-125) with Qa = (0, n, u.n), Qb = (1, v, h)
     R vnl = vl[D], vnr = vr[D];
-    R FL[NV], FR[NV];
+    R FL[N], FR[N], Qb[N];
     FL[0] = UL[0] * vnl; FR[0] = UR[0] * vnr;
-    FL[1] = FL[0] * vl[0]; FR[1] = FR[0] * vr[0];
-    FL[2] = FL[0] * vl[1]; FR[2] = FR[0] * vr[1];
-    FL[3] = FL[0] * vl[2]; FR[3] = FR[0] * vr[2];
-    FL[1 + D] += pl; FR[1 + D] += pr;
-    FL[4] = vnl * (UL[4] + pl); FR[4] = vnr * (UR[4] + pr);
-    R Qb[NV] = {R(1), v[0], v[1], v[2], h};
+    Qb[0] = R(1);
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-        R qa = (i == 4) ? uw : ((i == 1 + D) ? R(1) : R(0));
+    for (int i = 0; i < NM; i++) {
+        FL[1 + i] = FL[0] * vl[i];
+        FR[1 + i] = FR[0] * vr[i];
+        Qb[1 + i] = v[i];
+    }
+    FL[1 + D] += pl; FR[1 + D] += pr;
+    FL[N - 1] = vnl * (UL[N - 1] + pl); FR[N - 1] = vnr * (UR[N - 1] + pr);
+    Qb[N - 1] = h;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        R qa = (i == N - 1) ? uw : ((i == 1 + D) ? R(1) : R(0));
         R diss = Eig1 * (UL[i] - UR[i]) + Eiga * ((R2 - R1) * qa + (D2 - D1) * Qb[i]) +
                  Eigb * ((R2 - R1) * Qb[i] * C2 + (D2 - D1) * qa);
         F[i] = R(0.5) * (FL[i] + FR[i] + diss);
@@ -407,17 +463,16 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[NV], const R (&UR)
 // S* (E + p*).  A supersonic side takes its own velocity, pressure and energy in the places of
 // the star's.  (Against F_K + S_K (U* - U_K), which needs the whole flux of side K and
 // its velocities first: about 50 instructions fewer per face in double.)
-template <int D, typename R>
-__device__ inline void hllc_flux(R gamma, const R (&UL)[NV], const R (&UR)[NV], R (&F)[NV],
+template <int D, typename R, int N>
+__device__ inline void hllc_flux(R gamma, const R (&UL)[N], const R (&UR)[N], R (&F)[N],
                                  R& lam) {
     const IdealGasEOS<R> eos(gamma);
-    constexpr int T1 = D == 0 ? 2 : 1, T2 = D == 2 ? 2 : 3;  // tangential momenta
     const R il = frcp(UL[0]), ir = frcp(UR[0]);
     const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-    const R kl = R(0.5) * il * (UL[1] * UL[1] + UL[2] * UL[2] + UL[3] * UL[3]);
-    const R kr = R(0.5) * ir * (UR[1] * UR[1] + UR[2] * UR[2] + UR[3] * UR[3]);
-    const R pl = eos.PressureOfEnergyDensity(internal_energy(UL[4], kl, UL));
-    const R pr = eos.PressureOfEnergyDensity(internal_energy(UR[4], kr, UR));
+    const R kl = R(0.5) * il * momentum2(UL);
+    const R kr = R(0.5) * ir * momentum2(UR);
+    const R pl = eos.PressureOfEnergyDensity(internal_energy(UL[N - 1], kl, UL));
+    const R pr = eos.PressureOfEnergyDensity(internal_energy(UR[N - 1], kr, UR));
     const R al = eos.SoundSpeedOfPressure(pl, il), ar = eos.SoundSpeedOfPressure(pr, ir);
     const R SL = vmin(ul - al, ur - ar);
     const R SR = vmax(ul + al, ur + ar);
@@ -427,8 +482,7 @@ __device__ inline void hllc_flux(R gamma, const R (&UL)[NV], const R (&UR)[NV], 
     const R Ss = fdiv(pr - pl + ul * ml - ur * mr, ml - mr);
     const bool left = Ss >= R(0);
     const R S = left ? SL : SR, w = left ? wl : wr, m = left ? ml : mr;
-    const R rho = left ? UL[0] : UR[0], un = left ? ul : ur, p = left ? pl : pr, E = left ? UL[4] : UR[4];
-    const R t1 = left ? UL[T1] : UR[T1], t2 = left ? UL[T2] : UR[T2];
+    const R rho = left ? UL[0] : UR[0], un = left ? ul : ur, p = left ? pl : pr, E = left ? UL[N - 1] : UR[N - 1];
     const bool supersonic = left ? (S >= R(0)) : (S <= R(0));
     // on a subsonic side S - S* is not zero (S < 0 <= S*, or the mirror case)
     const R r = frcp(supersonic ? R(1) : S - Ss);
@@ -438,10 +492,11 @@ __device__ inline void hllc_flux(R gamma, const R (&UL)[NV], const R (&UR)[NV], 
     const R uf = supersonic ? un : Ss, pf = supersonic ? p : ps, Ef = supersonic ? E : Es;
     const R q = c * uf;
     F[0] = rho * q;
-    F[T1] = t1 * q;
-    F[T2] = t2 * q;
+#pragma unroll
+    for (int i = 1; i < N - 1; i++)
+        if (i != 1 + D) F[i] = (left ? UL[i] : UR[i]) * q;
     F[1 + D] = F[0] * uf + pf;
-    F[4] = uf * (Ef + pf);
+    F[N - 1] = uf * (Ef + pf);
 }
 
 // ---- exact Riemann solver (always double) -----------------------------------------------------
@@ -665,19 +720,27 @@ __device__ inline StarDev star_state_dev(double g, double rl, double ul, double 
 // Exact Godunov flux: the solution sampled at x/t = 0 (GodunovSolverPerfectGasEOS.h:276-433),
 // tangential velocity from the upwind side of the contact.  Computed in double for both
 // arithmetic forms.
-template <int D, typename R>
-__device__ inline void godunov_flux(R gammaR, const R (&ULr)[NV], const R (&URr)[NV], R (&F)[NV],
+template <int D, typename R, int N>
+__device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[N], R (&F)[N],
                                     R& lam) {
+    constexpr int NM = N - 2;  // velocity components
     const double g = double(gammaR);
     const IdealGasEOS<double> eos(g);
-    double UL[NV], UR[NV];
+    double UL[N], UR[N];
 #pragma unroll
-    for (int i = 0; i < NV; i++) { UL[i] = double(ULr[i]); UR[i] = double(URr[i]); }
+    for (int i = 0; i < N; i++) { UL[i] = double(ULr[i]); UR[i] = double(URr[i]); }
     double il = 1.0 / UL[0], ir = 1.0 / UR[0];
-    double vL[3] = {UL[1] * il, UL[2] * il, UL[3] * il};
-    double vR[3] = {UR[1] * ir, UR[2] * ir, UR[3] * ir};
-    double pL = eos.GetPressure(UL[0], UL[4] * il - (vL[0] * vL[0] + vL[1] * vL[1] + vL[2] * vL[2]) / 2.0);
-    double pR = eos.GetPressure(UR[0], UR[4] * ir - (vR[0] * vR[0] + vR[1] * vR[1] + vR[2] * vR[2]) / 2.0);
+    double vL[NM], vR[NM];
+    double kL = 0.0, kR = 0.0;
+#pragma unroll
+    for (int i = 0; i < NM; i++) {
+        vL[i] = UL[1 + i] * il;
+        vR[i] = UR[1 + i] * ir;
+        kL += vL[i] * vL[i];
+        kR += vR[i] * vR[i];
+    }
+    double pL = eos.GetPressure(UL[0], UL[N - 1] * il - kL / 2.0);
+    double pR = eos.GetPressure(UR[0], UR[N - 1] * ir - kR / 2.0);
     double uL = vL[D], uR = vR[D];
     StarDev st = star_state_dev(g, UL[0], uL, pL, UR[0], uR, pR);
     double ro, u, p;
@@ -720,72 +783,97 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[NV], const R (&URr)
         u = (sgn * aK + 0.5 * (g - 1) * uK + S) * (2 / (g + 1));
         p = w * C * C * pK;
     }
-    const double* vel = left ? vL : vR;
-    double Vf[3] = {vel[0], vel[1], vel[2]};
-    Vf[D] = vel[D] + (u - vel[D]);
-    double Fd[NV];
+    double Vf[NM];
+#pragma unroll
+    for (int i = 0; i < NM; i++) Vf[i] = left ? vL[i] : vR[i];
+    Vf[D] = Vf[D] + (u - Vf[D]);
+    double Fd[N];
     if (ro == 0.0) {
 #pragma unroll
-        for (int i = 0; i < NV; i++) Fd[i] = 0.0;
+        for (int i = 0; i < N; i++) Fd[i] = 0.0;
     } else {
         // Uface and F(Uface) (GodunovSolverPerfectGasEOS.h:416-427)
-        double U0 = ro, U1 = ro * Vf[0], U2 = ro * Vf[1], U3 = ro * Vf[2];
-        double U4 = ro * (eos.GetInternalEnergy(ro, p) + 0.5 * (Vf[0] * Vf[0] + Vf[1] * Vf[1] + Vf[2] * Vf[2]));
-        double iro = 1.0 / U0;
-        double vx = U1 * iro, vy = U2 * iro, vz = U3 * iro;
-        double pp = eos.PressureOfEnergyDensity(U4 - U0 * (vx * vx + vy * vy + vz * vz) / 2.0);
-        double vv[3] = {vx, vy, vz};
-        double vn = vv[D];
-        Fd[0] = U0 * vn;
-        Fd[1] = U0 * vn * vx;
-        Fd[2] = U0 * vn * vy;
-        Fd[3] = U0 * vn * vz;
+        double U[N], k = 0.0;
+        U[0] = ro;
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            U[1 + i] = ro * Vf[i];
+            k += Vf[i] * Vf[i];
+        }
+        U[N - 1] = ro * (eos.GetInternalEnergy(ro, p) + 0.5 * k);
+        const double iro = 1.0 / U[0];
+        double vv[NM];
+        k = 0.0;
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            vv[i] = U[1 + i] * iro;
+            k += vv[i] * vv[i];
+        }
+        const double pp = eos.PressureOfEnergyDensity(U[N - 1] - U[0] * k / 2.0);
+        const double vn = vv[D];
+        Fd[0] = U[0] * vn;
+#pragma unroll
+        for (int i = 0; i < NM; i++) Fd[1 + i] = U[0] * vn * vv[i];
         Fd[1 + D] += pp;
-        Fd[4] = vn * (U4 + pp);
+        Fd[N - 1] = vn * (U[N - 1] + pp);
     }
 #pragma unroll
-    for (int i = 0; i < NV; i++) F[i] = R(Fd[i]);
+    for (int i = 0; i < N; i++) F[i] = R(Fd[i]);
     lam = R(st.smax);
 }
 
 // Face eigenvalue only (the dt pass needs no flux).
-template <int FLUX, int D, typename R>
-__device__ inline R face_eigen(R gamma, const R (&UL)[NV], const R (&UR)[NV]) {
+template <int FLUX, int D, typename R, int N>
+__device__ inline R face_eigen(R gamma, const R (&UL)[N], const R (&UR)[N]) {
     if constexpr (FLUX == FX_ROE) {
         // |u.n| + c of the Roe average (RoeSolverPerfectGasEOS.h:60-88)
+        constexpr int NM = N - 2;
         const R gm1 = gamma - R(1);
         R il = frcp(UL[0]), ir = frcp(UR[0]);
-        R vl[3] = {UL[1] * il, UL[2] * il, UL[3] * il};
-        R vr[3] = {UR[1] * ir, UR[2] * ir, UR[3] * ir};
-        R kl = R(0.5) * (vl[0] * vl[0] + vl[1] * vl[1] + vl[2] * vl[2]);
-        R kr = R(0.5) * (vr[0] * vr[0] + vr[1] * vr[1] + vr[2] * vr[2]);
-        R hl = (UL[4] * il - kl) * gamma + kl;
-        R hr = (UR[4] * ir - kr) * gamma + kr;
+        R vl[NM], vr[NM];
+        R kl = R(0), kr = R(0);
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            vl[i] = UL[1 + i] * il;
+            vr[i] = UR[1 + i] * ir;
+            kl += vl[i] * vl[i];
+            kr += vr[i] * vr[i];
+        }
+        kl *= R(0.5);
+        kr *= R(0.5);
+        R hl = (UL[N - 1] * il - kl) * gamma + kl;
+        R hr = (UR[N - 1] * ir - kr) * gamma + kr;
         R sl = fsqrt(UL[0]), sr = fsqrt(UR[0]);
         R isum = frcp(sl + sr);
         R ql = sl * isum, qr = sr * isum;
-        R v[3] = {ql * vl[0] + qr * vr[0], ql * vl[1] + qr * vr[1], ql * vl[2] + qr * vr[2]};
+        R vv = R(0), vn = R(0);
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            const R v = ql * vl[i] + qr * vr[i];
+            vv += v * v;
+            if (i == D) vn = v;
+        }
         R h = ql * hl + qr * hr;
-        R phi2 = R(0.5) * gm1 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-        return __builtin_fabs(v[D]) + fsqrt(gm1 * h - phi2);
+        R phi2 = R(0.5) * gm1 * vv;
+        return __builtin_fabs(vn) + fsqrt(gm1 * h - phi2);
     } else if constexpr (FLUX == FX_HLLC) {
         const IdealGasEOS<R> eos(gamma);
         const R il = frcp(UL[0]), ir = frcp(UR[0]);
         const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-        const R kl = R(0.5) * il * (UL[1] * UL[1] + UL[2] * UL[2] + UL[3] * UL[3]);
-        const R kr = R(0.5) * ir * (UR[1] * UR[1] + UR[2] * UR[2] + UR[3] * UR[3]);
-        const R al = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UL[4], kl, UL)), il);
-        const R ar = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UR[4], kr, UR)), ir);
+        const R kl = R(0.5) * il * momentum2(UL);
+        const R kr = R(0.5) * ir * momentum2(UR);
+        const R al = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UL[N - 1], kl, UL)), il);
+        const R ar = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UR[N - 1], kr, UR)), ir);
         return vmax(vabs(vmin(ul - al, ur - ar)), vabs(vmax(ul + al, ur + ar)));
     } else {
-        R F[NV], lam;
+        R F[N], lam;
         godunov_flux<D, R>(gamma, UL, UR, F, lam);
         return lam;
     }
 }
 
-template <int FLUX, int D, typename R>
-__device__ inline void face_flux(R gamma, R eps, const R (&UL)[NV], const R (&UR)[NV], R (&F)[NV],
+template <int FLUX, int D, typename R, int N>
+__device__ inline void face_flux(R gamma, R eps, const R (&UL)[N], const R (&UR)[N], R (&F)[N],
                                  R& lam) {
     if constexpr (FLUX == FX_ROE) roe_flux<D, R>(gamma, eps, UL, UR, F, lam);
     else if constexpr (FLUX == FX_HLLC) hllc_flux<D, R>(gamma, UL, UR, F, lam);

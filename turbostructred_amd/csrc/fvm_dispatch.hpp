@@ -31,15 +31,17 @@ struct KernelSet {
     ChunkFn euler1d_chunk = nullptr;
 };
 
+// in_grid: the instances for states without momentum out of the grid's axes (1-D and 2-D; no viscous
+// and no unfused SSP kernels).
 // reconstruction variants: 0 PWC, 1 linear, 2 ENO2, 3 limited linear BJ, 4 limited linear Venkat
-bool get_kernels_d1_f0(int rv, int precision, KernelSet* ks);
-bool get_kernels_d1_f1(int rv, int precision, KernelSet* ks);
-bool get_kernels_d1_f3(int rv, int precision, KernelSet* ks);
-bool get_kernels_d2_f0(int rv, int precision, KernelSet* ks);
-bool get_kernels_d2_f1(int rv, int precision, KernelSet* ks);
-bool get_kernels_d2_f3(int rv, int precision, KernelSet* ks);
-bool get_kernels_d3_f0(int rv, int precision, KernelSet* ks);
-bool get_kernels_d3_f1(int rv, int precision, KernelSet* ks);
-bool get_kernels_d3_f3(int rv, int precision, KernelSet* ks);
+bool get_kernels_d1_f0(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d1_f1(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d1_f3(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d2_f0(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d2_f1(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d2_f3(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d3_f0(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d3_f1(int rv, int precision, bool in_grid, KernelSet* ks);
+bool get_kernels_d3_f3(int rv, int precision, bool in_grid, KernelSet* ks);
 
 }  // namespace tsd

@@ -51,7 +51,7 @@ struct StepCtl {
     int active;  // 1 while steps remain to be taken
     int go;      // 1 if the current step runs (set by the dt pass)
     int error;   // 1 = dt not finite and positive
-    int pad0;
+    int out_of_grid;  // set by an upload that finds momentum out of the grid's axes
     double* dt_log;
     long long dt_log_base, dt_log_cap;  // dt of iteration `it` goes to dt_log[it - base]
     double rnorm[5];                    // residual norms of the last step (MODE_RN)
@@ -400,12 +400,13 @@ __device__ inline void add_sources(const VisArgs& v, const R (&u)[NV], double vo
 // DT_ARG instances take the step's dt from `dt_arg` instead of the control block in memory;
 // LDS_STATE instances read and write the state through `uin_arg` / `uout_arg` with plane stride
 // `plane_arg` (LDS arrays, addressed generically) with plain stores.
-template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int VIS = 0,
-          bool DT_ARG = false, bool LDS_STATE = false, bool GP = false>
+template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int N = NV,
+          int VIS = 0, bool DT_ARG = false, bool LDS_STATE = false, bool GP = false>
 __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, double& block_min,
                                            double* rn = nullptr, double dt_arg = 0.0, const void* uin_arg = nullptr,
                                            void* uout_arg = nullptr, size_t plane_arg = 0) {
     using MT = ModeTraits<MODE>;
+    static_assert(!VIS || N == NV, "viscous instances carry every variable");
     const GridArgs& g = a.g;
     const StepCtl* ctl = a.ctl;
     const bool tile_ok = tile >= 0 && tile < a.ntiles;
@@ -453,8 +454,8 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
     // on the loaded values (stage 2's U^n + dt L, a ghost image) makes the wavefront wait for them
     // early.
     struct RawRow {
-        TIn u[NV];
-        TOut l[MODE == MODE_F2 ? NV : 1];
+        TIn u[N];
+        TOut l[MODE == MODE_F2 ? N : 1];
         int rs, yside;
     };
     auto issue_row = [&](int r, RawRow& q) {
@@ -464,36 +465,36 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
         q.yside = yside;
         const unsigned off = unsigned(rs) * unsigned(nx) + unsigned(xs);
 #pragma unroll
-        for (int v = 0; v < NV; v++) q.u[v] = ld_state<GP>(uin, P, v, off);
+        for (int v = 0; v < N; v++) q.u[v] = ld_state<GP>(uin, P, plane_of<N>(v), off);
         if constexpr (MODE == MODE_F2) {
 #pragma unroll
-            for (int v = 0; v < NV; v++) q.l[v] = ld_state<GP>(lin, P, v, off);
+            for (int v = 0; v < N; v++) q.l[v] = ld_state<GP>(lin, P, plane_of<N>(v), off);
         }
     };
-    auto complete_row = [&](const RawRow& q, R (&u)[NV]) {
+    auto complete_row = [&](const RawRow& q, R (&u)[N]) {
         if constexpr (MODE == MODE_F2) {
 #pragma unroll
-            for (int v = 0; v < NV; v++) u[v] = R(double(q.u[v]) + dt * double(q.l[v]));
+            for (int v = 0; v < N; v++) u[v] = R(double(q.u[v]) + dt * double(q.l[v]));
         } else {
 #pragma unroll
-            for (int v = 0; v < NV; v++) u[v] = R(q.u[v]);
+            for (int v = 0; v < N; v++) u[v] = R(q.u[v]);
         }
         if (xside != 0) {
             // one branch per side, so that the side (and, along a row, the condition) is
             // wave-uniform and its data come from scalar loads
-            R t[NV];
+            R t[N];
             if (xside < 0) bc_image(g.bc[bc_marker(g, 0, q.rs)], gamma, 0, u, t);
             else bc_image(g.bc[bc_marker(g, 1, q.rs)], gamma, 0, u, t);
 #pragma unroll
-            for (int v = 0; v < NV; v++) u[v] = t[v];
+            for (int v = 0; v < N; v++) u[v] = t[v];
         } else if (q.yside != 0) {
-            R t[NV];
+            R t[N];
             bc_image(g.bc[bc_marker(g, q.yside < 0 ? 2 : 3, xs)], gamma, 1, u, t);
 #pragma unroll
-            for (int v = 0; v < NV; v++) u[v] = t[v];
+            for (int v = 0; v < N; v++) u[v] = t[v];
         }
     };
-    auto load_row = [&](int r, R (&u)[NV]) {
+    auto load_row = [&](int r, R (&u)[N]) {
         RawRow q;
         issue_row(r, q);
         complete_row(q, u);
@@ -507,41 +508,41 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
     const bool inc = (INC_F2 && a.dout != nullptr) || (INC_S3 && a.din != nullptr);
     using IncT = typename std::conditional<MODE == MODE_F2, TOut, TIn>::type;
     const IncT* incsrc = (MODE == MODE_F2) ? (const IncT*)a.lin : (const IncT*)a.din;
-    auto load_inc = [&](unsigned off, IncT (&d)[NV]) {
+    auto load_inc = [&](unsigned off, IncT (&d)[N]) {
         if (inc) {
 #pragma unroll
-            for (int v = 0; v < NV; v++) d[v] = ld_state<GP>(incsrc, P, v, off);
+            for (int v = 0; v < N; v++) d[v] = ld_state<GP>(incsrc, P, plane_of<N>(v), off);
         }
     };
 
     // write the result for a finalized cell: the stage update, or L = R/V (MODE_F1)
-    auto finish = [&](unsigned off, const R (&u)[NV], const R (&res0)[NV], const double (&un)[NV],
-                      const IncT (&dc)[NV], double ivol, double vol) {
-        R res[NV];
+    auto finish = [&](unsigned off, const R (&u)[N], const R (&res0)[N], const double (&un)[N],
+                      const IncT (&dc)[N], double ivol, double vol) {
+        R res[N];
 #pragma unroll
-        for (int v = 0; v < NV; v++) res[v] = res0[v];
+        for (int v = 0; v < N; v++) res[v] = res0[v];
         if constexpr (VIS) add_sources(a.v, u, vol, res);
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
+        for (int v = 0; v < N; v++) {
             if constexpr (MODE == MODE_RN) {
                 if (out_lane) rn[v] += vol * __builtin_fabs(double(res[v]));
             } else if constexpr (MODE == MODE_F1) {
-                if (out_lane) store(v, off, TOut(double(res[v]) * ivol));
+                if (out_lane) store(plane_of<N>(v), off, TOut(double(res[v]) * ivol));
             } else {
                 if (inc && MODE == MODE_F2) {
                     const double d = 0.25 * dt * (double(dc[v]) + double(res[v]) * ivol);
                     if (out_lane) {
-                        st_state_stream<GP>((TOut*)a.dout, P, v, off, TOut(d));
-                        store(v, off, TOut(un[v] + d));
+                        st_state_stream<GP>((TOut*)a.dout, P, plane_of<N>(v), off, TOut(d));
+                        store(plane_of<N>(v), off, TOut(un[v] + d));
                     }
                 } else if (inc && MODE == MODE_S3) {
                     const double d = double(dc[v]);
                     const double q = un[v] + (2.0 / 3.0) * (d + dt * (double(res[v]) * ivol));
-                    if (out_lane) store(v, off, TOut(q));
+                    if (out_lane) store(plane_of<N>(v), off, TOut(q));
                 } else {
                     double q = double(u[v]) + dt * (double(res[v]) * ivol);
                     if constexpr (MT::use_un) q = MT::ca * un[v] + MT::cb * q;
-                    if (out_lane) store(v, off, TOut(q));
+                    if (out_lane) store(plane_of<N>(v), off, TOut(q));
                 }
             }
         }
@@ -550,22 +551,22 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
 
     if constexpr (DIM == 1) {
         // ---- one row ----
-        R c[NV], nb[2][NV], face[2][NV];
+        R c[N], nb[2][N], face[2][N];
         load_row(0, c);
-        double un[NV];
+        double un[N];
 #pragma unroll
-        for (int v = 0; v < NV; v++) un[v] = MT::use_un ? ld_state<GP>(a.un, P, v, unsigned(xs)) : 0.0;
-        IncT dc[NV];
+        for (int v = 0; v < N; v++) un[v] = MT::use_un ? ld_state<GP>(a.un, P, plane_of<N>(v), unsigned(xs)) : 0.0;
+        IncT dc[N];
         load_inc(unsigned(xs), dc);
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
+        for (int v = 0; v < N; v++) {
             nb[0][v] = dpp_from_left(c[v]);
             nb[1][v] = dpp_from_right(c[v]);
         }
         reconstruct<1, RECON, LIM, R, FLUX != FX_ROE>(c, nb, geo, face);
-        R UL[NV], UR[NV];
+        R UL[N], UR[N];
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
+        for (int v = 0; v < N; v++) {
             UL[v] = dpp_from_left(face[1][v]);
             UR[v] = face[0][v];
         }
@@ -575,14 +576,14 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
         }
         const R Sx = R(1);
         R lam;
-        R F[NV];
+        R F[N];
         if constexpr (MT::flux) face_flux<FLUX, 0, R>(gamma, eps, UL, UR, F, lam);
         else lam = face_eigen<FLUX, 0, R>(gamma, UL, UR);
         if constexpr (VIS && MT::flux) {
             if (a.v.viscous) {
                 const unsigned fi = unsigned(xg < 0 ? 0 : (xg > nx ? nx : xg));
 #pragma unroll
-                for (int v = 1; v < NV; v++) F[v] -= R(ld_plane(a.v.fv[0], a.v.nface[0], v - 1, fi));
+                for (int v = 1; v < N; v++) F[v] -= R(ld_plane(a.v.fv[0], a.v.nface[0], v - 1, fi));
             }
         }
         if constexpr (MT::sr) {
@@ -600,9 +601,9 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             if (ghost_x_lane) block_min = __builtin_fmin(block_min, dt_candidate(ld_geo_uniform<GP>(g.h[0], nx + 1), double(Sx * lam)));
         }
         if constexpr (MT::flux) {
-            R res[NV];
+            R res[N];
 #pragma unroll
-            for (int v = 0; v < NV; v++) {
+            for (int v = 0; v < N; v++) {
                 R Fr = dpp_from_right(F[v]);
                 res[v] = -((Fr - F[v]) * Sx);
             }
@@ -614,20 +615,20 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
         const int yend = (y0 + a.ty < ny) ? y0 + a.ty : ny;
         RawRow Pn;              // prefetched stencil row (completed and entered into the window one
                                 // iteration later)
-        double Nc[NV];          // U^n of the row finalized in this iteration (SSP stages 2, 3)
-        IncT Dc[NV];            // its L(U^n) or increment (FP32-residual stages 2, 3)
-        R ytop[NV];             // +y face state of the previously reconstructed row
+        double Nc[N];          // U^n of the row finalized in this iteration (SSP stages 2, 3)
+        IncT Dc[N];            // its L(U^n) or increment (FP32-residual stages 2, 3)
+        R ytop[N];             // +y face state of the previously reconstructed row
         // The three-row window (rows rc-1, rc, rc+1) and the values carried to the next row live
         // in LDS, one set per wavefront; no other lane reads them, so no barrier is needed.  The
         // window rotates by slot index instead of register moves, and out of the register file
         // these 20 doubles per lane (40 KB per 4-wavefront block in FP64) leave the occupancy to
         // the register count.
-        __shared__ R ring[4][3][NV][64];  // [wavefront][slot][variable][lane]
+        __shared__ R ring[4][3][N][64];  // [wavefront][slot][variable][lane]
         // residual carried to the pending row: its x part plus S_y times the y-flux through its
         // bottom face; the finalize subtracts S_y times the flux through its top face
-        __shared__ R carry[4][NV][64];
+        __shared__ R carry[4][N][64];
         const int wl = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
-        R (&cy)[NV][64] = carry[wl];
+        R (&cy)[N][64] = carry[wl];
         int sm = 0, s0 = 1, sp = 2;  // slots of rows rc-1, rc, rc+1
         // x-neighbours are read from the same LDS rows at lane -+ 1 (the end lanes, halo lanes
         // whose results are discarded, read themselves): LDS reads instead of VALU lane shifts
@@ -635,26 +636,26 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
         double srp = 0.0;       // spectral radius of the pending row without its top face
         R lam_gb = R(0);
         {
-            R t0[NV], t1[NV];
+            R t0[N], t1[N];
             load_row(y0 - 2, t0);
             load_row(y0 - 1, t1);
 #pragma unroll
-            for (int v = 0; v < NV; v++) {
+            for (int v = 0; v < N; v++) {
                 ring[wl][sm][v][lane] = t0[v];
                 ring[wl][s0][v][lane] = t1[v];
             }
         }
         issue_row(y0, Pn);
 #pragma unroll
-        for (int v = 0; v < NV; v++) Nc[v] = 0.0;
+        for (int v = 0; v < N; v++) Nc[v] = 0.0;
         const int nit = yend - y0 + 2;
         for (int t = 0; t < nit; t++) {
             const int rc = y0 - 1 + t;  // row being reconstructed
             {
-                R un1[NV];
+                R un1[N];
                 complete_row(Pn, un1);
 #pragma unroll
-                for (int v = 0; v < NV; v++) ring[wl][sp][v][lane] = un1[v];
+                for (int v = 0; v < N; v++) ring[wl][sp][v][lane] = un1[v];
             }
             if (t + 1 < nit) issue_row(rc + 2, Pn);
             if constexpr (MT::use_un) {
@@ -664,7 +665,7 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                 if (t >= 2) {
                     const unsigned offn = unsigned(rc - 1) * unsigned(nx) + unsigned(xs);
 #pragma unroll
-                    for (int v = 0; v < NV; v++) Nc[v] = ld_state<GP>(a.un, P, v, offn);
+                    for (int v = 0; v < N; v++) Nc[v] = ld_state<GP>(a.un, P, plane_of<N>(v), offn);
                     load_inc(offn, Dc);
                 }
             }
@@ -676,11 +677,11 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             geo.rl[1] = R(ld_geo_uniform<GP>(g.rl[1], rcs));
             geo.rr[1] = R(ld_geo_uniform<GP>(g.rr[1], rcs));
             if (ev_cells) geo.eps2 = R(ev_x * ld_geo_uniform<GP>(g.ev[1], rcs));
-            R nb[4][NV], face[4][NV];
+            R nb[4][N], face[4][N];
             {
-                R U0[NV];
+                R U0[N];
 #pragma unroll
-                for (int v = 0; v < NV; v++) {
+                for (int v = 0; v < N; v++) {
                     U0[v] = ring[wl][s0][v][lane];
                     nb[0][v] = ring[wl][s0][v][lm];
                     nb[1][v] = ring[wl][s0][v][lp];
@@ -691,22 +692,22 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             }
             if (t >= 1) {
                 // face between rows rc-1 and rc
-                R GL[NV], GR[NV];
+                R GL[N], GR[N];
 #pragma unroll
-                for (int v = 0; v < NV; v++) { GL[v] = ytop[v]; GR[v] = face[2][v]; }
+                for (int v = 0; v < N; v++) { GL[v] = ytop[v]; GR[v] = face[2][v]; }
                 if (!g.periodic[1]) {
                     if (rc == 0) bc_image(g.bc[bc_marker(g, 2, xs)], gamma, 1, GR, GL);
                     if (rc == ny) bc_image(g.bc[bc_marker(g, 3, xs)], gamma, 1, GL, GR);
                 }
                 const R Sy = R(hx);  // face area of a y-face (ERK:1268)
-                R G[NV], lam;
+                R G[N], lam;
                 if constexpr (MT::flux) face_flux<FLUX, 1, R>(gamma, eps, GL, GR, G, lam);
                 else lam = face_eigen<FLUX, 1, R>(gamma, GL, GR);
                 if constexpr (VIS && MT::flux) {
                     if (a.v.viscous) {
                         const unsigned fi = unsigned(rc) * unsigned(nx) + unsigned(xs);
 #pragma unroll
-                        for (int v = 1; v < NV; v++) G[v] -= R(ld_plane(a.v.fv[1], a.v.nface[1], v - 1, fi));
+                        for (int v = 1; v < N; v++) G[v] -= R(ld_plane(a.v.fv[1], a.v.nface[1], v - 1, fi));
                     }
                 }
                 if constexpr (MT::sr) {
@@ -729,28 +730,28 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                         // finalize row rc-1 = the row in slot sm
                         const int rf = rc - 1;
                         const double ivol = ihx * ld_geo_uniform<GP>(g.ih[1], rf + 1);
-                        R res[NV], Um[NV];
+                        R res[N], Um[N];
 #pragma unroll
-                        for (int v = 0; v < NV; v++) {
+                        for (int v = 0; v < N; v++) {
                             res[v] = cy[v][lane] - G[v] * Sy;
                             Um[v] = ring[wl][sm][v][lane];
                         }
                         finish(unsigned(rf) * unsigned(nx) + unsigned(xs), Um, res, Nc, Dc, ivol, hx * ld_geo_uniform<GP>(g.h[1], rf + 1));
                     }
 #pragma unroll
-                    for (int v = 0; v < NV; v++) cy[v][lane] = G[v] * Sy;
+                    for (int v = 0; v < N; v++) cy[v][lane] = G[v] * Sy;
                 }
                 if (rc < yend) {
                     // x-faces of row rc: each lane evaluates its minus face.  The plus-face
                     // states of the left neighbours, then the fluxes and eigenvalues of the right
                     // neighbours, pass through the LDS slot of row rc-1, free after its finalize
                     // (LDS operations of one wavefront complete in order).
-                    R (&xch)[NV][64] = ring[wl][sm];
-                    R UL[NV], UR[NV];
+                    R (&xch)[N][64] = ring[wl][sm];
+                    R UL[N], UR[N];
 #pragma unroll
-                    for (int v = 0; v < NV; v++) xch[v][lane] = face[1][v];
+                    for (int v = 0; v < N; v++) xch[v][lane] = face[1][v];
 #pragma unroll
-                    for (int v = 0; v < NV; v++) {
+                    for (int v = 0; v < N; v++) {
                         UL[v] = xch[v][lm];
                         UR[v] = face[0][v];
                     }
@@ -759,21 +760,21 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                         if (xg == nx) bc_image(g.bc[bc_marker(g, 1, rcs)], gamma, 0, UL, UR);
                     }
                     const R Sx = R(hy);  // face area of an x-face (ERK:1189)
-                    R F[NV], lamx;
+                    R F[N], lamx;
                     if constexpr (MT::flux) face_flux<FLUX, 0, R>(gamma, eps, UL, UR, F, lamx);
                     else lamx = face_eigen<FLUX, 0, R>(gamma, UL, UR);
                     if constexpr (VIS && MT::flux) {
                         if (a.v.viscous) {
                             const unsigned fi = unsigned(rcs) * unsigned(nx + 1) + unsigned(xg < 0 ? 0 : (xg > nx ? nx : xg));
 #pragma unroll
-                            for (int v = 1; v < NV; v++) F[v] -= R(ld_plane(a.v.fv[0], a.v.nface[0], v - 1, fi));
+                            for (int v = 1; v < N; v++) F[v] -= R(ld_plane(a.v.fv[0], a.v.nface[0], v - 1, fi));
                         }
                     }
                     if constexpr (MT::flux) {
 #pragma unroll
-                        for (int v = 0; v < NV; v++) xch[v][lane] = F[v];
+                        for (int v = 0; v < N; v++) xch[v][lane] = F[v];
 #pragma unroll
-                        for (int v = 0; v < NV; v++) cy[v][lane] = cy[v][lane] - (xch[v][lp] - F[v]) * Sx;
+                        for (int v = 0; v < N; v++) cy[v][lane] = cy[v][lane] - (xch[v][lp] - F[v]) * Sx;
                     }
                     if constexpr (MT::sr) {
                         xch[0][lane] = lamx;
@@ -796,7 +797,7 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                 }
             }
 #pragma unroll
-            for (int v = 0; v < NV; v++) ytop[v] = face[3][v];
+            for (int v = 0; v < N; v++) ytop[v] = face[3][v];
             const int st = sm;
             sm = s0;
             s0 = sp;
@@ -807,7 +808,7 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
 }
 
 // ---- single-solve kernel: one wavefront per tile, block-level dt reduction ----------------------
-template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int VIS = 0>
+template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int N = NV, int VIS = 0>
 __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
     static_assert(DIM == 1 || DIM == 2, "3-D uses its own kernel");
     using MT = ModeTraits<MODE>;
@@ -834,8 +835,8 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
         if (tile >= a.ntiles) return;  // only the norms reduce across the block
     }
     double block_min = __builtin_inf();
-    double rn[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, VIS>(a, tile < a.ntiles ? tile : -1, lane, block_min, rn);
+    double rn[N] = {};
+    stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, VIS>(a, tile < a.ntiles ? tile : -1, lane, block_min, rn);
     if constexpr (MT::sr) {
         // store the wavefront's minimum; dt_finalize_kernel turns the tiles' minima into dt after
         // this launch
@@ -845,7 +846,10 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
     }
     if constexpr (MODE == MODE_RN) {
         __shared__ double rred[4 * NV];
-        rn_reduce_finalize(ctl, a.rn_part, rn, rred, lane, wave, nwaves);
+        double rn5[NV] = {};
+#pragma unroll
+        for (int v = 0; v < N; v++) rn5[plane_of<N>(v)] = rn[v];
+        rn_reduce_finalize(ctl, a.rn_part, rn5, rred, lane, wave, nwaves);
     }
 }
 
@@ -870,7 +874,7 @@ constexpr int wg1d_waves = FLUX == FX_GODUNOV ? 8 : 16;
 constexpr int WG1D_LDS_CELLS = 1984;  // 2 buffers x 5 planes x 1984 doubles = 158720 bytes
 
 // one step; false when the loop has to end
-template <int RECON, int LIM, int FLUX, bool LDS>
+template <int RECON, int LIM, int FLUX, int N, bool LDS>
 __device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, double* red, int* run, int lane,
                                              int wave, const double* sin, double* sout) {
     if (threadIdx.x == 0) *run = ctl->active;
@@ -882,7 +886,7 @@ __device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, doubl
     double m = __builtin_inf();
     for (int tile = wave; tile < a.ntiles; tile += wg1d_waves<FLUX>) {
         double mt = __builtin_inf();
-        stage_tile<1, RECON, LIM, FLUX, MODE_DT, double, double, double, 0, false, LDS>(
+        stage_tile<1, RECON, LIM, FLUX, MODE_DT, double, double, double, N, 0, false, LDS, false>(
             a, tile, lane, mt, nullptr, 0.0, sin, sout, WG1D_LDS_CELLS);
         m = __builtin_fmin(m, mt);
     }
@@ -902,22 +906,22 @@ __device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, doubl
     const double dt = ctl->dt;
     for (int tile = wave; tile < a.ntiles; tile += wg1d_waves<FLUX>) {
         double unused = 0.0;
-        stage_tile<1, RECON, LIM, FLUX, MODE_S1, double, double, double, 0, true, LDS>(
+        stage_tile<1, RECON, LIM, FLUX, MODE_S1, double, double, double, N, 0, true, LDS, false>(
             a, tile, lane, unused, nullptr, dt, sin, sout, WG1D_LDS_CELLS);
     }
     __syncthreads();
     return true;
 }
 
-template <int RECON, int LIM, int FLUX, bool LDS>
+template <int RECON, int LIM, int FLUX, int N, bool LDS>
 __global__ void __launch_bounds__(64 * wg1d_waves<FLUX>) fvm_euler1d_workgroup(KArgs a0, KArgs a1, int cap) {
     constexpr int NT = 64 * wg1d_waves<FLUX>;
     __shared__ double red[wg1d_waves<FLUX>];
     __shared__ int run;
     __shared__ StepCtl ctl;  // a0.ctl and a1.ctl are the same block
-    __shared__ double st[LDS ? 2 * NV * WG1D_LDS_CELLS : 1];
+    __shared__ double st[LDS ? 2 * N * WG1D_LDS_CELLS : 1];
     double* b0 = st;
-    double* b1 = st + (LDS ? NV * WG1D_LDS_CELLS : 0);
+    double* b1 = st + (LDS ? N * WG1D_LDS_CELLS : 0);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ncell = a0.g.n[0];  // at most WG1D_LDS_CELLS when LDS (checked by the launcher)
     if (threadIdx.x == 0) ctl = *a0.ctl;  // read only by thread 0 until the first barrier
@@ -925,15 +929,15 @@ __global__ void __launch_bounds__(64 * wg1d_waves<FLUX>) fvm_euler1d_workgroup(K
         const double* g = (const double*)a0.uin;
         for (int c = threadIdx.x; c < ncell; c += NT)
 #pragma unroll
-            for (int v = 0; v < NV; v++) b0[v * WG1D_LDS_CELLS + c] = g[(size_t)v * a0.plane + c];
+            for (int v = 0; v < N; v++) b0[v * WG1D_LDS_CELLS + c] = g[(size_t)v * a0.plane + c];
         __syncthreads();
     }
     int done = 0;  // uniform: every wavefront takes the same branches
     for (int it = 0; it < cap; it += 2) {
-        if (!euler1d_step<RECON, LIM, FLUX, LDS>(a0, &ctl, red, &run, lane, wave, b0, b1)) break;
+        if (!euler1d_step<RECON, LIM, FLUX, N, LDS>(a0, &ctl, red, &run, lane, wave, b0, b1)) break;
         done++;
         if (it + 1 >= cap) break;
-        if (!euler1d_step<RECON, LIM, FLUX, LDS>(a1, &ctl, red, &run, lane, wave, b1, b0)) break;
+        if (!euler1d_step<RECON, LIM, FLUX, N, LDS>(a1, &ctl, red, &run, lane, wave, b1, b0)) break;
         done++;
     }
     if constexpr (LDS) {
@@ -944,7 +948,7 @@ __global__ void __launch_bounds__(64 * wg1d_waves<FLUX>) fvm_euler1d_workgroup(K
         double* g = (done & 1) ? (double*)a0.uout : (double*)const_cast<void*>(a0.uin);
         for (int c = threadIdx.x; c < ncell; c += NT)
 #pragma unroll
-            for (int v = 0; v < NV; v++) g[(size_t)v * a0.plane + c] = src[v * WG1D_LDS_CELLS + c];
+            for (int v = 0; v < N; v++) g[(size_t)v * a0.plane + c] = src[v * WG1D_LDS_CELLS + c];
     }
     if (threadIdx.x == 0) *a0.ctl = ctl;  // the other threads only ever read the LDS copy
 }
@@ -959,7 +963,7 @@ __global__ void __launch_bounds__(64 * wg1d_waves<FLUX>) fvm_euler1d_workgroup(K
 // its dt.  A cell's arithmetic depends only on its own problem, and the minimum is exact, so a
 // result is the same alone or in a mix.
 
-template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut>
+template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int N = NV>
 __global__ void __launch_bounds__(256) fvm_stage_batched(const KArgs* __restrict__ descs,
                                                          const int2* __restrict__ table,
                                                          const int* __restrict__ ntiles_p,
@@ -990,11 +994,11 @@ __global__ void __launch_bounds__(256) fvm_stage_batched(const KArgs* __restrict
             const int s1 = (s0 + a.ty < a.ntiles) ? s0 + a.ty : a.ntiles;
             for (int sidx = s0; sidx < s1; sidx++) {
                 double ms = __builtin_inf();
-                stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, 0, false, false, true>(a, sidx, lane, ms);
+                stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, false, true>(a, sidx, lane, ms);
                 m = __builtin_fmin(m, ms);
             }
         } else {
-            stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, 0, false, false, true>(a, e.y, lane, m);
+            stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, false, true>(a, e.y, lane, m);
         }
         if constexpr (MT::sr) {
             // the entry's minimum; dt_finalize_batched reduces each solve's entries after the launch

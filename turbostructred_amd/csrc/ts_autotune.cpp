@@ -92,10 +92,22 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
         std::lock_guard<std::mutex> lk(g_mu);
         g_table.erase(key_of(*cfg));
     }
+    const size_t nst = ts_state_size_cfg(cfg);
+    std::vector<double> quiet;
+    if (!aos) {
+        // a quiescent uniform state: the arithmetic of the flux kernels barely depends on the data
+        quiet.assign(nst, 0.0);
+        for (size_t i = 0; i < nst / 5; i++) {
+            quiet[i * 5 + 0] = 1.0;
+            quiet[i * 5 + 4] = 2.5;
+        }
+        aos = quiet.data();
+    }
     std::vector<int> cands;
     {
         ts_ctx* c = nullptr;
         if (ts_create(cfg, &c) == TS_OK) {
+            (void)ts_set_state(c, aos, nst);  // the tiling is that of the kernels the state runs
             const int m = c->ty;
             cands = {m, m > 1 ? m - (m + 3) / 4 : 1, m + m / 4 + 1};
             const long long strips = c->nstrips, tiles_m = c->ntiles;
@@ -117,17 +129,6 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
     std::vector<int> uniq;
     for (int ty : cands)
         if (ty >= 1 && ty <= ymax && std::find(uniq.begin(), uniq.end(), ty) == uniq.end()) uniq.push_back(ty);
-    const size_t nst = ts_state_size_cfg(cfg);
-    std::vector<double> quiet;
-    if (!aos) {
-        // a quiescent uniform state: the arithmetic of the flux kernels barely depends on the data
-        quiet.assign(nst, 0.0);
-        for (size_t i = 0; i < nst / 5; i++) {
-            quiet[i * 5 + 0] = 1.0;
-            quiet[i * 5 + 4] = 2.5;
-        }
-        aos = quiet.data();
-    }
     int best = -1, k = 0;
     double bms = 1e300;
     for (int ty : uniq) {

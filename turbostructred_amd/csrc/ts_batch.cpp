@@ -106,7 +106,7 @@ class Arena {
     }
 };
 
-using FamilyKey = std::tuple<int, int, int, int>;  // ndims, riemann, recon variant, precision
+using FamilyKey = std::tuple<int, int, int, int, int>;  // ndims, riemann, recon variant, precision, in_grid
 
 struct Problem {
     long long ticket = 0;
@@ -296,16 +296,17 @@ Layout layout_of(const ts_config& c) {
     return L;
 }
 
-// every (ndims, flux, reconstruction variant, precision) key: 3 x 3 x 5 x 2
-constexpr size_t kMaxFamilies = 90;
+// every (ndims, flux, reconstruction variant, precision, in_grid) key: 3 x 3 x 5 x 2 x 2
+constexpr size_t kMaxFamilies = 180;
 
-int family_of(ts_batch* b, const ts_config& c) {
-    FamilyKey k(c.ndims, c.riemann, tsr::recon_variant(c), c.precision);
+// in_grid: the problem has no momentum out of the grid's axes and none can arise
+int family_of(ts_batch* b, const ts_config& c, bool in_grid) {
+    FamilyKey k(c.ndims, c.riemann, tsr::recon_variant(c), c.precision, in_grid);
     for (size_t i = 0; i < b->families.size(); i++)
         if (b->families[i].key == k) return (int)i;
     Family f;
     f.key = k;
-    if (!tsr::lookup_kernels(c.ndims, c.riemann, tsr::recon_variant(c), c.precision, &f.ks) || !f.ks.bf1) return -1;
+    if (!tsr::lookup_kernels(c.ndims, c.riemann, tsr::recon_variant(c), c.precision, in_grid, &f.ks) || !f.ks.bf1) return -1;
     f.occupancy = f.ks.bocc ? f.ks.bocc() : 1;
     if (b->families.size() >= kMaxFamilies) return -1;
     b->families.push_back(f);
@@ -822,9 +823,24 @@ int ts_batch_submit(ts_batch* b, const ts_config* cfg, const double* init_state,
     p->bytes = layout_of(*cfg).total;
     if (p->bytes > b->arena.capacity) return fail(b, TS_ERR_NOMEM, "solve is larger than the HBM budget");
     size_t nst = ts_state_size_cfg(cfg);
-    p->init.assign(init_state, init_state + nst);
+    // copied in blocks that stay in the cache while they are searched for momentum out of the grid's
+    // axes (any bit but the sign's: NaN counts)
+    p->init.reserve(nst);
+    const double* const out_of_grid = init_state + (cfg->ndims == 1 ? 2 : 3);
+    uint64_t bits = 0;
+    for (size_t i = 0; i < nst; i += 5 * 1024) {
+        const size_t end = std::min(nst, i + 5 * 1024);
+        p->init.insert(p->init.end(), init_state + i, init_state + end);
+        for (size_t j = i; j < end; j += 5) {
+            uint64_t u[2];
+            std::memcpy(u, out_of_grid + j, (cfg->ndims == 1 ? 2 : 1) * sizeof(uint64_t));
+            bits |= u[0] << 1;
+            if (cfg->ndims == 1) bits |= u[1] << 1;
+        }
+    }
+    const bool in_grid = bits == 0 && tsr::boundaries_in_grid(*cfg);
     std::lock_guard<std::mutex> lk(b->mu);
-    int fam = family_of(b, *cfg);
+    int fam = family_of(b, *cfg, in_grid);
     if (fam < 0) return fail(b, TS_ERR_UNSUPPORTED, "no batched kernel for this configuration");
     p->family = fam;
     p->ticket = b->next_ticket++;

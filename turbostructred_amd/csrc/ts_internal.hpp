@@ -41,6 +41,17 @@ struct ts_ctx {
     double* dt_log = nullptr;
     long long dt_log_cap = 0, dt_log_base = 0;
 
+    // The kernels in use and their tiling, chosen between two variants at every ts_set_state:
+    // variant[0] carries every variable, variant[1] (may_reduce) only those of a flow within the
+    // grid's axes.
+    struct Variant {
+        tsd::KernelSet ks;
+        int ty = 16, ntiles = 1;
+        dim3 grid_dim;
+    };
+    Variant variant[2];
+    bool may_reduce = false, reduced = false;
+    size_t most_blocks = 1;  // of the variants' grids
     tsd::KernelSet ks;
     int ty = 16;
     int nstrips = 1, ntiles = 1;
@@ -96,7 +107,9 @@ double venkat_eps2(int nd, double hx, double hy, double hz);
 // per-axis factors (K h_i)^(3/nd) of that value for the n interior cells of an axis whose sizes
 // start at h (null for an inactive axis: one factor 1)
 void venkat_axis_factors(int nd, int n, const double* h, std::vector<double>& out);
-bool lookup_kernels(int dim, int flux, int rv, int precision, tsd::KernelSet* ks);
+bool lookup_kernels(int dim, int flux, int rv, int precision, bool in_grid, tsd::KernelSet* ks);
+// whether no boundary condition of the table can give momentum out of the grid's axes (1-D, 2-D)
+bool boundaries_in_grid(const ts_config& c);
 void host_bc_image(const ts_bc_config& bc, double g, int axis, const double* u, double* o);
 // output rows per tile; the GPU holds `occ` tiles on each of `units` SIMDs (3-D: CUs) at once
 // (0: unknown)
@@ -108,13 +121,18 @@ void set_thread_error(const std::string& m);
 // the reference AoS layout (5 values per cell, ghost layers on active axes) <-> SoA interior
 // planes, on the device; the AoS ghost entries are neither read nor written
 size_t aos_doubles(int nd, const int n[3]);
-hipError_t device_aos_to_soa(const double* d_aos, double* d_soa, int nd, const int n[3], hipStream_t stream);
+// (out_of_grid: set to 1 where a cell has momentum out of the grid's axes, or null)
+hipError_t device_aos_to_soa(const double* d_aos, double* d_soa, int nd, const int n[3], hipStream_t stream,
+                             int* out_of_grid = nullptr);
 hipError_t device_soa_to_aos(const double* d_soa, double* d_aos, int nd, const int n[3], hipStream_t stream);
 }  // namespace tsr
 
 size_t ts_state_size_cfg(const ts_config* c);
 int init_device_ctx(ts_ctx* c, const ts_config* cfg);
 void destroy_device_ctx(ts_ctx* c);
+int drop_graphs(ts_ctx* c);
+// make the kernels of variant[reduced] the ones in use
+int use_variant(ts_ctx* c, bool reduced);
 void fill_ghost_images(const ts_ctx* c, double* aos);
 int get_cells(ts_ctx* c, const int* ijk, size_t n, double* out);
 int run_steps(ts_ctx* c, int max_steps, double t_max, double next_snap);

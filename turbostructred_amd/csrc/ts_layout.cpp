@@ -24,13 +24,16 @@ __device__ __forceinline__ size_t aos_cell(const Shape& s, unsigned c, int& i, i
 }
 
 __global__ void __launch_bounds__(256) aos_to_soa_kernel(const double* __restrict__ aos, double* __restrict__ soa,
-                                                         Shape s) {
+                                                         Shape s, int* __restrict__ out_of_grid) {
     const size_t c = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (c >= s.plane) return;
     int i, j, k;
     const size_t a = aos_cell(s, unsigned(c), i, j, k);
 #pragma unroll
     for (int v = 0; v < 5; v++) soa[size_t(v) * s.plane + c] = aos[a + v];
+    // NaN counts as out of the grid's axes
+    const bool out = (s.g[2] == 0 && !(aos[a + 3] == 0.0)) || (s.g[1] == 0 && !(aos[a + 2] == 0.0));
+    if (out_of_grid && out) *out_of_grid = 1;
 }
 
 __global__ void __launch_bounds__(256) soa_to_aos_kernel(const double* __restrict__ soa, double* __restrict__ aos,
@@ -63,10 +66,12 @@ size_t aos_doubles(int nd, const int n[3]) {
     return t;
 }
 
-hipError_t device_aos_to_soa(const double* d_aos, double* d_soa, int nd, const int n[3], hipStream_t stream) {
+hipError_t device_aos_to_soa(const double* d_aos, double* d_soa, int nd, const int n[3], hipStream_t stream,
+                             int* out_of_grid) {
     const Shape s = shape_of(nd, n);
     if (s.plane == 0) return hipSuccess;
-    hipLaunchKernelGGL(aos_to_soa_kernel, dim3(unsigned((s.plane + 255) / 256)), dim3(256), 0, stream, d_aos, d_soa, s);
+    hipLaunchKernelGGL(aos_to_soa_kernel, dim3(unsigned((s.plane + 255) / 256)), dim3(256), 0, stream, d_aos, d_soa, s,
+                       out_of_grid);
     return hipGetLastError();
 }
 

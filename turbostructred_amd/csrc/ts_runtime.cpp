@@ -126,21 +126,30 @@ int recon_variant(const ts_config& c) {
     return c.recon;
 }
 
-bool lookup_kernels(int dim, int flux, int rv, int precision, KernelSet* ks) {
+bool lookup_kernels(int dim, int flux, int rv, int precision, bool in_grid, KernelSet* ks) {
     if (dim == 1) {
-        if (flux == 0) return get_kernels_d1_f0(rv, precision, ks);
-        if (flux == 1) return get_kernels_d1_f1(rv, precision, ks);
-        if (flux == 3) return get_kernels_d1_f3(rv, precision, ks);
+        if (flux == 0) return get_kernels_d1_f0(rv, precision, in_grid, ks);
+        if (flux == 1) return get_kernels_d1_f1(rv, precision, in_grid, ks);
+        if (flux == 3) return get_kernels_d1_f3(rv, precision, in_grid, ks);
     } else if (dim == 2) {
-        if (flux == 0) return get_kernels_d2_f0(rv, precision, ks);
-        if (flux == 1) return get_kernels_d2_f1(rv, precision, ks);
-        if (flux == 3) return get_kernels_d2_f3(rv, precision, ks);
+        if (flux == 0) return get_kernels_d2_f0(rv, precision, in_grid, ks);
+        if (flux == 1) return get_kernels_d2_f1(rv, precision, in_grid, ks);
+        if (flux == 3) return get_kernels_d2_f3(rv, precision, in_grid, ks);
     } else {
-        if (flux == 0) return get_kernels_d3_f0(rv, precision, ks);
-        if (flux == 1) return get_kernels_d3_f1(rv, precision, ks);
-        if (flux == 3) return get_kernels_d3_f3(rv, precision, ks);
+        if (flux == 0) return get_kernels_d3_f0(rv, precision, in_grid, ks);
+        if (flux == 1) return get_kernels_d3_f1(rv, precision, in_grid, ks);
+        if (flux == 3) return get_kernels_d3_f3(rv, precision, in_grid, ks);
     }
     return false;
+}
+
+bool boundaries_in_grid(const ts_config& c) {
+    for (int m = 0; m < c.n_bc; m++) {
+        if (c.bc[m].type != TS_BC_MOVING_WALL && c.bc[m].type != TS_BC_SUBSONIC_INLET) continue;
+        for (int a = c.ndims; a < 3; a++)
+            if (c.bc[m].velocity[a] != 0.0) return false;
+    }
+    return c.ndims < 3;
 }
 
 // Host copy of the BC images used for the ghost layers of ts_get_state.
@@ -269,11 +278,14 @@ int ts_set_state(ts_ctx* c, const double* aos, size_t n) {
     HIPCHK(c, hipSetDevice(c->cfg.device));
     int r = ensure_aos(c);
     if (r) return r;
+    // the conversion also notes whether any momentum points out of the grid's axes
     HIPCHK(c, hipMemcpyAsync(c->d_aos, aos, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, tsr::device_aos_to_soa(c->d_aos, (double*)c->dU[0], c->nd, c->n, c->stream));
+    HIPCHK(c, hipMemsetAsync(&c->dctl->out_of_grid, 0, sizeof(int), c->stream));
+    HIPCHK(c, tsr::device_aos_to_soa(c->d_aos, (double*)c->dU[0], c->nd, c->n, c->stream, &c->dctl->out_of_grid));
+    HIPCHK(c, hipMemcpyAsync(&c->hctl->out_of_grid, &c->dctl->out_of_grid, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->cur = 0;
-    return TS_OK;
+    return use_variant(c, c->may_reduce && !c->hctl->out_of_grid);
 }
 
 int ts_get_state(ts_ctx* c, double* aos, size_t n) {
@@ -309,17 +321,13 @@ int ts_enable_residual_norms(ts_ctx* c, int enable) {
     if (!c) return TS_ERR_INVALID;
     HIPCHK(c, hipSetDevice(c->cfg.device));
     if (enable && !c->rn_part) {
-        HIPCHK(c, hipMalloc((void**)&c->rn_part, (size_t)c->grid_dim.x * 5 * sizeof(double)));
-        c->device_bytes += (size_t)c->grid_dim.x * 5 * sizeof(double);
+        HIPCHK(c, hipMalloc((void**)&c->rn_part, c->most_blocks * 5 * sizeof(double)));
+        c->device_bytes += c->most_blocks * 5 * sizeof(double);
     }
     if (c->norms != (enable != 0)) {
         // the captured step graphs hold the launch sequence: re-capture with or without the pass
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        for (int i = 0; i < 2; i++) {
-            if (c->graph_exec[i]) HIPCHK(c, hipGraphExecDestroy(c->graph_exec[i]));
-            c->graph_exec[i] = nullptr;
-            c->graph_steps[i] = 0;
-        }
+        int r = drop_graphs(c);
+        if (r) return r;
     }
     c->norms = enable != 0;
     for (int v = 0; v < 5; v++) c->h_rnorm[v] = 0.0;

@@ -65,12 +65,22 @@ inline size_t gidx(const ts_ctx* c, int i, int j, int k) {
 
 constexpr int CHUNK = 256;  // steps issued between host checks of the termination flag
 
-// rows per tile for the CUs of the device and the resident workgroups per CU of the kernels
-// (tiles_per_block tiles to a workgroup)
-int rows_per_tile(const ts_ctx* c, const ts_config& cfg, int tiles_per_block) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, c->cfg.device) != hipSuccess || !c->ks.socc) return tsr::tuned_rows_per_tile(cfg, 0, 0);
-    return tsr::tuned_rows_per_tile(cfg, (long long)prop.multiProcessorCount * tiles_per_block, c->ks.socc());
+// Tiling of one kernel variant: output rows per tile for the CUs of the device and the resident
+// workgroups per CU of its kernels, tiles and grid.
+void tile_variant(const ts_ctx* c, const ts_config& cfg, ts_ctx::Variant& v) {
+    const int per_block = c->nd == 3 ? 1 : 4;  // 1-D, 2-D: a tile (1-D: a strip) per wavefront, four to a block
+    int cus = 0;
+    if (c->nd == 1) {
+        v.ty = 1;
+    } else if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device) != hipSuccess || !v.ks.socc) {
+        v.ty = tsr::tuned_rows_per_tile(cfg, 0, 0);
+    } else {
+        v.ty = tsr::tuned_rows_per_tile(cfg, (long long)cus * per_block, v.ks.socc());
+    }
+    const int nyb = c->nd > 1 ? (c->n[1] + v.ty - 1) / v.ty : 1;
+    const int nzb = c->nd > 2 ? (c->n[2] + ZOUT - 1) / ZOUT : 1;
+    v.ntiles = c->nstrips * nyb * nzb;
+    v.grid_dim = dim3((v.ntiles + per_block - 1) / per_block);
 }
 
 }  // namespace
@@ -159,7 +169,7 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
             g.face_marker[s] = d;
         }
     }
-    if (!tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, &c->ks) || !c->ks.dt) {
+    if (!tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, false, &c->ks) || !c->ks.dt) {
         c->err = "no kernel instance for this (dimension, flux, reconstruction) combination";
         return TS_ERR_UNSUPPORTED;
     }
@@ -212,36 +222,57 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
         CHK(hipHostMalloc((void**)&c->hctl, sizeof(StepCtl), hipHostMallocDefault));
     }
     std::memset(c->hctl, 0, sizeof(StepCtl));
-    // tiling
-    if (c->nd == 1) {
-        c->ty = 1;
-        c->nstrips = (c->n[0] + STRIP - 1) / STRIP;
-        c->ntiles = c->nstrips;
-        // four strips (one per wavefront) per block
-        c->block_dim = dim3(256);
-        c->grid_dim = dim3((c->ntiles + 3) / 4);
-    } else if (c->nd == 2) {
-        c->ty = rows_per_tile(c, *cfg, 4);
-        c->nstrips = (c->n[0] + STRIP - 1) / STRIP;
-        int nyb = (c->n[1] + c->ty - 1) / c->ty;
-        c->ntiles = c->nstrips * nyb;
-        c->block_dim = dim3(256);
-        c->grid_dim = dim3((c->ntiles + 3) / 4);
-    } else {
-        c->ty = rows_per_tile(c, *cfg, 1);
-        c->nstrips = (c->n[0] + STRIP - 1) / STRIP;
-        int nyb = (c->n[1] + c->ty - 1) / c->ty;
-        int nzb = (c->n[2] + ZOUT - 1) / ZOUT;
-        c->ntiles = c->nstrips * nyb * nzb;
-        c->block_dim = dim3(64 * ZW);
-        c->grid_dim = dim3(c->ntiles);
-    }
-    // one minimum of V/SR per tile from every dt pass and fused stage 1
-    if ((r = dalloc(c, &c->dt_part, (size_t)c->ntiles))) return r;
     const char* sep = getenv("TS_SEPARATE_DT");
     c->fused_dt = k.rk_stages == 3 && !(sep && sep[0] == '1') && c->ks.f1 && c->ks.f2 && !c->vis;
+    // tiling of the kernels that carry every variable and, where a state may do without the momenta
+    // out of the grid's axes, of those that leave them out (borrowed-memory calls do not inspect
+    // the state)
+    c->nstrips = (c->n[0] + STRIP - 1) / STRIP;
+    c->block_dim = dim3(c->nd == 3 ? 64 * ZW : 256);
+    c->variant[0].ks = c->ks;
+    c->may_reduce = !c->arena && !c->vis && (k.rk_stages == 1 || c->fused_dt) && tsr::boundaries_in_grid(k) &&
+                    tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, true, &c->variant[1].ks);
+    size_t most_tiles = 0;
+    for (int i = 0; i < (c->may_reduce ? 2 : 1); i++) {
+        tile_variant(c, *cfg, c->variant[i]);
+        most_tiles = std::max(most_tiles, (size_t)c->variant[i].ntiles);
+        c->most_blocks = std::max(c->most_blocks, (size_t)c->variant[i].grid_dim.x);
+    }
+    // one minimum of V/SR per tile from every dt pass and fused stage 1
+    if ((r = dalloc(c, &c->dt_part, most_tiles))) return r;
+    if ((r = use_variant(c, false))) return r;
     c->euler1d_wg = k.rk_stages == 1 && c->nd == 1 && k.precision == TS_FP64 && !c->vis && c->ks.euler1d_chunk &&
                     c->ntiles <= 64 && !(sep && sep[0] == '1');
+    return TS_OK;
+}
+
+int drop_graphs(ts_ctx* c) {
+    CHK(hipStreamSynchronize(c->stream));
+    for (int i = 0; i < 2; i++) {
+        if (c->graph_exec[i]) CHK(hipGraphExecDestroy(c->graph_exec[i]));
+        c->graph_exec[i] = nullptr;
+        c->graph_steps[i] = 0;
+    }
+    return TS_OK;
+}
+
+int use_variant(ts_ctx* c, bool reduced) {
+    if (reduced && c->cfg.rk_stages == 1) {
+        // forward Euler ping-pongs: the planes that the kernels leave out are zero in the other
+        // buffer too (SSP-RK3 updates U^n in place)
+        const size_t first = 1 + c->nd;
+        CHK(hipMemsetAsync((double*)c->dU[1] + first * c->ncell, 0, (4 - first) * c->ncell * sizeof(double), c->stream));
+    }
+    const ts_ctx::Variant& v = c->variant[reduced];
+    if (reduced != c->reduced) {
+        int r = drop_graphs(c);  // they hold the other variant's launches
+        if (r) return r;
+    }
+    c->reduced = reduced;
+    c->ks = v.ks;
+    c->ty = v.ty;
+    c->ntiles = v.ntiles;
+    c->grid_dim = v.grid_dim;
     return TS_OK;
 }
 
