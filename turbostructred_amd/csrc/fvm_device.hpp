@@ -570,11 +570,11 @@ struct SideDev {
     double c2a;   // 2 a_K / (g-1)
 };
 // cA = 2/(g+1), cB = (g-1)/(g+1), c2 = 2/(g-1)
-__device__ inline SideDev side_dev(double cA, double cB, double c2, double r, double pk, double ak) {
+__device__ inline SideDev side_dev(double cA, double cB, double c2, double ir, double pk, double ak, double r) {
     SideDev s;
     s.pk = pk;
     s.ak = ak;
-    s.A = cA * frcp(r);
+    s.A = cA * ir;
     s.B = pk * cB;
     s.ipk = frcp(pk);
     s.ira = frcp(r * ak);
@@ -620,19 +620,31 @@ struct StarDev {
 
 // Star state by Newton-Raphson from Toro's adaptive initial guess (Toro sec. 4.3, 9.5.1); the
 // reference uses ALGLIB's bounded Levenberg-Marquardt for the same root
-// (GodunovSolverPerfectGasEOS.h:143-185).  Divergent lanes simply run a masked loop.
+// (GodunovSolverPerfectGasEOS.h:143-185).  Divergent lanes simply run a masked loop, so a
+// wavefront pays for its slowest lane: what bounds the exact solver is the number of evaluations
+// of f_K (a power, two branches, about 190 instructions) and, in a short grid, their serial chain.
+//   - The loop ends after a step D with |D| <= 1e-8 p: f is concave with |f''| < f' / p, so the error
+//     after that step is below (D/p)^2 / 2 = 5e-17 p, and the evaluation that would confirm it is
+//     not made.
+//   - f_K and (p/p_K)^z at the final p come from the last evaluation, one such step away, to
+//     first order: the next term is as small.
+//   - Pressures within a factor of two start from the primitive-variable guess wherever that is
+//     not far below both: Newton takes no more steps from it than from the two-rarefaction formula,
+//     whose three powers every lane of the wavefront would wait for.
 __device__ inline StarDev star_state_dev(double g, double rl, double ul, double pl, double rr,
-                                         double ur, double pr) {
+                                         double ur, double pr, double irl, double irr) {
     StarDev s;
-    double pe = -1.0, fle = 0.0, fre = 0.0, zle = 0.0, zre = 0.0;  // last Newton evaluation
-    double al = __builtin_sqrt(g * pl / rl), ar = __builtin_sqrt(g * pr / rr);
-    double du = ur - ul;
-    s.vacuum = (2.0 / (g - 1.0)) * (al + ar) <= du;
-    const double z = (g - 1.0) / (2.0 * g);
-    const double cA = 2.0 / (g + 1.0), cB = (g - 1.0) / (g + 1.0), c2 = 2.0 / (g - 1.0);
-    const SideDev sl = side_dev(cA, cB, c2, rl, pl, al), sr = side_dev(cA, cB, c2, rr, pr, ar);
+    const double al = fsqrt(g * pl * irl), ar = fsqrt(g * pr * irr);
+    const double du = ur - ul;
+    const double ig = frcp(g), igp = frcp(g + 1.0), c2 = 2.0 * frcp(g - 1.0);
+    s.vacuum = c2 * (al + ar) <= du;
+    const double z = 0.5 * (g - 1.0) * ig;
+    const double cA = 2.0 * igp, cB = (g - 1.0) * igp;
+    const SideDev sl = side_dev(cA, cB, c2, irl, pl, al, rl), sr = side_dev(cA, cB, c2, irr, pr, ar, rr);
     const double rho_lr = dpow(pl * sr.ipk, z);  // (pL/pR)^z
     double p = 0.0;
+    double f1 = 0.0, f2 = 0.0, pzl = 0.0, pzr = 0.0;
+    bool known = false;  // f_L, f_R and the powers at p are formed
     // Inputs that are not a physical state (zero, negative or NaN density or pressure) give a
     // NaN star pressure straight away.  Such inputs reach the solver on halo lanes, which are
     // fed by a cross-lane shift and whose flux is discarded; iterating on them to the cap would
@@ -641,44 +653,47 @@ __device__ inline StarDev star_state_dev(double g, double rl, double ul, double 
     if (!physical) {
         p = __builtin_nan("");
     } else if (!s.vacuum) {
-        double pmin = __builtin_fmin(pl, pr), pmax = __builtin_fmax(pl, pr);
+        const double pmin = __builtin_fmin(pl, pr), pmax = __builtin_fmax(pl, pr);
         double ppv = 0.5 * (pl + pr) - 0.125 * du * (rl + rr) * (al + ar);
         ppv = __builtin_fmax(0.0, ppv);
-        if (pmax / pmin <= 2.0 && pmin <= ppv && ppv <= pmax) {
+        if (pmax <= 2.0 * pmin && ppv >= 0.5 * pmin && ppv <= pmax) {
             p = ppv;
         } else if (ppv < pmin) {
-            double plz = dpow(pl, z), prz = dpow(pr, z);
-            double t = (al + ar - 0.5 * (g - 1.0) * du) / (al / plz + ar / prz);
-            p = dpow(t, 1.0 / z);
+            const double plz = dpow(pl, z), prz = dpow(pr, z);
+            const double t = fdiv(al + ar - 0.5 * (g - 1.0) * du, fdiv(al, plz) + fdiv(ar, prz));
+            p = dpow(t, g * c2);
         } else {
-            double A = 2.0 / ((g + 1.0) * rl), B = (g - 1.0) / (g + 1.0) * pl;
-            double gl = __builtin_sqrt(A / (ppv + B));
-            A = 2.0 / ((g + 1.0) * rr);
-            B = (g - 1.0) / (g + 1.0) * pr;
-            double gr = __builtin_sqrt(A / (ppv + B));
-            p = (gl * pl + gr * pr - du) / (gl + gr);
+            const double gl = fsqrt(sl.A * frcp(ppv + sl.B));
+            const double gr = fsqrt(sr.A * frcp(ppv + sr.B));
+            p = fdiv(gl * pl + gr * pr - du, gl + gr);
         }
         if (!(p > 0.0)) p = 1e-12 * pmin;
         for (int it = 1; it <= 60; it++) {
             double dl, dr, zl, zr;
             double ql, qr;
             side_powers(sl, sr, z, rho_lr, p, ql, qr);
-            double fl = fk_dev(sl, p, ql, dl, zl), fr = fk_dev(sr, p, qr, dr, zr);
-            pe = p, fle = fl, fre = fr, zle = zl, zre = zr;
-            double f = fl + fr + du;
+            const double fl = fk_dev(sl, p, ql, dl, zl), fr = fk_dev(sr, p, qr, dr, zr);
+            const double f = fl + fr + du;
             double pn = p - fdiv(f, dl + dr);
             if (!(pn > 0.0)) pn = 0.01 * p;
-            // relative change |pn - p| / (pn + p) <= 1e-15, without the division (pn + p > 0)
-            const bool done = __builtin_fabs(pn - p) <= 1e-15 * (pn + p);
+            const double dp = pn - p;
+            if (__builtin_fabs(dp) <= 1e-8 * p) {
+                known = true;
+                f1 = fl + dl * dp;
+                f2 = fr + dr * dp;
+                // on a shock's side at the last evaluation the power was not formed; where the step
+                // leads to that side's own pressure it is next to 1
+                const double zp = z * fdiv(dp, p);
+                pzl = p > pl ? 1.0 + z * (pn * sl.ipk - 1.0) : zl + zl * zp;
+                pzr = p > pr ? 1.0 + z * (pn * sr.ipk - 1.0) : zr + zr * zp;
+                p = pn;
+                break;
+            }
             p = pn;
-            if (done) break;
         }
     }
     s.p = p;
-    double f1, f2, pzl, pzr;
-    if (p == pe) {  // Newton stopped on a fixed point (e.g. equal states): f_L, f_R are known
-        f1 = fle, f2 = fre, pzl = zle, pzr = zre;
-    } else {
+    if (!known) {  // vacuum, a non-physical input, or the iteration cap
         double d1, d2;
         double ql, qr;
         side_powers(sl, sr, z, rho_lr, p, ql, qr);
@@ -687,11 +702,11 @@ __device__ inline StarDev star_state_dev(double g, double rl, double ul, double 
     }
     s.u = 0.5 * (ul + ur) + 0.5 * (f2 - f1);
     s.smax = 0.0;
-    double prl = p / pl;
     s.SL = s.SHL = s.STL = s.SR = s.SHR = s.STR = 0.0;
+    const double gs = 0.5 * (g + 1.0) * ig;
     if (p > pl) {
         s.shock_l = true;
-        s.SL = ul - al * __builtin_sqrt((g + 1) * prl / (2 * g) + (g - 1) / (2 * g));
+        s.SL = ul - al * fsqrt(gs * (p * sl.ipk) + z);
         s.smax = __builtin_fmax(s.smax, __builtin_fabs(s.SL));
     } else {
         s.shock_l = false;
@@ -699,10 +714,9 @@ __device__ inline StarDev star_state_dev(double g, double rl, double ul, double 
         s.STL = s.u - al * pzl;  // (p/pL)^((g-1)/2g), from f_L
         s.smax = __builtin_fmax(s.smax, __builtin_fabs(s.SHL));
     }
-    double prr = p / pr;
     if (p > pr) {
         s.shock_r = true;
-        s.SR = ur + ar * __builtin_sqrt((g + 1) * prr / (2 * g) + (g - 1) / (2 * g));
+        s.SR = ur + ar * fsqrt(gs * (p * sr.ipk) + z);
         s.smax = __builtin_fmax(s.smax, __builtin_fabs(s.SR));
     } else {
         s.shock_r = false;
@@ -711,8 +725,8 @@ __device__ inline StarDev star_state_dev(double g, double rl, double ul, double 
         s.smax = __builtin_fmax(s.smax, __builtin_fabs(s.SHR));
     }
     if (s.vacuum) {  // the fan tails bound the vacuum (Toro sec. 4.6)
-        s.STL = ul + 2.0 * al / (g - 1.0);
-        s.STR = ur - 2.0 * ar / (g - 1.0);
+        s.STL = ul + c2 * al;
+        s.STR = ur - c2 * ar;
     }
     return s;
 }
@@ -729,7 +743,7 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
     double UL[N], UR[N];
 #pragma unroll
     for (int i = 0; i < N; i++) { UL[i] = double(ULr[i]); UR[i] = double(URr[i]); }
-    double il = 1.0 / UL[0], ir = 1.0 / UR[0];
+    const double il = frcp(UL[0]), ir = frcp(UR[0]);
     double vL[NM], vR[NM];
     double kL = 0.0, kR = 0.0;
 #pragma unroll
@@ -742,7 +756,7 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
     double pL = eos.GetPressure(UL[0], UL[N - 1] * il - kL / 2.0);
     double pR = eos.GetPressure(UR[0], UR[N - 1] * ir - kR / 2.0);
     double uL = vL[D], uR = vR[D];
-    StarDev st = star_state_dev(g, UL[0], uL, pL, UR[0], uR, pR);
+    const StarDev st = star_state_dev(g, UL[0], uL, pL, UR[0], uR, pR, il, ir);
     double ro, u, p;
     const double S = 0.0;
     bool left = st.vacuum ? (S <= 0.5 * (st.STL + st.STR)) : (st.u >= S);
@@ -762,12 +776,12 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
     if (cs == 0) { ro = rK; u = uK; p = pK; }
     else if (cs == 1) {
         // star density behind a shock (Toro eq. 4.50) or a rarefaction (eq. 4.53)
-        const double prK = st.p / pK;
+        const double prK = fdiv(st.p, pK);
         if (shockK) {
-            const double C = (g - 1.0) / (g + 1.0);
-            ro = (prK + C) / (C * prK + 1.0) * rK;
+            const double C = (g - 1.0) * frcp(g + 1.0);
+            ro = fdiv(prK + C, C * prK + 1.0) * rK;
         } else {
-            ro = rK * dpow(prK, 1.0 / g);
+            ro = rK * dpow(prK, frcp(g));
         }
         u = st.u;
         p = st.p;
@@ -776,11 +790,11 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
     else {
         // inside the fan (Toro eq. 4.56): C^(2/(g-1)) scales the density, and the pressure by
         // C^(2g/(g-1)) = C^(2/(g-1)) C^2
-        const double aK = __builtin_sqrt(g * pK / rK);
-        const double C = 2.0 / (g + 1) + sgn * ((g - 1) * (uK - S) / ((g + 1) * aK));
-        const double w = dpow(C, 2.0 / (g - 1));
+        const double aK = fsqrt(fdiv(g * pK, rK)), igp = frcp(g + 1);
+        const double C = igp * (2.0 + sgn * (g - 1) * fdiv(uK - S, aK));
+        const double w = dpow(C, 2.0 * frcp(g - 1));
         ro = w * rK;
-        u = (sgn * aK + 0.5 * (g - 1) * uK + S) * (2 / (g + 1));
+        u = (sgn * aK + 0.5 * (g - 1) * uK + S) * (2 * igp);
         p = w * C * C * pK;
     }
     double Vf[NM];
@@ -792,30 +806,16 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
 #pragma unroll
         for (int i = 0; i < N; i++) Fd[i] = 0.0;
     } else {
-        // Uface and F(Uface) (GodunovSolverPerfectGasEOS.h:416-427)
-        double U[N], k = 0.0;
-        U[0] = ro;
+        // the flux of the sampled state (GodunovSolverPerfectGasEOS.h:416-427)
+        double k = 0.0;
 #pragma unroll
-        for (int i = 0; i < NM; i++) {
-            U[1 + i] = ro * Vf[i];
-            k += Vf[i] * Vf[i];
-        }
-        U[N - 1] = ro * (eos.GetInternalEnergy(ro, p) + 0.5 * k);
-        const double iro = 1.0 / U[0];
-        double vv[NM];
-        k = 0.0;
+        for (int i = 0; i < NM; i++) k += Vf[i] * Vf[i];
+        const double un = Vf[D];
+        Fd[0] = ro * un;
 #pragma unroll
-        for (int i = 0; i < NM; i++) {
-            vv[i] = U[1 + i] * iro;
-            k += vv[i] * vv[i];
-        }
-        const double pp = eos.PressureOfEnergyDensity(U[N - 1] - U[0] * k / 2.0);
-        const double vn = vv[D];
-        Fd[0] = U[0] * vn;
-#pragma unroll
-        for (int i = 0; i < NM; i++) Fd[1 + i] = U[0] * vn * vv[i];
-        Fd[1 + D] += pp;
-        Fd[N - 1] = vn * (U[N - 1] + pp);
+        for (int i = 0; i < NM; i++) Fd[1 + i] = Fd[0] * Vf[i];
+        Fd[1 + D] += p;
+        Fd[N - 1] = un * (p * frcp(g - 1.0) + 0.5 * ro * k + p);
     }
 #pragma unroll
     for (int i = 0; i < N; i++) F[i] = R(Fd[i]);
