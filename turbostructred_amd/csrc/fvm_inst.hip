@@ -97,17 +97,19 @@ static void launch_vis(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
 }
 
 #if TS_DIM == 1
-template <int RC, int LM>
+template <int RC, int LM, int N>
 static void launch_euler1d_chunk(const KArgs& a, int steps, hipStream_t s) {
+    if (a.g.n[0] <= euler1d_cells<RC, N>) {
+        // a thread per face (faces 0..n), whole wavefronts
+        const int threads = (a.g.n[0] + 64) / 64 * 64;
+        hipLaunchKernelGGL((fvm_euler1d_lds<RC, LM, TS_FLUX, N>), dim3(1),
+                           dim3(threads < euler1d_threads<TS_FLUX> ? threads : euler1d_threads<TS_FLUX>), 0, s, a, steps);
+        return;
+    }
     KArgs b = a;  // the other direction of the ping-pong
     b.uin = a.uout;
     b.uout = const_cast<void*>(a.uin);
-    if (a.g.n[0] <= WG1D_LDS_CELLS)
-        hipLaunchKernelGGL((fvm_euler1d_workgroup<RC, LM, TS_FLUX, NV, true>), dim3(1), dim3(64 * wg1d_waves<TS_FLUX>), 0, s,
-                           a, b, steps);
-    else
-        hipLaunchKernelGGL((fvm_euler1d_workgroup<RC, LM, TS_FLUX, NV, false>), dim3(1), dim3(64 * wg1d_waves<TS_FLUX>), 0, s,
-                           a, b, steps);
+    hipLaunchKernelGGL((fvm_euler1d_workgroup<RC, LM, TS_FLUX, N>), dim3(1), dim3(64 * wg1d_waves<TS_FLUX>), 0, s, a, b, steps);
 }
 #endif
 
@@ -140,7 +142,7 @@ static void fill(int precision, KernelSet* ks) {
             ks->vrn = launch_vis<RC, LM, MODE_RN>;
         }
 #if TS_DIM == 1
-        ks->euler1d_chunk = launch_euler1d_chunk<RC, LM>;
+        ks->euler1d_chunk = launch_euler1d_chunk<RC, LM, N>;
 #endif
     } else {
         ks->dt = launch<RC, LM, N, MODE_DT, float, double, double>;

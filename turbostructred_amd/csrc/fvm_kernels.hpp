@@ -397,14 +397,11 @@ __device__ inline void add_sources(const VisArgs& v, const R (&u)[NV], double vo
 // VIS instances (FP64) add the viscous face fluxes of the pre-pass (subtracted from the convective
 // flux before it is differenced, ERK:1221-1222), the viscous spectral-radius term after each
 // plus face's eigenvalue, and the body-force sources after the flux sweeps.
-// DT_ARG instances take the step's dt from `dt_arg` instead of the control block in memory;
-// LDS_STATE instances read and write the state through `uin_arg` / `uout_arg` with plane stride
-// `plane_arg` (LDS arrays, addressed generically) with plain stores.
+// DT_ARG instances take the step's dt from `dt_arg` instead of the control block in memory.
 template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int N = NV,
-          int VIS = 0, bool DT_ARG = false, bool LDS_STATE = false, bool GP = false>
+          int VIS = 0, bool DT_ARG = false, bool GP = false>
 __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, double& block_min,
-                                           double* rn = nullptr, double dt_arg = 0.0, const void* uin_arg = nullptr,
-                                           void* uout_arg = nullptr, size_t plane_arg = 0) {
+                                           double* rn = nullptr, double dt_arg = 0.0) {
     using MT = ModeTraits<MODE>;
     static_assert(!VIS || N == NV, "viscous instances carry every variable");
     const GridArgs& g = a.g;
@@ -439,13 +436,12 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
     const double ev_x = ev_cells ? ld_geo<GP>(g.ev[0], xs) : 0.0;
     if (ev_cells && DIM == 1) geo.eps2 = R(ev_x);
 
-    const TIn* __restrict__ uin = LDS_STATE ? (const TIn*)uin_arg : (const TIn*)a.uin;
+    const TIn* __restrict__ uin = (const TIn*)a.uin;
     const TOut* __restrict__ lin = (const TOut*)a.lin;
-    TOut* uo = LDS_STATE ? (TOut*)uout_arg : (TOut*)a.uout;
-    const size_t P = LDS_STATE ? plane_arg : a.plane;
+    TOut* uo = (TOut*)a.uout;
+    const size_t P = a.plane;
     auto store = [&](int v, unsigned off, TOut x) {
-        if constexpr (LDS_STATE) st_plane(uo, P, v, off, x);
-        else st_state_stream<GP>(uo, P, v, off, x);
+        st_state_stream<GP>(uo, P, v, off, x);
     };
 
     // One stencil value, the input state at a (possibly ghost) cell of row r, in two steps: the
@@ -854,29 +850,186 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
 }
 
 // ---- small 1-D forward-Euler solves: a chunk of steps in one workgroup -------------------------
-// A grid of a few strips is launch-bound (two short kernels per step).  One workgroup of W
-// wavefronts runs up to `cap` steps of a ts_step call instead: the dt pass over its strips (each
-// wavefront takes strips w, w + W, ...), the workgroup minimum in LDS, the finalize by one
-// thread, a barrier, the forward-Euler stage into the other state buffer and a barrier before
-// the next dt pass reads it.  The two directions of the state ping-pong come as two kernel
-// arguments (a0: buffer 0 -> 1, a1: 1 -> 0), so that nothing is copied per step.  Every
-// wavefront leaves the loop together: after a step that ends the run (stop rule, error) or
-// after `cap` steps.  The control block lives in LDS for the chunk (thread 0 copies it in at the
-// start and back at the end), so the per-step bookkeeping -- the stop test, the dt update and
-// the stage's read of dt -- makes no global round trip.
-// W = 16 covers the 17 strips of 1000 cells in two rounds instead of three; the exact solver's
-// registers do not fit the 128 per lane of a 1024-thread workgroup, so Godunov keeps W = 8.
-// Grids of at most WG1D_LDS_CELLS cells keep both state buffers in LDS for the chunk (copied in
-// from the input buffer at the start, the final state copied out to the buffer the host expects
-// it in at the end): the dt pass and the stage then make no global round trip at all.
+// A grid of a few strips is launch-bound (two short kernels per step).  One workgroup runs up to
+// `cap` steps of a ts_step call instead.  Every wavefront leaves the loop together: after a step
+// that ends the run (stop rule, error) or after `cap` steps.
+//
+// Grids that fit keep the whole problem in LDS, a thread to each cell and to the face on its
+// minus side (strided where the cells outnumber the threads): the state, the face fluxes and
+// eigenvalues and the cell sizes; with a reconstruction also the plus-face states (the minus-face
+// ones wait in the places of the fluxes).  A face is evaluated once, for its eigenvalue and its
+// flux, and a step is the face pass, the minimum of V/SR, and the update, with three barriers (four
+// with a reconstruction).  What bounds it is the latency of that chain; each thread keeps time, dt
+// and the step count itself, so that no bookkeeping passes through memory.  (The former kernel walked
+// 60-cell strips twice per step, first for the eigenvalues and then for the fluxes, and 1000
+// cells are 17 strips: two rounds for 16 wavefronts.  1000 cells, first-order Roe:
+// 5.1 us per step, now 2.7.)
+template <int FLUX>
+constexpr int euler1d_threads = FLUX == FX_GODUNOV ? 512 : 1024;  // Godunov: over 128 registers
+constexpr int EULER1D_LDS = 20000;                               // doubles of the state and face arrays
+template <int RECON, int N>
+constexpr int euler1d_cells = EULER1D_LDS / (2 * N + 3 + (RECON == RC_PWC ? 0 : N)) - 1;
+
+// minimum over the wavefront, in lane 63 (row shifts, then row broadcasts)
+__device__ inline double wave_min_lane63(double v) {
+#define TS_MIN_STEP(ctrl)                                                              \
+    {                                                                                  \
+        const int lo = __double2loint(v), hi = __double2hiint(v);                      \
+        v = __builtin_fmin(v, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, ctrl, 0xF, 0xF, false), \
+                                               __builtin_amdgcn_update_dpp(lo, lo, ctrl, 0xF, 0xF, false))); \
+    }
+    TS_MIN_STEP(0x111) TS_MIN_STEP(0x112) TS_MIN_STEP(0x114) TS_MIN_STEP(0x118)  // row_shr 1, 2, 4, 8
+    TS_MIN_STEP(0x142) TS_MIN_STEP(0x143)                                        // row_bcast 15, 31
+#undef TS_MIN_STEP
+    return v;
+}
+// the same lane's value in every lane
+__device__ inline double read_lane63(double v) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63), __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// a0: input buffer 0 -> output buffer 1 of the ping-pong; the final state goes to buffer 0 after an
+// even number of steps and to buffer 1 after an odd one.  n <= euler1d_cells<RECON, N>.
+template <int RECON, int LIM, int FLUX, int N>
+__global__ void __launch_bounds__(euler1d_threads<FLUX>) fvm_euler1d_lds(KArgs a, int cap) {
+    const GridArgs& g = a.g;
+    const int n = g.n[0], T = blockDim.x, tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6, nwaves = T >> 6;
+    const bool per = g.periodic[0] != 0;
+    const int S = n + 1;  // plane stride: a plane holds the faces 0..n
+    __shared__ double pool[EULER1D_LDS];
+    __shared__ double red[16];
+    double* U = pool;           // [N][S] cells
+    double* F = U + N * S;      // [N][S] minus-face states, then fluxes, of faces 0..n
+    double* lam = F + N * S;    // [S] eigenvalues of the faces
+    double* h = lam + S;        // [S] sizes of cells 0..n (n: the right ghost)
+    double* ih = h + S;         // [S]
+    double* FP = ih + S;        // [N][S] plus-face states (RECON != PWC)
+    StepCtl* ctl = a.ctl;
+    const double* u0 = (const double*)a.uin;
+    for (int c = tid; c <= n; c += T) {
+        h[c] = g.h[0][c + 1];
+        ih[c] = g.ih[0][c + 1];
+        if (c < n)
+#pragma unroll
+            for (int v = 0; v < N; v++) U[v * S + c] = ld_plane(u0, a.plane, plane_of<N>(v), unsigned(c));
+    }
+    double time = ctl->time, dt = ctl->dt;
+    const double t_max = ctl->t_max, next_snap = ctl->next_snap;
+    const long long iter0 = ctl->iter;
+    const int sd0 = ctl->steps_done, max_steps = ctl->max_steps;
+    bool active = ctl->active != 0, failed = false;
+    int done = 0;
+    __syncthreads();
+    while (active && done < cap) {
+        if constexpr (RECON != RC_PWC) {
+            for (int c = tid; c < n; c += T) {
+                double u[N], nb[2][N], face[2][N];
+                const int l = c > 0 ? c - 1 : (per ? n - 1 : 0), r = c < n - 1 ? c + 1 : (per ? 0 : n - 1);
+#pragma unroll
+                for (int v = 0; v < N; v++) {
+                    u[v] = U[v * S + c];
+                    nb[0][v] = U[v * S + l];
+                    nb[1][v] = U[v * S + r];
+                }
+                if (!per && c == 0) bc_image(g.bc[bc_marker(g, 0, 0)], g.gamma, 0, u, nb[0]);
+                if (!per && c == n - 1) bc_image(g.bc[bc_marker(g, 1, 0)], g.gamma, 0, u, nb[1]);
+                CellGeo<1, double> geo;
+                geo.hh[0] = 0.5 * h[c];
+                geo.rc[0] = g.rc[0][c];
+                geo.rl[0] = g.rl[0][c];
+                geo.rr[0] = g.rr[0][c];
+                geo.eps2 = (RECON == RC_LINLIM && LIM == LIM_VENKAT && g.ev[0]) ? g.ev[0][c] : g.eps2;
+                reconstruct<1, RECON, LIM, double, FLUX != FX_ROE>(u, nb, geo, face);
+#pragma unroll
+                for (int v = 0; v < N; v++) {
+                    F[v * S + c] = face[0][v];
+                    FP[v * S + c] = face[1][v];
+                    if (per && c == 0) F[v * S + n] = face[0][v];
+                }
+            }
+            __syncthreads();
+        }
+        // faces: the state on the minus side, the state on the plus side, eigenvalue and flux
+        for (int c = tid; c <= n; c += T) {
+            const double* L = RECON == RC_PWC ? U : FP;
+            const double* R = RECON == RC_PWC ? U : F;
+            const int l = c > 0 ? c - 1 : (per ? n - 1 : 0);
+            const int r = (RECON == RC_PWC && c == n) ? (per ? 0 : n - 1) : c;
+            double UL[N], UR[N], Fx[N], lx;
+#pragma unroll
+            for (int v = 0; v < N; v++) {
+                UL[v] = L[v * S + l];
+                UR[v] = R[v * S + r];
+            }
+            if (!per && c == 0) bc_image(g.bc[bc_marker(g, 0, 0)], g.gamma, 0, UR, UL);
+            if (!per && c == n) bc_image(g.bc[bc_marker(g, 1, 0)], g.gamma, 0, UL, UR);
+            face_flux<FLUX, 0, double>(g.gamma, g.eps, UL, UR, Fx, lx);
+            lam[c] = lx;
+#pragma unroll
+            for (int v = 0; v < N; v++) F[v * S + c] = Fx[v];
+        }
+        __syncthreads();
+        double m = __builtin_inf();
+        for (int c = tid; c <= n; c += T) {
+            const double sr = c < n ? lam[c] + lam[c + 1] : lam[n];  // the right ghost cell has one face
+            m = __builtin_fmin(m, dt_candidate(h[c], sr));
+        }
+        m = wave_min_lane63(m);
+        if (lane == 63) red[wave] = m;
+        __syncthreads();
+        m = read_lane63(wave_min_lane63(red[lane < nwaves ? lane : 0]));
+        // dt_apply's rule, by every thread
+        double dtn = m * g.cfl;
+        if (next_snap > 0 && next_snap < time + dtn) dtn = next_snap - time;
+        if (!(dtn > 0.0) || !(dtn < __builtin_inf())) {
+            failed = true;
+            break;  // the state of the last good step stays in place
+        }
+        dt = dtn;
+        time += dtn;
+        for (int c = tid; c < n; c += T) {
+            const double iv = ih[c];
+#pragma unroll
+            for (int v = 0; v < N; v++) U[v * S + c] += dtn * ((F[v * S + c] - F[v * S + c + 1]) * iv);
+        }
+        if (tid == 0 && ctl->dt_log) {
+            const long long li = iter0 + done - ctl->dt_log_base;
+            if (li >= 0 && li < ctl->dt_log_cap) ctl->dt_log[li] = dtn;
+        }
+        done++;
+        active = !((time >= t_max) || (next_snap > 0 && time == next_snap) || (sd0 + done >= max_steps));
+        __syncthreads();
+    }
+    double* out = (done & 1) ? (double*)a.uout : (double*)const_cast<void*>(a.uin);
+    for (int c = tid; c < n; c += T)
+#pragma unroll
+        for (int v = 0; v < N; v++) st_plane(out, a.plane, plane_of<N>(v), unsigned(c), U[v * S + c]);
+    if (tid == 0) {
+        ctl->time = time;
+        ctl->dt = dt;
+        ctl->iter = iter0 + done;
+        ctl->steps_done = sd0 + done;
+        ctl->active = active && !failed ? 1 : 0;
+        ctl->go = active && !failed ? 1 : 0;
+        if (failed) ctl->error = 1;
+    }
+}
+
+// Larger grids (up to 64 strips) keep the state in memory: the dt pass over the workgroup's strips
+// (each wavefront takes strips w, w + W, ...), the workgroup minimum in LDS, the finalize by one
+// thread, a barrier, the forward-Euler stage into the other state buffer and a barrier before the
+// next dt pass reads it.  The two directions of the state ping-pong come as two kernel arguments
+// (a0: buffer 0 -> 1, a1: 1 -> 0), so that nothing is copied per step; the control block lives in
+// LDS for the chunk (thread 0 copies it in at the start and back at the end).  The exact
+// solver's registers do not fit the 128 per lane of a 1024-thread workgroup, so Godunov has 8
+// wavefronts instead of 16.
 template <int FLUX>
 constexpr int wg1d_waves = FLUX == FX_GODUNOV ? 8 : 16;
-constexpr int WG1D_LDS_CELLS = 1984;  // 2 buffers x 5 planes x 1984 doubles = 158720 bytes
 
 // one step; false when the loop has to end
-template <int RECON, int LIM, int FLUX, int N, bool LDS>
-__device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, double* red, int* run, int lane,
-                                             int wave, const double* sin, double* sout) {
+template <int RECON, int LIM, int FLUX, int N>
+__device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, double* red, int* run, int lane, int wave) {
     if (threadIdx.x == 0) *run = ctl->active;
     __syncthreads();
     if (!*run) {
@@ -886,8 +1039,7 @@ __device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, doubl
     double m = __builtin_inf();
     for (int tile = wave; tile < a.ntiles; tile += wg1d_waves<FLUX>) {
         double mt = __builtin_inf();
-        stage_tile<1, RECON, LIM, FLUX, MODE_DT, double, double, double, N, 0, false, LDS, false>(
-            a, tile, lane, mt, nullptr, 0.0, sin, sout, WG1D_LDS_CELLS);
+        stage_tile<1, RECON, LIM, FLUX, MODE_DT, double, double, double, N>(a, tile, lane, mt);
         m = __builtin_fmin(m, mt);
     }
 #pragma unroll
@@ -906,49 +1058,23 @@ __device__ __forceinline__ bool euler1d_step(const KArgs& a, StepCtl* ctl, doubl
     const double dt = ctl->dt;
     for (int tile = wave; tile < a.ntiles; tile += wg1d_waves<FLUX>) {
         double unused = 0.0;
-        stage_tile<1, RECON, LIM, FLUX, MODE_S1, double, double, double, N, 0, true, LDS, false>(
-            a, tile, lane, unused, nullptr, dt, sin, sout, WG1D_LDS_CELLS);
+        stage_tile<1, RECON, LIM, FLUX, MODE_S1, double, double, double, N, 0, true>(a, tile, lane, unused, nullptr, dt);
     }
     __syncthreads();
     return true;
 }
 
-template <int RECON, int LIM, int FLUX, int N, bool LDS>
+template <int RECON, int LIM, int FLUX, int N>
 __global__ void __launch_bounds__(64 * wg1d_waves<FLUX>) fvm_euler1d_workgroup(KArgs a0, KArgs a1, int cap) {
-    constexpr int NT = 64 * wg1d_waves<FLUX>;
     __shared__ double red[wg1d_waves<FLUX>];
     __shared__ int run;
     __shared__ StepCtl ctl;  // a0.ctl and a1.ctl are the same block
-    __shared__ double st[LDS ? 2 * N * WG1D_LDS_CELLS : 1];
-    double* b0 = st;
-    double* b1 = st + (LDS ? N * WG1D_LDS_CELLS : 0);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int ncell = a0.g.n[0];  // at most WG1D_LDS_CELLS when LDS (checked by the launcher)
     if (threadIdx.x == 0) ctl = *a0.ctl;  // read only by thread 0 until the first barrier
-    if constexpr (LDS) {
-        const double* g = (const double*)a0.uin;
-        for (int c = threadIdx.x; c < ncell; c += NT)
-#pragma unroll
-            for (int v = 0; v < N; v++) b0[v * WG1D_LDS_CELLS + c] = g[(size_t)v * a0.plane + c];
-        __syncthreads();
-    }
-    int done = 0;  // uniform: every wavefront takes the same branches
     for (int it = 0; it < cap; it += 2) {
-        if (!euler1d_step<RECON, LIM, FLUX, N, LDS>(a0, &ctl, red, &run, lane, wave, b0, b1)) break;
-        done++;
+        if (!euler1d_step<RECON, LIM, FLUX, N>(a0, &ctl, red, &run, lane, wave)) break;
         if (it + 1 >= cap) break;
-        if (!euler1d_step<RECON, LIM, FLUX, N, LDS>(a1, &ctl, red, &run, lane, wave, b1, b0)) break;
-        done++;
-    }
-    if constexpr (LDS) {
-        // the state after `done` steps is in b0 (even) or b1 (odd); the host expects it in the
-        // input buffer after an even number of steps and in the other one after an odd number.
-        // Every step ends at a barrier, and one that stops early writes no state after it.
-        const double* src = (done & 1) ? b1 : b0;
-        double* g = (done & 1) ? (double*)a0.uout : (double*)const_cast<void*>(a0.uin);
-        for (int c = threadIdx.x; c < ncell; c += NT)
-#pragma unroll
-            for (int v = 0; v < N; v++) g[(size_t)v * a0.plane + c] = src[v * WG1D_LDS_CELLS + c];
+        if (!euler1d_step<RECON, LIM, FLUX, N>(a1, &ctl, red, &run, lane, wave)) break;
     }
     if (threadIdx.x == 0) *a0.ctl = ctl;  // the other threads only ever read the LDS copy
 }
@@ -994,11 +1120,11 @@ __global__ void __launch_bounds__(256) fvm_stage_batched(const KArgs* __restrict
             const int s1 = (s0 + a.ty < a.ntiles) ? s0 + a.ty : a.ntiles;
             for (int sidx = s0; sidx < s1; sidx++) {
                 double ms = __builtin_inf();
-                stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, false, true>(a, sidx, lane, ms);
+                stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, true>(a, sidx, lane, ms);
                 m = __builtin_fmin(m, ms);
             }
         } else {
-            stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, false, true>(a, e.y, lane, m);
+            stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, true>(a, e.y, lane, m);
         }
         if constexpr (MT::sr) {
             // the entry's minimum; dt_finalize_batched reduces each solve's entries after the launch
