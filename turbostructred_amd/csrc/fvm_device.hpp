@@ -217,19 +217,16 @@ struct CellGeo {
     R eps2;     // Venkatakrishnan (K dx)^3 (Limiters.h:93-96)
 };
 
-// Reconstruct one cell and return its face states: face[2a] on the minus face of axis a,
-// face[2a+1] on the plus face.  nb[2a], nb[2a+1] are the axis neighbours (x-,x+,y-,y+,z-,z+),
-// the stencil of ComputeSolutionReconstruction (ERK:897-916).
-// With POS set (the HLLC and exact-Godunov paths, which need a real sound speed), a face state
-// with rho <= 0 or 2 rho E <= |m|^2 falls back to the cell value.
-template <int ND, int RECON, int LIM, typename R, bool POS = false, int N>
-__device__ inline void reconstruct(const R (&c)[N], const R (&nb)[2 * ND][N],
-                                   const CellGeo<ND, R>& geo, R (&face)[2 * ND][N]) {
+// Reconstruct one cell: its state on the minus face of axis a is c - t[a], on the plus face c + t[a].
+// nb[2a], nb[2a+1] are the axis neighbours (x-,x+,y-,y+,z-,z+), the stencil of
+// ComputeSolutionReconstruction (ERK:897-916).
+template <int ND, int RECON, int LIM, typename R, int N>
+__device__ inline void face_offsets(const R (&c)[N], const R (&nb)[2 * ND][N], const CellGeo<ND, R>& geo, R (&t)[ND][N]) {
 #pragma unroll
     for (int v = 0; v < N; v++) {
         if constexpr (RECON == RC_PWC) {  // PiecewiseConstant.h:15
 #pragma unroll
-            for (int f = 0; f < 2 * ND; f++) face[f][v] = c[v];
+            for (int a = 0; a < ND; a++) t[a][v] = R(0);
         } else if constexpr (RECON == RC_LINLIM && LIM == LIM_BJ) {
             // Limited linear with Barth-Jespersen (Linear2psLim.h:64-96, Limiters.h:28-67,80-82).
             // Along each axis the two face projections are +-d_a, d_a = g_a h_a / 2 with the
@@ -258,11 +255,7 @@ __device__ inline void reconstruct(const R (&c)[N], const R (&nb)[2 * ND][N],
             const R hi = umax - c[v], lo = c[v] - umin;
             const R lim = vmin(fdiv(vmin(hi, lo), dmax), R(1));
 #pragma unroll
-            for (int a = 0; a < ND; a++) {
-                const R t = lim * d[a];
-                face[2 * a][v] = c[v] - t;
-                face[2 * a + 1][v] = c[v] + t;
-            }
+            for (int a = 0; a < ND; a++) t[a][v] = lim * d[a];
         } else {
             R g[ND];
 #pragma unroll
@@ -318,24 +311,42 @@ __device__ inline void reconstruct(const R (&c)[N], const R (&nb)[2 * ND][N],
             }
 #pragma unroll
             for (int a = 0; a < ND; a++) {
-                R d = g[a] * geo.hh[a];
-                if constexpr (RECON == RC_LINLIM) {  // Linear2psLim.h:17-21 (Venkatakrishnan)
-                    face[2 * a][v] = c[v] + lim * (g[a] * (-geo.hh[a]));
-                    face[2 * a + 1][v] = c[v] + lim * d;
-                } else {  // Linear2PointsStencil.h:26-30
-                    face[2 * a][v] = c[v] - d;
-                    face[2 * a + 1][v] = c[v] + d;
-                }
+                t[a][v] = g[a] * geo.hh[a];  // Linear2PointsStencil.h:26-30
+                if constexpr (RECON == RC_LINLIM) t[a][v] *= lim;  // Linear2psLim.h:17-21
             }
         }
+    }
+}
+
+// whether a state has no real sound speed (rho <= 0 or 2 rho E <= |m|^2)
+template <typename R, int N>
+__device__ __forceinline__ bool no_sound_speed(const R (&u)[N]) {
+    return !(u[0] > R(0) && R(2) * u[0] * u[N - 1] - momentum2(u) > R(0));
+}
+
+// The face states themselves, face[2a] on the minus face of axis a and face[2a+1] on the plus face.
+// With POS set (the HLLC and exact-Godunov paths), a face state without a real sound speed falls
+// back to the cell value.
+template <int ND, int RECON, int LIM, typename R, bool POS = false, int N>
+__device__ inline void reconstruct(const R (&c)[N], const R (&nb)[2 * ND][N],
+                                   const CellGeo<ND, R>& geo, R (&face)[2 * ND][N]) {
+    {
+        R t[ND][N];
+        face_offsets<ND, RECON, LIM>(c, nb, geo, t);
+#pragma unroll
+        for (int a = 0; a < ND; a++)
+#pragma unroll
+            for (int v = 0; v < N; v++) {
+                face[2 * a][v] = c[v] - t[a][v];
+                face[2 * a + 1][v] = c[v] + t[a][v];
+            }
     }
     if constexpr (POS && RECON != RC_PWC) {
         bool bad[2 * ND];
         bool any = false;
 #pragma unroll
         for (int f = 0; f < 2 * ND; f++) {
-            R q = R(2) * face[f][0] * face[f][N - 1] - momentum2(face[f]);
-            bad[f] = !(face[f][0] > R(0) && q > R(0));
+            bad[f] = no_sound_speed(face[f]);
             any = any || bad[f];
         }
         // rare: a branch the wavefront skips when none of its lanes needs the fallback

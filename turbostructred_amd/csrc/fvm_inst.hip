@@ -22,10 +22,20 @@
 namespace tsd {
 
 #if !(TS_DIM == 3 && !defined(TS_HAVE_3D))
+#if TS_DIM == 3
+// one workgroup per tile: strips, row blocks, and blocks of the z-planes the instance outputs
+template <typename R, int VIS, int MODE>
+static dim3 grid3d(const KArgs& a) {
+    constexpr int zout = z_waves<R, VIS, MODE> - 2;
+    return dim3(a.nstrips * ((a.g.n[1] + a.ty - 1) / a.ty) * ((a.g.n[2] + zout - 1) / zout));
+}
+#endif
 template <int RC, int LM, int N, int MODE, typename R, typename TIn, typename TOut>
 static void launch(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
 #if TS_DIM == 3
-    hipLaunchKernelGGL((fvm_stage3d<RC, LM, TS_FLUX, MODE, R, TIn, TOut>), g, b, 0, s, a);
+    KArgs b3 = a;
+    if (MODE == MODE_F2) b3.ty = a.ty2;
+    hipLaunchKernelGGL((fvm_stage3d<RC, LM, TS_FLUX, MODE, R, TIn, TOut>), (grid3d<R, 0, MODE>(b3)), dim3(64 * (z_waves<R, 0, MODE>)), 0, s, b3);
 #else
     hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, R, TIn, TOut, N>), g, b, 0, s, a);
 #endif
@@ -42,16 +52,17 @@ template <typename K> static int blocks_per_cu(K kernel, int threads) {
 template <int RC, int LM, int N, typename R, typename S, typename E>
 static int single_occupancy() {
 #if TS_DIM == 3
-    const int T = 64 * ZW;
+#define TS_T(MODE) 64 * z_waves<R, 0, MODE>
 #define TS_K(MODE, A, B, C) fvm_stage3d<RC, LM, TS_FLUX, MODE, A, B, C>
 #else
-    const int T = 256;
+#define TS_T(MODE) 256
 #define TS_K(MODE, A, B, C) fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, A, B, C, N>
 #endif
-    int m = blocks_per_cu(TS_K(MODE_F1, R, double, S), T);
-    int v[] = {blocks_per_cu(TS_K(MODE_F2, R, double, S), T), blocks_per_cu(TS_K(MODE_S3, R, S, double), T),
-               blocks_per_cu(TS_K(MODE_DT, R, double, double), T), blocks_per_cu(TS_K(MODE_S1, R, double, E), T)};
+    int m = blocks_per_cu(TS_K(MODE_F1, R, double, S), TS_T(MODE_F1));
+    int v[] = {blocks_per_cu(TS_K(MODE_F2, R, double, S), TS_T(MODE_F2)), blocks_per_cu(TS_K(MODE_S3, R, S, double), TS_T(MODE_S3)),
+               blocks_per_cu(TS_K(MODE_DT, R, double, double), TS_T(MODE_DT)), blocks_per_cu(TS_K(MODE_S1, R, double, E), TS_T(MODE_S1))};
 #undef TS_K
+#undef TS_T
     for (int x : v) m = x < m ? x : m;
     return m;
 }
@@ -89,7 +100,8 @@ static void launch_vis_prepass(const KArgs& a, dim3, dim3, hipStream_t s) {
 template <int RC, int LM, int MODE>
 static void launch_vis(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
 #if TS_DIM == 3
-    hipLaunchKernelGGL((fvm_stage3d<RC, LM, TS_FLUX, MODE, double, double, double, 1>), g, b, 0, s, a);
+    hipLaunchKernelGGL((fvm_stage3d<RC, LM, TS_FLUX, MODE, double, double, double, 1>), (grid3d<double, 1, MODE>(a)),
+                       dim3(64 * (z_waves<double, 1, MODE>)), 0, s, a);
 #else
     hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, double, double, double, NV, 1>), g, b, 0, s, a);
 #endif

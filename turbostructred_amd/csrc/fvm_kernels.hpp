@@ -37,8 +37,13 @@ namespace tsd {
 
 enum : int { MODE_DT = 0, MODE_S1 = 1, MODE_S2 = 2, MODE_S3 = 3, MODE_F1 = 4, MODE_F2 = 5, MODE_RN = 6 };
 constexpr int STRIP = 60;   // output columns per wavefront
-constexpr int ZW = 8;         // wavefronts (z-planes) per 3-D workgroup
-constexpr int ZOUT = ZW - 2;  // output z-planes per 3-D workgroup
+// Wavefronts (z-planes) per 3-D workgroup; all but two produce output.  In double, whose kernels
+// hold about 200 registers, a SIMD takes two.  In float four fit, but stage 2 then spills 15 registers
+// of its two prefetched rows: three (256^3: 899 us against 1078 with four).
+template <typename R, int VIS, int MODE>
+constexpr int z_waves = sizeof(R) == 8 ? 8 : (MODE == MODE_F2 ? 12 : 16);
+// output planes of stage 2 and of the others (which set the number of dt minima)
+constexpr int z_out_of(int real_bytes, bool stage2) { return (real_bytes == 8 ? 8 : stage2 ? 12 : 16) - 2; }
 constexpr int MAX_BC = 8;
 
 // Device-resident control block of one solve: the step bookkeeping of StepInfo (kernel.h:56) and
@@ -104,6 +109,7 @@ struct KArgs {
     size_t plane;      // cells per plane
     StepCtl* ctl;
     int ty;            // output rows per tile
+    int ty2;           // the same for 3-D fused stage 2, whose workgroups output other planes in float
     int nstrips;       // strips along x
     int ntiles;        // strips * row blocks
     double* rn_part;   // per-block partial residual norms, 5 per block (MODE_RN)

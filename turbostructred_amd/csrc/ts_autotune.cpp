@@ -45,7 +45,7 @@ double march_cost(long long tiles, int ty, long long units, int occ) {
     return c * (ty + 2);
 }
 
-int tuned_rows_per_tile(const ts_config& c, long long units, int occ) {
+int tuned_rows_per_tile(const ts_config& c, int zout, long long units, int occ) {
     if (c.ndims == 1) return 1;
     {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -53,7 +53,7 @@ int tuned_rows_per_tile(const ts_config& c, long long units, int occ) {
         if (it != g_table.end()) return it->second;
     }
     const long long strips = (c.nx + 59) / 60;
-    const long long zb = c.ndims == 3 ? (c.nz + 5) / 6 : 1;  // z blocks of a 3-D tile column
+    const long long zb = (c.nz + zout - 1) / zout;  // z blocks of a 3-D tile column
     if (units <= 0 || occ <= 0) {
         // no occupancy known: enough tiles to fill 256 CUs several times over, at most 32 rows
         long long rows = (long long)c.ny * zb;
@@ -111,7 +111,8 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
             const int m = c->ty;
             cands = {m, m > 1 ? m - (m + 3) / 4 : 1, m + m / 4 + 1};
             const long long strips = c->nstrips, tiles_m = c->ntiles;
-            const long long zb = cfg->ndims == 3 ? (cfg->nz + tsd::ZOUT - 1) / tsd::ZOUT : 1;
+            const int zout = tsd::z_out_of(cfg->precision == TS_FP64 ? 8 : 4, false);
+            const long long zb = cfg->ndims == 3 ? (cfg->nz + zout - 1) / zout : 1;
             // slots implied by the model's choice: its tile count rounded up to a whole round
             for (long long rounds = 1; rounds <= 2; rounds++) {
                 const long long target = tiles_m * rounds;

@@ -46,14 +46,14 @@ struct ts_ctx {
     // grid's axes.
     struct Variant {
         tsd::KernelSet ks;
-        int ty = 16, ntiles = 1;
+        int ty = 16, ty2 = 16, ntiles = 1;
         dim3 grid_dim;
     };
     Variant variant[2];
     bool may_reduce = false, reduced = false;
     size_t most_blocks = 1;  // of the variants' grids
     tsd::KernelSet ks;
-    int ty = 16;
+    int ty = 16, ty2 = 16;  // rows per tile (ty2: 3-D stage 2)
     int nstrips = 1, ntiles = 1;
     dim3 grid_dim, block_dim;
 
@@ -111,9 +111,9 @@ bool lookup_kernels(int dim, int flux, int rv, int precision, bool in_grid, tsd:
 // whether no boundary condition of the table can give momentum out of the grid's axes (1-D, 2-D)
 bool boundaries_in_grid(const ts_config& c);
 void host_bc_image(const ts_bc_config& bc, double g, int axis, const double* u, double* o);
-// output rows per tile; the GPU holds `occ` tiles on each of `units` SIMDs (3-D: CUs) at once
-// (0: unknown)
-int tuned_rows_per_tile(const ts_config& c, long long units, int occ);
+// output rows per tile of `zout` planes (1 below 3-D); the GPU holds `occ` tiles on each of `units`
+// SIMDs (3-D: CUs) at once (0: unknown)
+int tuned_rows_per_tile(const ts_config& c, int zout, long long units, int occ);
 // modelled time of marching `tiles` tiles of ty rows
 double march_cost(long long tiles, int ty, long long units, int occ);
 // the calling thread's error text for entry points without a context (ts_last_error(NULL))

@@ -69,16 +69,13 @@ constexpr int CHUNK = 256;  // steps issued between host checks of the terminati
 // workgroups per CU of its kernels, tiles and grid.
 void tile_variant(const ts_ctx* c, const ts_config& cfg, ts_ctx::Variant& v) {
     const int per_block = c->nd == 3 ? 1 : 4;  // 1-D, 2-D: a tile (1-D: a strip) per wavefront, four to a block
-    int cus = 0;
-    if (c->nd == 1) {
-        v.ty = 1;
-    } else if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device) != hipSuccess || !v.ks.socc) {
-        v.ty = tsr::tuned_rows_per_tile(cfg, 0, 0);
-    } else {
-        v.ty = tsr::tuned_rows_per_tile(cfg, (long long)cus * per_block, v.ks.socc());
-    }
+    const int real = cfg.precision == TS_FP64 ? 8 : 4, zout = c->nd > 2 ? z_out_of(real, false) : 1;
+    int cus = 0, occ = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device) == hipSuccess && v.ks.socc) occ = v.ks.socc();
+    v.ty = tsr::tuned_rows_per_tile(cfg, zout, (long long)cus * per_block, occ);
+    v.ty2 = c->nd > 2 ? tsr::tuned_rows_per_tile(cfg, z_out_of(real, true), cus, occ) : v.ty;
     const int nyb = c->nd > 1 ? (c->n[1] + v.ty - 1) / v.ty : 1;
-    const int nzb = c->nd > 2 ? (c->n[2] + ZOUT - 1) / ZOUT : 1;
+    const int nzb = (c->n[2] + zout - 1) / zout;
     v.ntiles = c->nstrips * nyb * nzb;
     v.grid_dim = dim3((v.ntiles + per_block - 1) / per_block);
 }
@@ -228,7 +225,7 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
     // out of the grid's axes, of those that leave them out (borrowed-memory calls do not inspect
     // the state)
     c->nstrips = (c->n[0] + STRIP - 1) / STRIP;
-    c->block_dim = dim3(c->nd == 3 ? 64 * ZW : 256);
+    c->block_dim = dim3(256);
     c->variant[0].ks = c->ks;
     c->may_reduce = !c->arena && !c->vis && (k.rk_stages == 1 || c->fused_dt) && tsr::boundaries_in_grid(k) &&
                     tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, true, &c->variant[1].ks);
@@ -271,6 +268,7 @@ int use_variant(ts_ctx* c, bool reduced) {
     c->reduced = reduced;
     c->ks = v.ks;
     c->ty = v.ty;
+    c->ty2 = v.ty2;
     c->ntiles = v.ntiles;
     c->grid_dim = v.grid_dim;
     return TS_OK;
@@ -343,6 +341,7 @@ void step_launches(const ts_ctx* c, int start_buf, int s, Launch (&L)[MAX_LAUNCH
     a.plane = c->ncell;
     a.ctl = c->dctl;
     a.ty = c->ty;
+    a.ty2 = c->ty2;
     a.nstrips = c->nstrips;
     a.ntiles = c->ntiles;
     a.un = (const double*)c->dU[0];
