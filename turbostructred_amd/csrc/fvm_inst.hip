@@ -39,7 +39,9 @@ static void launch(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
 #else
     hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, R, TIn, TOut, N>), g, b, 0, s, a);
 #endif
-    if constexpr (ModeTraits<MODE>::sr) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, a.ntiles);
+    if constexpr (ModeTraits<MODE>::sr) {
+        if (!a.dt_minima) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, a.ntiles);
+    }
 }
 
 // resident workgroups per CU of the single-solve stage kernels (the minimum over the kernels of

@@ -114,6 +114,8 @@ struct KArgs {
     int ntiles;        // strips * row blocks
     double* rn_part;   // per-block partial residual norms, 5 per block (MODE_RN)
     double* dt_part;   // single solves: each tile's minimum of V/SR (dt passes, fused stage 1)
+    int dt_minima;     // fused stages 2 and 3: number of those minima where they apply the step's dt
+                       // themselves (see step_dt); 0 where dt_finalize_kernel has done it
 };
 
 // ---- wave-level helpers -------------------------------------------------------------------------
@@ -249,30 +251,82 @@ __device__ inline double dt_candidate(double vol, double sr) {
 }
 
 // dt = min(V/SR) * CFL (ERK:1430) from the grid minimum mn, clamped to the next snapshot
-// (ERK:1433); advances Time / Iteration, logs dt and evaluates the stop rule of Kernel::Run
-// (kernel.h:1834-1846).  One thread.
-__device__ inline void dt_apply(StepCtl* ctl, double cfl, double mn) {
-    double dtn = mn * cfl;
-    double t0 = ctl->time;
+// (ERK:1433); false where it is not finite and positive
+__device__ inline bool dt_rule(const StepCtl* ctl, double cfl, double mn, double& dtn) {
+    dtn = mn * cfl;
+    const double t0 = ctl->time;
     if (ctl->next_snap > 0 && ctl->next_snap < t0 + dtn) dtn = ctl->next_snap - t0;
-    if (!(dtn > 0.0) || !(dtn < __builtin_inf())) {
-        ctl->error = 1;
-        ctl->go = 0;
-        ctl->active = 0;
-    } else {
-        double t1 = t0 + dtn;
-        ctl->dt = dtn;
-        ctl->time = t1;
-        long long it = ctl->iter;
-        ctl->iter = it + 1;
-        int sd = ctl->steps_done + 1;
-        ctl->steps_done = sd;
-        long long li = it - ctl->dt_log_base;
-        if (ctl->dt_log && li >= 0 && li < ctl->dt_log_cap) ctl->dt_log[li] = dtn;
-        ctl->go = 1;
-        bool stop = (t1 >= ctl->t_max) || (ctl->next_snap > 0 && t1 == ctl->next_snap) || (sd >= ctl->max_steps);
-        ctl->active = stop ? 0 : 1;
+    return dtn > 0.0 && dtn < __builtin_inf();
+}
+__device__ inline void step_fails(StepCtl* ctl) {
+    ctl->error = 1;
+    ctl->go = 0;
+    ctl->active = 0;
+}
+// advances Time / Iteration, logs dt and evaluates the stop rule of Kernel::Run
+// (kernel.h:1834-1846).  One thread.
+__device__ inline void step_advances(StepCtl* ctl, double dtn) {
+    const double t1 = ctl->time + dtn;
+    ctl->time = t1;
+    long long it = ctl->iter;
+    ctl->iter = it + 1;
+    int sd = ctl->steps_done + 1;
+    ctl->steps_done = sd;
+    long long li = it - ctl->dt_log_base;
+    if (ctl->dt_log && li >= 0 && li < ctl->dt_log_cap) ctl->dt_log[li] = dtn;
+    bool stop = (t1 >= ctl->t_max) || (ctl->next_snap > 0 && t1 == ctl->next_snap) || (sd >= ctl->max_steps);
+    ctl->active = stop ? 0 : 1;
+}
+// the step's dt from the grid minimum.  One thread.
+__device__ inline void dt_apply(StepCtl* ctl, double cfl, double mn) {
+    double dtn;
+    if (!dt_rule(ctl, cfl, mn, dtn)) {
+        step_fails(ctl);
+        return;
     }
+    ctl->dt = dtn;
+    ctl->go = 1;
+    step_advances(ctl, dtn);
+}
+
+// minimum over the wavefront, in lane 63 (row shifts, then row broadcasts)
+__device__ inline double wave_min_lane63(double v) {
+#define TS_MIN_STEP(ctrl)                                                              \
+    {                                                                                  \
+        const int lo = __double2loint(v), hi = __double2hiint(v);                      \
+        v = __builtin_fmin(v, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, ctrl, 0xF, 0xF, false), \
+                                               __builtin_amdgcn_update_dpp(lo, lo, ctrl, 0xF, 0xF, false))); \
+    }
+    TS_MIN_STEP(0x111) TS_MIN_STEP(0x112) TS_MIN_STEP(0x114) TS_MIN_STEP(0x118)  // row_shr 1, 2, 4, 8
+    TS_MIN_STEP(0x142) TS_MIN_STEP(0x143)                                        // row_bcast 15, 31
+#undef TS_MIN_STEP
+    return v;
+}
+// the same lane's value in every lane
+__device__ inline double read_lane63(double v) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63), __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// A launch between stage 1 and stage 2 for one reduction costs 4 to 5 us, a tenth of the step of a
+// small grid.  Where the minima are few, every wavefront of stage 2 reduces them itself and so
+// knows the step's dt (the minimum is exact: all get the same); `first` marks the one that writes
+// what stage 3 reads, dt and go.  Time, the step count and the stop rule, which the other wavefronts
+// of stage 2 still read, are advanced by stage 3.  False where the step does not run.
+__device__ inline bool step_dt(StepCtl* ctl, double cfl, const double* part, int n, int lane, bool first, double& dt) {
+    double m = __builtin_inf();
+    for (int i = lane; i < n; i += 64) m = __builtin_fmin(m, part[i]);
+    if (!ctl->active) return false;  // stage 1 has cleared go
+    m = read_lane63(wave_min_lane63(m));
+    const bool ok = dt_rule(ctl, cfl, m, dt);
+    if (first && lane == 0) {
+        if (ok) {
+            ctl->dt = dt;
+            ctl->go = 1;
+        } else {
+            step_fails(ctl);
+        }
+    }
+    return ok;
 }
 
 // Single solves: the step's dt from the `n` per-tile minima of V/SR that a dt pass or fused
@@ -297,7 +351,7 @@ __global__ void __launch_bounds__(1024) dt_finalize_kernel(StepCtl* ctl, double 
     }
 }
 
-// Batched solves: the dt of every resident solve from its work items' minima of V/SR, which
+// Batched 2-D solves: the dt of every resident solve from its work items' minima of V/SR, which
 // fused stage 1 stored by table entry (a solve's entries are contiguous: `ranges` holds the
 // descriptor slot, first entry and count of each member).  One wavefront per member, launched
 // right after stage 1; skipped for a solve whose run has ended.  Per-item atomics on the solve's
@@ -821,7 +875,8 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
             return;
         }
     } else {
-        if (!ctl->go) return;
+        // stage 2 that applies the step's dt itself is the one that sets go
+        if (!(MODE == MODE_F2 && a.dt_minima) && !ctl->go) return;
         if constexpr (MODE == MODE_RN) {
             if (ctl->active) return;  // not the last step of this call
         }
@@ -838,13 +893,25 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
     }
     double block_min = __builtin_inf();
     double rn[N] = {};
-    stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, VIS>(a, tile < a.ntiles ? tile : -1, lane, block_min, rn);
+    if constexpr (MODE == MODE_F2) {
+        double dt = 0.0;
+        if (a.dt_minima) {
+            if (!step_dt(ctl, a.g.cfl, a.dt_part, a.dt_minima, lane, tile == 0, dt)) return;
+        } else {
+            dt = ctl->dt;
+        }
+        stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, VIS, true>(a, tile, lane, block_min, rn, dt);
+    } else {
+        stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, VIS>(a, tile < a.ntiles ? tile : -1, lane, block_min, rn);
+    }
+    if constexpr (MODE == MODE_S3) {
+        if (a.dt_minima && tile == 0 && lane == 0) step_advances(ctl, ctl->dt);
+    }
     if constexpr (MT::sr) {
-        // store the wavefront's minimum; dt_finalize_kernel turns the tiles' minima into dt after
-        // this launch
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) block_min = __builtin_fmin(block_min, __shfl_xor(block_min, o));
-        if (lane == 0) st_plane(a.dt_part, 0, 0, unsigned(tile), block_min);
+        // store the wavefront's minimum; stage 2 or dt_finalize_kernel turns the tiles' minima into dt
+        // after this launch
+        block_min = wave_min_lane63(block_min);
+        if (lane == 63) st_plane(a.dt_part, 0, 0, unsigned(tile), block_min);
     }
     if constexpr (MODE == MODE_RN) {
         __shared__ double rred[4 * NV];
@@ -875,24 +942,6 @@ constexpr int euler1d_threads = FLUX == FX_GODUNOV ? 512 : 1024;  // Godunov: ov
 constexpr int EULER1D_LDS = 20000;                               // doubles of the state and face arrays
 template <int RECON, int N>
 constexpr int euler1d_cells = EULER1D_LDS / (2 * N + 3 + (RECON == RC_PWC ? 0 : N)) - 1;
-
-// minimum over the wavefront, in lane 63 (row shifts, then row broadcasts)
-__device__ inline double wave_min_lane63(double v) {
-#define TS_MIN_STEP(ctrl)                                                              \
-    {                                                                                  \
-        const int lo = __double2loint(v), hi = __double2hiint(v);                      \
-        v = __builtin_fmin(v, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, ctrl, 0xF, 0xF, false), \
-                                               __builtin_amdgcn_update_dpp(lo, lo, ctrl, 0xF, 0xF, false))); \
-    }
-    TS_MIN_STEP(0x111) TS_MIN_STEP(0x112) TS_MIN_STEP(0x114) TS_MIN_STEP(0x118)  // row_shr 1, 2, 4, 8
-    TS_MIN_STEP(0x142) TS_MIN_STEP(0x143)                                        // row_bcast 15, 31
-#undef TS_MIN_STEP
-    return v;
-}
-// the same lane's value in every lane
-__device__ inline double read_lane63(double v) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63), __builtin_amdgcn_readlane(__double2loint(v), 63));
-}
 
 // a0: input buffer 0 -> output buffer 1 of the ping-pong; the final state goes to buffer 0 after an
 // even number of steps and to buffer 1 after an odd one.  n <= euler1d_cells<RECON, N>.
@@ -1117,23 +1166,32 @@ __global__ void __launch_bounds__(256) fvm_stage_batched(const KArgs* __restrict
                 continue;
             }
         } else {
-            if (!ctl->go) continue;
+            if (!(DIM == 1 && MODE == MODE_F2) && !ctl->go) continue;
         }
         double m = __builtin_inf();
+        // 1-D solves have few entries: their stage 2 applies dt itself (see step_dt).  A solve's entries
+        // are contiguous, so its first one is this entry's index less its place in the solve.
+        double dt = 0.0;
+        if constexpr (DIM == 1 && MODE == MODE_F2) {
+            if (!step_dt(ctl, a.g.cfl, part + (t - e.y), (a.ntiles + a.ty - 1) / a.ty, lane, e.y == 0, dt)) continue;
+        }
         if constexpr (DIM == 1) {
             // a 1-D work item is a group of a.ty consecutive strips, walked by one wavefront
             const int s0 = e.y * a.ty;
             const int s1 = (s0 + a.ty < a.ntiles) ? s0 + a.ty : a.ntiles;
             for (int sidx = s0; sidx < s1; sidx++) {
                 double ms = __builtin_inf();
-                stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, true>(a, sidx, lane, ms);
+                stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, MODE == MODE_F2, true>(a, sidx, lane, ms, nullptr, dt);
                 m = __builtin_fmin(m, ms);
             }
         } else {
             stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, true>(a, e.y, lane, m);
         }
+        if constexpr (DIM == 1 && MODE == MODE_S3) {
+            if (e.y == 0 && lane == 0) step_advances(ctl, ctl->dt);
+        }
         if constexpr (MT::sr) {
-            // the entry's minimum; dt_finalize_batched reduces each solve's entries after the launch
+            // the entry's minimum; stage 2 or dt_finalize_batched reduces each solve's entries
 #pragma unroll
             for (int o = 32; o >= 1; o >>= 1) m = __builtin_fmin(m, __shfl_xor(m, o));
             if (lane == 0) part[t] = m;

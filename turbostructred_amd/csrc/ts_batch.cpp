@@ -613,8 +613,8 @@ namespace {
 void issue_step(ts_batch* b, Family& f) {
     int nblk = b->ncu * f.occupancy;
     f.ks.bf1(f.d_desc, f.d_table, f.d_ntiles, f.d_part, nblk, b->stream);
-    // each member's dt from its entries' minima: one wavefront per member, 8 per CU
-    hipLaunchKernelGGL(tsd::dt_finalize_batched<0>, dim3(2 * b->ncu), dim3(256), 0, b->stream, f.d_desc, f.d_ranges,
+    // each member's dt from its entries' minima: one wavefront per member, 8 per CU (1-D: by stage 2)
+    if (std::get<0>(f.key) > 1) hipLaunchKernelGGL(tsd::dt_finalize_batched<0>, dim3(2 * b->ncu), dim3(256), 0, b->stream, f.d_desc, f.d_ranges,
                        f.d_nmem, f.d_part);
     f.ks.bf2(f.d_desc + f.cap_desc, f.d_table, f.d_ntiles, f.d_part, nblk, b->stream);
     f.ks.bs3(f.d_desc + 2 * f.cap_desc, f.d_table, f.d_ntiles, f.d_part, nblk, b->stream);

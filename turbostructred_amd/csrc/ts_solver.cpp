@@ -402,6 +402,11 @@ void step_launches(const ts_ctx* c, int start_buf, int s, Launch (&L)[MAX_LAUNCH
         a.uout = c->dU[out];
         L[n++] = {c->ks.s1e, a, 1};
     } else if (c->fused_dt) {
+        // stages 2 and 3 apply dt themselves where stage 1 leaves few enough minima (10 loads a lane;
+        // with the 1539 of a 512^2 grid stage 2 lost more than the launch took: 51 against 54 us a step)
+        // and nothing else needs it in between
+        constexpr int most_minima = 640;
+        a.dt_minima = (c->nd < 3 && !c->norms && c->ntiles <= most_minima) ? c->ntiles : 0;
         a.uin = c->dU[0];
         a.uout = c->dU[1];
         L[n++] = {c->ks.f1, a, 1};  // L(U^n) and dt
