@@ -626,6 +626,12 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             UL[v] = dpp_from_left(face[1][v]);
             UR[v] = face[0][v];
         }
+        // the end lanes lack a neighbour (the fluxes of lanes 0, 1 and 63 are not used): nothing in them
+        // may keep the exact solver from finding the strip constant
+        if (FLUX == FX_GODUNOV && (lane < 2 || lane == 63)) {
+#pragma unroll
+            for (int v = 0; v < N; v++) UL[v] = UR[v];
+        }
         if (!g.periodic[0]) {
             if (xg == 0) bc_image(g.bc[bc_marker(g, 0, 0)], gamma, 0, UR, UL);
             if (xg == nx) bc_image(g.bc[bc_marker(g, 1, 0)], gamma, 0, UL, UR);

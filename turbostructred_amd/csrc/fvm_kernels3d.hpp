@@ -447,7 +447,11 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
             face_of(1, UL);
             face_of(0, UR);
 #pragma unroll
-            for (int v = 0; v < NV; v++) UL[v] = dpp_from_left(UL[v]);
+            for (int v = 0; v < NV; v++) {
+                UL[v] = dpp_from_left(UL[v]);
+                // lane 0 has no left neighbour and its flux is not used: as in the 1-D stage
+                if (FLUX == FX_GODUNOV && lane == 0) UL[v] = UR[v];
+            }
             if (!g.periodic[0]) {
                 if (xg == 0) bc_image(g.bc[bc_marker(g, 0, ks * ny + rcs)], gamma, 0, UR, UL);
                 if (xg == nx) bc_image(g.bc[bc_marker(g, 1, ks * ny + rcs)], gamma, 0, UL, UR);
