@@ -21,9 +21,9 @@ struct KernelSet {
     BatchLaunchFn bf1 = nullptr, bf2 = nullptr, bs3 = nullptr;  // fused-dt SSP-RK3, batched
     OccupancyFn bocc = nullptr;
     OccupancyFn socc = nullptr;  // resident workgroups per CU of the single-solve kernels
-    // FP64 instances with viscous terms and body forces: the pre-pass (velocity
-    // gradients and viscous face fluxes of the stage input), the dt pass, the three stages and
-    // the residual norms
+    // FP64 instances with viscous terms and body forces: the pre-pass (velocity gradients and viscous
+    // face fluxes of the stage input; none in 2-D, whose stages form them), the dt pass, the three
+    // stages and the residual norms
     LaunchFn vpre = nullptr, vdt = nullptr, vs1 = nullptr, vs2 = nullptr, vs3 = nullptr, vrn = nullptr;
     // small 1-D forward-Euler solves: a chunk of steps in one workgroup (KArgs.uin = U^n,
     // uout = the other state buffer); FP64, 1-D units only
@@ -31,8 +31,8 @@ struct KernelSet {
     ChunkFn euler1d_chunk = nullptr;
 };
 
-// in_grid: the instances for states without momentum out of the grid's axes (1-D and 2-D; no viscous
-// and no unfused SSP kernels).
+// in_grid: the instances for states without momentum out of the grid's axes (1-D and 2-D; no
+// unfused SSP kernels, and viscous ones in 2-D only).
 // reconstruction variants: 0 PWC, 1 linear, 2 ENO2, 3 limited linear BJ, 4 limited linear Venkat
 bool get_kernels_d1_f0(int rv, int precision, bool in_grid, KernelSet* ks);
 bool get_kernels_d1_f1(int rv, int precision, bool in_grid, KernelSet* ks);

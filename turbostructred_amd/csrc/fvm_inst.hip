@@ -87,25 +87,25 @@ static int batched_occupancy() {
 }
 #endif
 
+#if TS_DIM != 2
 // viscous pre-pass: gradients of the interior cells, then the faces of every axis
 static void launch_vis_prepass(const KArgs& a, dim3, dim3, hipStream_t s) {
     const unsigned nb = unsigned((a.plane + 255) / 256);
     hipLaunchKernelGGL(vis_gradients<TS_DIM>, dim3(nb), dim3(256), 0, s, a);
     hipLaunchKernelGGL((vis_face_flux<TS_DIM, 0>), dim3((a.v.nface[0] + 255) / 256), dim3(256), 0, s, a);
-#if TS_DIM > 1
-    hipLaunchKernelGGL((vis_face_flux<TS_DIM, 1>), dim3((a.v.nface[1] + 255) / 256), dim3(256), 0, s, a);
-#endif
 #if TS_DIM > 2
+    hipLaunchKernelGGL((vis_face_flux<TS_DIM, 1>), dim3((a.v.nface[1] + 255) / 256), dim3(256), 0, s, a);
     hipLaunchKernelGGL((vis_face_flux<TS_DIM, 2>), dim3((a.v.nface[2] + 255) / 256), dim3(256), 0, s, a);
 #endif
 }
-template <int RC, int LM, int MODE>
+#endif
+template <int RC, int LM, int N, int MODE>
 static void launch_vis(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
 #if TS_DIM == 3
     hipLaunchKernelGGL((fvm_stage3d<RC, LM, TS_FLUX, MODE, double, double, double, 1>), (grid3d<double, 1, MODE>(a)),
                        dim3(64 * (z_waves<double, 1, MODE>)), 0, s, a);
 #else
-    hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, double, double, double, NV, 1>), g, b, 0, s, a);
+    hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, double, double, double, N, 1>), g, b, 0, s, a);
 #endif
     if constexpr (ModeTraits<MODE>::sr) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, a.ntiles);
 }
@@ -128,7 +128,7 @@ static void launch_euler1d_chunk(const KArgs& a, int steps, hipStream_t s) {
 #endif
 
 // the instances that carry N variables; the ones with every variable also cover the unfused SSP
-// sequence and the viscous terms
+// sequence, and they and the 2-D ones the viscous terms
 template <int RC, int LM, int N>
 static void fill(int precision, KernelSet* ks) {
     if (precision == 0) {
@@ -148,12 +148,16 @@ static void fill(int precision, KernelSet* ks) {
         if constexpr (N == NV) {
             ks->s1r = ks->s1e;
             ks->s2 = launch<RC, LM, N, MODE_S2, double, double, double>;
+        }
+        if constexpr (N == NV || TS_DIM == 2) {
+#if TS_DIM != 2
             ks->vpre = launch_vis_prepass;
-            ks->vdt = launch_vis<RC, LM, MODE_DT>;
-            ks->vs1 = launch_vis<RC, LM, MODE_S1>;
-            ks->vs2 = launch_vis<RC, LM, MODE_S2>;
-            ks->vs3 = launch_vis<RC, LM, MODE_S3>;
-            ks->vrn = launch_vis<RC, LM, MODE_RN>;
+#endif
+            ks->vdt = launch_vis<RC, LM, N, MODE_DT>;
+            ks->vs1 = launch_vis<RC, LM, N, MODE_S1>;
+            ks->vs2 = launch_vis<RC, LM, N, MODE_S2>;
+            ks->vs3 = launch_vis<RC, LM, N, MODE_S3>;
+            ks->vrn = launch_vis<RC, LM, N, MODE_RN>;
         }
 #if TS_DIM == 1
         ks->euler1d_chunk = launch_euler1d_chunk<RC, LM, N>;

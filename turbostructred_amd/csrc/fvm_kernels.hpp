@@ -86,8 +86,8 @@ struct GridArgs {
 // of the stage kernels and by the viscous pre-pass.
 struct VisArgs {
     const double* x[3];  // cell-centre coordinates, ghost layer included (n + 2 entries)
-    double* grad;        // velocity gradients of the interior cells: plane d*nd + e = d vel_d / d x_e
-    double* fv[3];       // viscous fluxes of the faces normal to axis a: 4 planes (momentum x, y, z,
+    double* grad;        // (1-D, 3-D pre-pass) velocity gradients of the interior cells: plane d*nd + e = d vel_d / d x_e
+    double* fv[3];       // (1-D, 3-D pre-pass) viscous fluxes of the faces normal to axis a: 4 planes (momentum x, y, z,
                          // energy), faces numbered like cells with n_a + 1 along a
     unsigned nface[3];   // faces normal to axis a (the plane size of fv[a])
     double mu;           // gas viscosity (viscous fluxes and the spectral-radius term)
@@ -423,47 +423,90 @@ template <int MODE> struct ModeTraits {
 // max(4/(3 rho_f), gamma/rho_f) mu fS^2 / V: the viscous part of a cell's spectral radius from
 // one face, rho_f = sqrt(rho_L rho_R) of the face states (ERK:1239-1248)
 __device__ inline double viscous_sr(double rho_l, double rho_r, double gamma, double mu, double fS, double vol) {
-#pragma clang fp contract(off)
-    const double ro = __builtin_sqrt(rho_l * rho_r);
-    const double a = 4.0 / (3.0 * ro), b = gamma / ro;
-    double v = (a < b) ? b : a;
-    v *= mu / 1.0;
-    v *= fS * fS;
-    v /= vol;
-    return v;
+    const double k = (4.0 / 3.0 < gamma) ? gamma : 4.0 / 3.0;
+    return fdiv(k * mu * (fS * fS), fsqrt(rho_l * rho_r) * vol);
 }
 
 // residual += force and acceleration sources of a cell (kernel.h:941-989)
-template <typename R>
-__device__ inline void add_sources(const VisArgs& v, const R (&u)[NV], double vol, R (&res)[NV]) {
+template <typename R, int N>
+__device__ inline void add_sources(const VisArgs& v, const R (&u)[N], double vol, R (&res)[N]) {
     const double ro = double(u[0]);
-    const double vx = double(u[1]) / ro, vy = double(u[2]) / ro, vz = double(u[3]) / ro;
+    double vel[N - 2];
+#pragma unroll
+    for (int i = 0; i < N - 2; i++) vel[i] = double(u[1 + i]) / ro;
     if (v.force) {
-        const double* s = v.sigma;
-        res[1] = R(double(res[1]) + vol * s[0]);
-        res[2] = R(double(res[2]) + vol * s[1]);
-        res[3] = R(double(res[3]) + vol * s[2]);
-        res[4] = R(double(res[4]) + (s[0] * vx + s[1] * vy + s[2] * vz) * vol);
+        double w = 0.0;
+#pragma unroll
+        for (int i = 0; i < N - 2; i++) {
+            res[1 + i] = R(double(res[1 + i]) + vol * v.sigma[i]);
+            w += v.sigma[i] * vel[i];
+        }
+        res[N - 1] = R(double(res[N - 1]) + w * vol);
     }
     if (v.accel_on) {
-        const double* g = v.accel;
-        res[1] = R(double(res[1]) + ro * vol * g[0]);
-        res[2] = R(double(res[2]) + ro * vol * g[1]);
-        res[3] = R(double(res[3]) + ro * vol * g[2]);
-        res[4] = R(double(res[4]) + (ro * g[0] * vx + ro * g[1] * vy + ro * g[2] * vz) * vol);
+        double w = 0.0;
+#pragma unroll
+        for (int i = 0; i < N - 2; i++) {
+            res[1 + i] = R(double(res[1 + i]) + ro * vol * v.accel[i]);
+            w += ro * v.accel[i] * vel[i];
+        }
+        res[N - 1] = R(double(res[N - 1]) + w * vol);
     }
 }
 
-// VIS instances (FP64) add the viscous face fluxes of the pre-pass (subtracted from the convective
-// flux before it is differenced, ERK:1221-1222), the viscous spectral-radius term after each
-// plus face's eigenvalue, and the body-force sources after the flux sweeps.
+// ---- viscous face fluxes of the 2-D stage ------------------------------------------------------
+// Flux of x momentum, y momentum, (z momentum) and energy through a face normal to axis D
+// (ComputeViscousFluxes, ERK:668-874): normal derivatives from the two cell velocities vl, vr,
+// tangential ones tan[] (of the first two components) already weighted, l = h_L / dx and r = h_R / dx.
+template <int D, int NM>
+__device__ __forceinline__ void vis_flux2(double mu, double idx, double l, double r, const double (&vl)[NM], const double (&vr)[NM],
+                                          const double (&tan)[2], double (&t)[NM + 1]) {
+    constexpr int T = 1 - D;
+    double dn[NM];
+#pragma unroll
+    for (int d = 0; d < NM; d++) dn[d] = (vr[d] - vl[d]) * idx;
+    t[D] = mu * ((-2.0 / 3.0) * (dn[D] + tan[T]) + 2.0 * dn[D]);
+    t[T] = mu * (dn[T] + tan[D]);
+    if constexpr (NM == 3) t[2] = mu * dn[2];
+    double e = 0.0;
+#pragma unroll
+    for (int d = 0; d < NM; d++) e += 0.5 * (l * vr[d] + r * vl[d]) * t[d];
+    t[NM] = e;
+}
+
+// Tangential derivative of the dummy cell across a boundary face (ComputeDummyCellGradients, ERK:303-665,
+// GradientComputer.h:19-53): 2 g_face - g_in, with g_face the least-squares gradient at the face centre
+// over the boundary cell, its two transverse neighbours and the dummy cell, anchored at the
+// face value; solved from the 2 x 2 normal equations.  rn, rd: distances along the normal from
+// the boundary cell and from the dummy cell to the face centre; rp, rm: along the face from the
+// transverse neighbours.
+struct FaceLsq {
+    double rn, rd, rp, rm;
+    __device__ __forceinline__ double operator()(double face, double in, double plus, double minus, double dummy, double g_in) const {
+        const double mnn = 3.0 * rn * rn + rd * rd, mnt = rn * (rp + rm), mtt = rp * rp + rm * rm;
+        const double dp = face - plus, dm = face - minus;
+        const double bn = rn * ((face - in) + dp + dm) + rd * (face - dummy), bt = rp * dp + rm * dm;
+        return 2.0 * fdiv(mnn * bt - mnt * bn, mnn * mtt - mnt * mnt) - g_in;
+    }
+};
+
+// VIS instances (FP64) subtract the viscous face fluxes from the convective ones before these are
+// differenced (ERK:1221-1222), add the viscous spectral-radius term after each plus face's eigenvalue,
+// and the body-force sources after the flux sweeps.  1-D takes the viscous fluxes from the pre-pass.
+// 2-D forms them here, from the velocities of the window that the march holds anyway: a lane keeps those
+// of its column in three rows and takes its x neighbours' by lane shifts, a dummy cell's gradient is
+// formed by the lane of its face.  (A pre-pass of three launches wrote 6 gradients per cell and 8
+// values per cell for the faces, and the stages read the latter back: 72 us of a 164 us forward-Euler
+// step at 1024^2.  The stage costs as much as it did with those reads, 54 us, so the step is at 87 us, of
+// which leaving out the momentum out of the plane is 7; it is bound by VALU issue.)
 // DT_ARG instances take the step's dt from `dt_arg` instead of the control block in memory.
 template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int N = NV,
           int VIS = 0, bool DT_ARG = false, bool GP = false>
 __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, double& block_min,
                                            double* rn = nullptr, double dt_arg = 0.0) {
     using MT = ModeTraits<MODE>;
-    static_assert(!VIS || N == NV, "viscous instances carry every variable");
+    constexpr bool VIN = VIS != 0 && DIM == 2 && MT::flux;  // viscous fluxes formed here
+    constexpr int NM = N - 2;                               // velocity components
     const GridArgs& g = a.g;
     const StepCtl* ctl = a.ctl;
     const bool tile_ok = tile >= 0 && tile < a.ntiles;
@@ -695,6 +738,24 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
         // x-neighbours are read from the same LDS rows at lane -+ 1 (the end lanes, halo lanes
         // whose results are discarded, read themselves): LDS reads instead of VALU lane shifts
         const int lm = lane > 0 ? lane - 1 : 0, lp = lane < 63 ? lane + 1 : 63;
+        // velocities of this lane's column in rows rc-1, rc, rc+1; x derivatives of the first two of them
+        // in rows rc-1 and rc, y derivatives in row rc; of the face on the minus x side: 1/dx and the
+        // weights h_L/dx, h_R/dx
+        const bool vin = VIN && a.v.viscous;
+        double vm[NM], v0[NM], vp[NM], gxm[2], gx[2], gy[2], vdx = 0.0, vhl = 0.0, vhr = 0.0;
+        if constexpr (VIN) {
+            if (vin) {
+                const int f = xg < 0 ? 0 : (xg > nx ? nx : xg);
+                vdx = fdiv(1.0, a.v.x[0][f + 1] - a.v.x[0][f]);
+                vhl = g.h[0][f] * vdx;
+                vhr = g.h[0][f + 1] * vdx;
+            }
+        }
+        auto velocity = [&](const R (&u)[N], double (&vel)[NM]) {
+            const double ir = frcp(double(u[0]));
+#pragma unroll
+            for (int d = 0; d < NM; d++) vel[d] = double(u[1 + d]) * ir;
+        };
         double srp = 0.0;       // spectral radius of the pending row without its top face
         R lam_gb = R(0);
         {
@@ -705,6 +766,12 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             for (int v = 0; v < N; v++) {
                 ring[wl][sm][v][lane] = t0[v];
                 ring[wl][s0][v][lane] = t1[v];
+            }
+            if constexpr (VIN) {
+                if (vin) {
+                    velocity(t0, vm);
+                    velocity(t1, v0);
+                }
             }
         }
         issue_row(y0, Pn);
@@ -718,6 +785,9 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                 complete_row(Pn, un1);
 #pragma unroll
                 for (int v = 0; v < N; v++) ring[wl][sp][v][lane] = un1[v];
+                if constexpr (VIN) {
+                    if (vin) velocity(un1, vp);
+                }
             }
             if (t + 1 < nit) issue_row(rc + 2, Pn);
             if constexpr (MT::use_un) {
@@ -739,6 +809,15 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             geo.rl[1] = R(ld_geo_uniform<GP>(g.rl[1], rcs));
             geo.rr[1] = R(ld_geo_uniform<GP>(g.rr[1], rcs));
             if (ev_cells) geo.eps2 = R(ev_x * ld_geo_uniform<GP>(g.ev[1], rcs));
+            if constexpr (VIN) {
+                if (vin) {
+#pragma unroll
+                    for (int d = 0; d < 2; d++) {
+                        gx[d] = (dpp_from_right(v0[d]) - dpp_from_left(v0[d])) * double(geo.rc[0]);
+                        gy[d] = (vp[d] - vm[d]) * double(geo.rc[1]);
+                    }
+                }
+            }
             R nb[4][N], face[4][N];
             {
                 R U0[N];
@@ -765,11 +844,35 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                 R G[N], lam;
                 if constexpr (MT::flux) face_flux<FLUX, 1, R>(gamma, eps, GL, GR, G, lam);
                 else lam = face_eigen<FLUX, 1, R>(gamma, GL, GR);
-                if constexpr (VIS && MT::flux) {
-                    if (a.v.viscous) {
-                        const unsigned fi = unsigned(rc) * unsigned(nx) + unsigned(xs);
+                if constexpr (VIN) {
+                    if (vin) {
+                        const double yl = a.v.x[1][rc], yr = a.v.x[1][rc + 1], hl = g.h[1][rc], hr = g.h[1][rc + 1];
+                        const double idy = fdiv(1.0, yr - yl), l = hl * idy, r = hr * idy;
+                        double gl[2] = {gxm[0], gxm[1]}, gr[2] = {gx[0], gx[1]};
+                        if (!g.periodic[1] && (rc == 0 || rc == ny)) {
+                            // the dummy cell is below (rc = 0) or above the face, the boundary cell on the
+                            // other side
+                            const bool below = rc == 0;
+                            const int si = below ? s0 : sm, sd = below ? sm : s0;
+                            const double yf = below ? yr - 0.5 * hr : yl + 0.5 * hl;
+                            const double xc = a.v.x[0][xs + 1];
+                            const FaceLsq lsq{yf - (below ? yr : yl), yf - (below ? yl : yr), xc - a.v.x[0][xs + 2], xc - a.v.x[0][xs]};
+                            const double ir = frcp(0.5 * double(ring[wl][si][0][lane] + ring[wl][sd][0][lane]));
 #pragma unroll
-                        for (int v = 1; v < N; v++) G[v] -= R(ld_plane(a.v.fv[1], a.v.nface[1], v - 1, fi));
+                            for (int d = 0; d < 2; d++) {
+                                const double in = below ? v0[d] : vm[d], dummy = below ? vm[d] : v0[d];
+                                const double face = 0.5 * double(ring[wl][si][1 + d][lane] + ring[wl][sd][1 + d][lane]) * ir;
+                                const double g_in = below ? gx[d] : gxm[d];
+                                const double gd = lsq(face, in, dpp_from_right(in), dpp_from_left(in), dummy, g_in);
+                                if (below) gl[d] = gd;
+                                else gr[d] = gd;
+                            }
+                        }
+                        const double tan[2] = {0.5 * (r * gl[0] + l * gr[0]), 0.5 * (r * gl[1] + l * gr[1])};
+                        double tv[NM + 1];
+                        vis_flux2<1, NM>(a.v.mu, idy, l, r, vm, v0, tan, tv);
+#pragma unroll
+                        for (int v = 1; v < N; v++) G[v] -= R(tv[v - 1]);
                     }
                 }
                 if constexpr (MT::sr) {
@@ -825,11 +928,48 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
                     R F[N], lamx;
                     if constexpr (MT::flux) face_flux<FLUX, 0, R>(gamma, eps, UL, UR, F, lamx);
                     else lamx = face_eigen<FLUX, 0, R>(gamma, UL, UR);
-                    if constexpr (VIS && MT::flux) {
-                        if (a.v.viscous) {
-                            const unsigned fi = unsigned(rcs) * unsigned(nx + 1) + unsigned(xg < 0 ? 0 : (xg > nx ? nx : xg));
+                    if constexpr (VIN) {
+                        if (vin) {
+                            double gl[2], gr[2], vl[NM];
 #pragma unroll
-                            for (int v = 1; v < N; v++) F[v] -= R(ld_plane(a.v.fv[0], a.v.nface[0], v - 1, fi));
+                            for (int d = 0; d < NM; d++) vl[d] = dpp_from_left(v0[d]);
+#pragma unroll
+                            for (int d = 0; d < 2; d++) {
+                                gl[d] = dpp_from_left(gy[d]);
+                                gr[d] = gy[d];
+                            }
+                            double pl[2], ml[2];  // lane shifts outside the lanes' branch: they read every lane
+                            if (!g.periodic[0] && (strip == 0 || strip == a.nstrips - 1)) {
+#pragma unroll
+                                for (int d = 0; d < 2; d++) {
+                                    pl[d] = dpp_from_left(vp[d]);
+                                    ml[d] = dpp_from_left(vm[d]);
+                                }
+                                if (xg == 0 || xg == nx) {
+                                    // the dummy cell is on the left (xg = 0, the boundary cell this lane's) or
+                                    // this lane's own (xg = nx, the boundary cell the left neighbour's)
+                                    const bool west = xg == 0;
+                                    const int f = west ? 0 : nx;
+                                    const double xl = a.v.x[0][f], xr = a.v.x[0][f + 1], hb = g.h[0][west ? 1 : nx];
+                                    const double xf = west ? xr - 0.5 * hb : xl + 0.5 * hb;
+                                    const double yc = a.v.x[1][rc + 1];
+                                    const FaceLsq lsq{xf - (west ? xr : xl), xf - (west ? xl : xr), yc - a.v.x[1][rc + 2], yc - a.v.x[1][rc]};
+                                    const double ir = frcp(0.5 * double(ring[wl][s0][0][lm] + ring[wl][s0][0][lane]));
+#pragma unroll
+                                    for (int d = 0; d < 2; d++) {
+                                        const double face = 0.5 * double(ring[wl][s0][1 + d][lm] + ring[wl][s0][1 + d][lane]) * ir;
+                                        const double gd = west ? lsq(face, v0[d], vp[d], vm[d], vl[d], gr[d])
+                                                               : lsq(face, vl[d], pl[d], ml[d], v0[d], gl[d]);
+                                        if (west) gl[d] = gd;
+                                        else gr[d] = gd;
+                                    }
+                                }
+                            }
+                            const double tan[2] = {0.5 * (vhr * gl[0] + vhl * gr[0]), 0.5 * (vhr * gl[1] + vhl * gr[1])};
+                            double tv[NM + 1];
+                            vis_flux2<0, NM>(a.v.mu, vdx, vhl, vhr, vl, v0, tan, tv);
+#pragma unroll
+                            for (int v = 1; v < N; v++) F[v] -= R(tv[v - 1]);
                         }
                     }
                     if constexpr (MT::flux) {
@@ -860,6 +1000,15 @@ __device__ __forceinline__ void stage_tile(const KArgs& a, int tile, int lane, d
             }
 #pragma unroll
             for (int v = 0; v < N; v++) ytop[v] = face[3][v];
+            if constexpr (VIN) {
+#pragma unroll
+                for (int d = 0; d < NM; d++) {
+                    vm[d] = v0[d];
+                    v0[d] = vp[d];
+                }
+#pragma unroll
+                for (int d = 0; d < 2; d++) gxm[d] = gx[d];
+            }
             const int st = sm;
             sm = s0;
             s0 = sp;

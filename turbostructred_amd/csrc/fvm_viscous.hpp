@@ -1,5 +1,5 @@
-// fvm_viscous.hpp -- viscous pre-pass of one stage: velocity gradients of the
-// interior cells, then the viscous flux of every face, written for the stage kernel to subtract
+// fvm_viscous.hpp -- viscous pre-pass of one stage in 1-D and 3-D (the 2-D stages form these fluxes
+// themselves, from the window they hold): velocity gradients of the interior cells, then the viscous flux of every face, written for the stage kernel to subtract
 // from its convective fluxes.
 //
 //   vis_gradients   ComputeGradientNonUniformStructured (kernel.h:918-938): central differences

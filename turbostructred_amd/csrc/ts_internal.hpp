@@ -64,7 +64,8 @@ struct ts_ctx {
 
     // kernel timing
     bool timing = false;
-    // per kind: dt, stages 1-3, (unused), residual norms, viscous pre-pass
+    // per kind: dt, stages 1-3, (unused), residual norms, launches that form viscous fluxes (the
+    // pre-pass; in 2-D the stages, counted under both kinds)
     double t_ms[7] = {0, 0, 0, 0, 0, 0, 0};
     long long t_n[7] = {0, 0, 0, 0, 0, 0, 0};
     // viscous terms / body forces / viscous spectral radius: the VIS kernel instances run

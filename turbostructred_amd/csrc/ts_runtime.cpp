@@ -408,10 +408,11 @@ int ts_algorithmic_bytes_per_cell(const ts_ctx* c, int kind, double* bytes) {
         b[2] = s + d + s;    // read U^1, U^n, write U^2
         b[3] = s + d + d;    // read U^2, U^n, write U^{n+1}
     }
-    // viscous fluxes: each stage also reads 4 face values per axis; the pre-pass writes 3 nd
-    // gradients per cell (reading the state), then reads state and gradients and writes the faces
+    // viscous fluxes of a pre-pass (2-D stages form them from the state they hold): each stage also
+    // reads 4 face values per axis; the pre-pass writes 3 nd gradients per cell (reading the state),
+    // then reads state and gradients and writes the faces
     double pre = 0.0;
-    if (c->vis && c->cfg.viscous) {
+    if (c->vis && c->cfg.viscous && c->ks.vpre) {
         const double nd = c->nd;
         for (int k = 1; k <= 3; k++)
             if (b[k] > 0) b[k] += 32.0 * nd;

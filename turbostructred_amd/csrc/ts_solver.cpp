@@ -172,7 +172,7 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
     }
     c->vis = k.viscous || k.external_force || k.external_accel || k.viscosity != 0.0;
     if (c->vis) {
-        if (!c->ks.vdt || !c->ks.vpre) {
+        if (!c->ks.vdt) {
             c->err = "no viscous kernel instance for this combination";
             return TS_ERR_UNSUPPORTED;
         }
@@ -187,9 +187,10 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
         }
         if (k.viscous) {
             int r;
-            if ((r = dalloc(c, &v.grad, c->ncell * 3 * c->nd))) return r;
-            for (int a = 0; a < c->nd; a++) {
+            for (int a = 0; a < c->nd; a++)
                 if ((r = upload(c, c->X[a].data(), c->X[a].size(), &v.x[a]))) return r;
+            if (c->ks.vpre && (r = dalloc(c, &v.grad, c->ncell * 3 * c->nd))) return r;
+            for (int a = 0; c->ks.vpre && a < c->nd; a++) {
                 v.nface[a] = (unsigned)(c->ncell / c->n[a] * (c->n[a] + 1));
                 if ((r = dalloc(c, &v.fv[a], (size_t)v.nface[a] * 4))) return r;
             }
@@ -227,7 +228,8 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
     c->nstrips = (c->n[0] + STRIP - 1) / STRIP;
     c->block_dim = dim3(256);
     c->variant[0].ks = c->ks;
-    c->may_reduce = !c->arena && !c->vis && (k.rk_stages == 1 || c->fused_dt) && tsr::boundaries_in_grid(k) &&
+    const bool sources_in_grid = !(k.external_force && k.sigma[2] != 0.0) && !(k.external_accel && k.accel[2] != 0.0);
+    c->may_reduce = !c->arena && (c->vis ? c->nd == 2 && sources_in_grid : k.rk_stages == 1 || c->fused_dt) && tsr::boundaries_in_grid(k) &&
                     tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, true, &c->variant[1].ks);
     size_t most_tiles = 0;
     for (int i = 0; i < (c->may_reduce ? 2 : 1); i++) {
@@ -329,6 +331,7 @@ struct Launch {
     LaunchFn fn;
     KArgs args;
     int kind;
+    bool forms_viscous = false;  // a stage that forms the viscous fluxes itself: also timed as kind 6
 };
 
 constexpr int MAX_LAUNCHES = 8;  // per step: 3 viscous pre-passes, dt, norms, 3 stages
@@ -360,13 +363,14 @@ void step_launches(const ts_ctx* c, int start_buf, int s, Launch (&L)[MAX_LAUNCH
     // viscous pre-pass over the stage input: while steps remain (before the dt pass), or when the
     // step runs (later stages)
     auto prepass = [&](const void* in, int gate_go) {
-        if (!c->cfg.viscous) return;
+        if (!c->cfg.viscous || !c->ks.vpre) return;
         KArgs p = a;
         p.uin = in;
         p.v.gate_go = gate_go;
         L[n++] = {c->ks.vpre, p, 6};
     };
     if (c->vis) {
+        const bool forms = c->cfg.viscous && !c->ks.vpre;
         if (c->cfg.rk_stages == 1) {
             int in = (start_buf + s) & 1, out = in ^ 1;
             a.uin = c->dU[in];
@@ -374,22 +378,22 @@ void step_launches(const ts_ctx* c, int start_buf, int s, Launch (&L)[MAX_LAUNCH
             L[n++] = {c->ks.vdt, a, 0};
             norms(c->dU[in]);
             a.uout = c->dU[out];
-            L[n++] = {c->ks.vs1, a, 1};
+            L[n++] = {c->ks.vs1, a, 1, forms};
         } else {
             a.uin = c->dU[0];
             prepass(a.uin, 0);
             L[n++] = {c->ks.vdt, a, 0};
             norms(c->dU[0]);
             a.uout = c->dU[1];
-            L[n++] = {c->ks.vs1, a, 1};
+            L[n++] = {c->ks.vs1, a, 1, forms};
             a.uin = c->dU[1];
             prepass(a.uin, 1);
             a.uout = c->dU[2];
-            L[n++] = {c->ks.vs2, a, 2};
+            L[n++] = {c->ks.vs2, a, 2, forms};
             a.uin = c->dU[2];
             prepass(a.uin, 1);
             a.uout = c->dU[0];
-            L[n++] = {c->ks.vs3, a, 3};
+            L[n++] = {c->ks.vs3, a, 3, forms};
         }
         return;
     }
@@ -438,7 +442,12 @@ void step_launches(const ts_ctx* c, int start_buf, int s, Launch (&L)[MAX_LAUNCH
 }
 
 int issue_direct(ts_ctx* c, int start_buf, int first, int count) {
-    std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> rec;
+    struct Timed {
+        int kind;
+        bool forms_viscous;
+        hipEvent_t e0, e1;
+    };
+    std::vector<Timed> rec;
     size_t need = c->timing ? (size_t)count * 2 * MAX_LAUNCHES : 0;
     while (c->events.size() < need) {
         hipEvent_t e;
@@ -456,7 +465,7 @@ int issue_direct(ts_ctx* c, int start_buf, int first, int count) {
                 CHK(hipEventRecord(e0, c->stream));
                 L[i].fn(L[i].args, c->grid_dim, c->block_dim, c->stream);
                 CHK(hipEventRecord(e1, c->stream));
-                rec.push_back({L[i].kind, {e0, e1}});
+                rec.push_back({L[i].kind, L[i].forms_viscous, e0, e1});
             } else {
                 L[i].fn(L[i].args, c->grid_dim, c->block_dim, c->stream);
             }
@@ -467,9 +476,13 @@ int issue_direct(ts_ctx* c, int start_buf, int first, int count) {
         CHK(hipStreamSynchronize(c->stream));
         for (auto& r : rec) {
             float ms = 0;
-            CHK(hipEventElapsedTime(&ms, r.second.first, r.second.second));
-            c->t_ms[r.first] += ms;
-            c->t_n[r.first] += 1;
+            CHK(hipEventElapsedTime(&ms, r.e0, r.e1));
+            c->t_ms[r.kind] += ms;
+            c->t_n[r.kind] += 1;
+            if (r.forms_viscous) {
+                c->t_ms[6] += ms;
+                c->t_n[6] += 1;
+            }
         }
     }
     return TS_OK;
