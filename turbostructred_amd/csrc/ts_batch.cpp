@@ -113,7 +113,7 @@ struct Problem {
     ts_config cfg{};
     int max_steps = 0;
     double t_end = 0;
-    std::vector<double> init;  // reference AoS state until admission
+    tsr::HostArray init;  // reference AoS state until admission
     std::vector<double> coord[3], h[3];  // owned copies of optional non-uniform grid arrays
     size_t bytes = 0, off = 0;
     KArgs desc{};
@@ -121,7 +121,8 @@ struct Problem {
     int ntiles = 0;
     size_t ncell = 0;
     int n[3] = {1, 1, 1};
-    std::vector<double> result;
+    tsr::HostArray result;
+    size_t region = 0;  // its place in the outgoing staging buffer
     ts_step_info info{};
     int status = 0;  // 0 queued, 1 resident (or being admitted), 2 done
     int error = 0;
@@ -129,10 +130,6 @@ struct Problem {
     int slot = -1;       // index of its descriptors in its family's descriptor blocks
     StepCtl final_ctl{};  // its control block when it finished (published with its state)
     bool uploaded = false;  // its descriptors are in place for the family's current tiling
-    // admission: the host sources of its asynchronous uploads, kept until the copy stream is
-    // synchronised
-    std::vector<double> geo_host;
-    StepCtl init_ctl{};
 };
 
 // Tile-shape autotuning of a family (ts_batch_config.autotune_tiles): for each load bucket
@@ -228,6 +225,7 @@ struct ts_batch {
     // Finished solves leave through a second stream: their states are converted and copied out
     // while the next pass's kernels run, and published (done, memory released) at that pass.
     hipStream_t cstream = nullptr;
+    tsr::Staging staging;        // pinned, for the copy stream's transfers (the pass thread's)
     double* d_rstage = nullptr;  // staging of the outgoing AoS states, one region per solve
     size_t rstage_cap = 0;
     std::vector<Problem*> retiring;
@@ -327,8 +325,7 @@ int ensure_stage(ts_batch* b, size_t doubles) {
 
 // upload geometry/state/control of a problem into its arena block and fill its descriptor.  The
 // copies and the layout conversion go on the copy stream, so that they overlap the kernels of
-// a pass in flight; the caller synchronises that stream before the problem runs and before the
-// host sources (init, geo_host, init_ctl) are released.
+// a pass in flight; the caller synchronises that stream before the problem runs.
 int admit(ts_batch* b, Problem& p) {
     const ts_config& c = p.cfg;
     Layout L = layout_of(c);
@@ -341,8 +338,7 @@ int admit(ts_batch* b, Problem& p) {
     g.gamma = c.gamma;
     g.eps = c.eps;
     g.cfl = c.cfl;
-    std::vector<double>& geo = p.geo_host;
-    geo.clear();
+    std::vector<double> geo;
     geo.reserve(L.geo_doubles);
     double* dgeo = (double*)(base + L.geo);
     bool uniform = true;
@@ -390,21 +386,42 @@ int admit(ts_batch* b, Problem& p) {
         g.bc[m].rho = c.bc[m].density;
     }
     for (int s = 0; s < 6; s++) g.side_marker[s] = c.side_marker[s];
-    BCHK(hipMemcpyAsync(dgeo, geo.data(), geo.size() * 8, hipMemcpyHostToDevice, b->cstream));
     // state: the AoS array with ghosts crosses as it is and is converted on the device (the
     // staging buffer is reused by the next admission in the stream's order)
     size_t n = p.ncell;
     int r = ensure_stage(b, p.init.size());
     if (r) return r;
-    BCHK(hipMemcpyAsync(b->d_stage, p.init.data(), p.init.size() * 8, hipMemcpyHostToDevice, b->cstream));
+    const size_t state_bytes = p.init.size() * sizeof(double);
+    hipError_t e;
+    if (state_bytes < tsr::kSmallState) {
+        // (from pinned memory a copy is issued in 4 us; from the caller's pageable kind each holds the host)
+        char* src = b->staging.take(state_bytes, b->cstream, &e);
+        BCHK(e);
+        std::memcpy(src, p.init.data(), state_bytes);
+        BCHK(hipMemcpyAsync(b->d_stage, src, state_bytes, hipMemcpyHostToDevice, b->cstream));
+    } else {
+        BCHK(b->staging.to_device(b->d_stage, p.init.data(), state_bytes, b->bc.device, b->cstream));
+    }
     BCHK(tsr::device_aos_to_soa(b->d_stage, (double*)(base + L.u0), c.ndims, p.n, b->cstream));
-    StepCtl& ctl = p.init_ctl;
-    ctl = StepCtl{};
+    StepCtl ctl{};
     ctl.t_max = p.t_end > 0 ? p.t_end : 1e300;
     ctl.next_snap = p.t_end > 0 ? p.t_end : 0.0;
     ctl.max_steps = p.max_steps;
     ctl.active = p.max_steps > 0 ? 1 : 0;
-    BCHK(hipMemcpyAsync(base + L.ctl, &ctl, sizeof(StepCtl), hipMemcpyHostToDevice, b->cstream));
+    // the geometry and the control block lie one after the other: one copy
+    const size_t block = L.ctl + sizeof(StepCtl) - L.geo;
+    if (block <= tsr::Staging::kBytes) {
+        char* src = b->staging.take(block, b->cstream, &e);
+        BCHK(e);
+        std::memset(src, 0, block);
+        std::memcpy(src, geo.data(), geo.size() * sizeof(double));
+        std::memcpy(src + (L.ctl - L.geo), &ctl, sizeof(StepCtl));
+        BCHK(hipMemcpyAsync(dgeo, src, block, hipMemcpyHostToDevice, b->cstream));
+    } else {
+        BCHK(hipMemcpyAsync(dgeo, geo.data(), geo.size() * sizeof(double), hipMemcpyHostToDevice, b->cstream));
+        BCHK(hipMemcpyAsync(base + L.ctl, &ctl, sizeof(StepCtl), hipMemcpyHostToDevice, b->cstream));
+        BCHK(hipStreamSynchronize(b->cstream));  // the sources are local
+    }
     KArgs& d = p.desc;
     d.uin = nullptr;
     d.lin = nullptr;
@@ -680,16 +697,51 @@ int credit_trial(ts_batch* b, Family& f) {
 }
 
 // Issue, on the copy stream, the conversion of a finished problem's state to the reference AoS
-// layout (ghosts zero) in its region of the outgoing staging buffer and the copy to the host.
-// Needs no lock: the problem is out of its family but not yet published, so poll does not read it.
+// layout (ghosts zero) in its region of the outgoing staging buffer.  The copy to the host waits until
+// the next pass's kernels are issued (complete_retiring).  Needs no lock: the problem is out of its
+// family but not yet published, so poll does not read it.
 int issue_retire(ts_batch* b, Problem& p, size_t region) {
     Layout L = layout_of(p.cfg);
     const size_t na = tsr::aos_doubles(p.cfg.ndims, p.n);
     double* st = b->d_rstage + region;
-    p.result.resize(na);
+    p.region = region;
     BCHK(hipMemsetAsync(st, 0, na * sizeof(double), b->cstream));
     BCHK(tsr::device_soa_to_aos((const double*)(b->d_arena + p.off + L.u0), st, p.cfg.ndims, p.n, b->cstream));
-    BCHK(hipMemcpyAsync(p.result.data(), st, na * sizeof(double), hipMemcpyDeviceToHost, b->cstream));
+    return TS_OK;
+}
+
+// The outgoing states of b->retiring, from their regions to their results.  Large ones one by one; runs of
+// small ones, whose regions follow one another, in one copy to pinned memory.  No lock, as above.
+int fetch_results(ts_batch* b) {
+    auto bytes_of = [](const Problem& p) { return tsr::aos_doubles(p.cfg.ndims, p.n) * sizeof(double); };
+    std::vector<Problem*>& R = b->retiring;
+    for (Problem* p : R)
+        if (!p->result.allocate(bytes_of(*p) / sizeof(double))) return fail(b, TS_ERR_NOMEM, "no host memory for a result");
+    for (size_t i = 0; i < R.size();) {
+        size_t bytes = bytes_of(*R[i]), j = i + 1;
+        if (bytes >= tsr::kSmallState) {
+            BCHK(b->staging.to_host(R[i]->result.data(), b->d_rstage + R[i]->region, bytes, b->bc.device, b->cstream));
+            i = j;
+            continue;
+        }
+        for (; j < R.size(); j++) {
+            const size_t more = bytes_of(*R[j]);
+            if (more >= tsr::kSmallState || bytes + more > tsr::Staging::kBytes ||
+                R[j]->region != R[i]->region + bytes / sizeof(double))
+                break;
+            bytes += more;
+        }
+        hipError_t e;
+        const char* from = b->staging.take(bytes, b->cstream, &e);
+        BCHK(e);
+        BCHK(hipMemcpyAsync((void*)from, b->d_rstage + R[i]->region, bytes, hipMemcpyDeviceToHost, b->cstream));
+        BCHK(hipStreamSynchronize(b->cstream));
+        b->staging.all_free();
+        for (; i < j; i++) {
+            std::memcpy(R[i]->result.data(), from, bytes_of(*R[i]));
+            from += bytes_of(*R[i]);
+        }
+    }
     return TS_OK;
 }
 
@@ -761,6 +813,7 @@ int ts_batch_destroy(ts_batch* b) {
     if (b->d_arena) (void)hipFree(b->d_arena);
     if (b->d_stage) (void)hipFree(b->d_stage);
     if (b->d_rstage) (void)hipFree(b->d_rstage);
+    b->staging.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
     if (b->cstream) (void)hipStreamDestroy(b->cstream);
     delete b;
@@ -824,21 +877,27 @@ int ts_batch_submit(ts_batch* b, const ts_config* cfg, const double* init_state,
     if (p->bytes > b->arena.capacity) return fail(b, TS_ERR_NOMEM, "solve is larger than the HBM budget");
     size_t nst = ts_state_size_cfg(cfg);
     // copied in blocks that stay in the cache while they are searched for momentum out of the grid's
-    // axes (any bit but the sign's: NaN counts)
-    p->init.reserve(nst);
-    const double* const out_of_grid = init_state + (cfg->ndims == 1 ? 2 : 3);
-    uint64_t bits = 0;
-    for (size_t i = 0; i < nst; i += 5 * 1024) {
-        const size_t end = std::min(nst, i + 5 * 1024);
-        p->init.insert(p->init.end(), init_state + i, init_state + end);
-        for (size_t j = i; j < end; j += 5) {
-            uint64_t u[2];
-            std::memcpy(u, out_of_grid + j, (cfg->ndims == 1 ? 2 : 1) * sizeof(uint64_t));
-            bits |= u[0] << 1;
-            if (cfg->ndims == 1) bits |= u[1] << 1;
+    // axes (any bit but the sign's: NaN counts); the blocks of a large state by several threads
+    if (!p->init.allocate(nst)) return fail(b, TS_ERR_NOMEM, "no host memory for the initial state");
+    const bool one_axis = cfg->ndims == 1;
+    const double* const out_of_grid = init_state + (one_axis ? 2 : 3);
+    std::atomic<uint64_t> any{0};
+    const size_t bytes = nst * sizeof(double);
+    tsr::for_chunks(nst, 5 * 16384, bytes < tsr::kThreadedCopy ? 1 : tsr::copy_threads(), [&](int, size_t b0, size_t e0) {
+        uint64_t bits = 0;
+        for (size_t i = b0; i < e0; i += 5 * 1024) {
+            const size_t end = std::min(e0, i + 5 * 1024);
+            std::memcpy(p->init.data() + i, init_state + i, (end - i) * sizeof(double));
+            for (size_t j = i; j < end; j += 5) {
+                uint64_t u[2];
+                std::memcpy(u, out_of_grid + j, (one_axis ? 2 : 1) * sizeof(uint64_t));
+                bits |= u[0] << 1;
+                if (one_axis) bits |= u[1] << 1;
+            }
         }
-    }
-    const bool in_grid = bits == 0 && tsr::boundaries_in_grid(*cfg);
+        any |= bits;
+    });
+    const bool in_grid = any == 0 && tsr::boundaries_in_grid(*cfg);
     std::lock_guard<std::mutex> lk(b->mu);
     int fam = family_of(b, *cfg, in_grid);
     if (fam < 0) return fail(b, TS_ERR_UNSUPPORTED, "no batched kernel for this configuration");
@@ -851,13 +910,15 @@ int ts_batch_submit(ts_batch* b, const ts_config* cfg, const double* init_state,
     return TS_OK;
 }
 
-// wait for the outgoing copies in flight and publish those solves (done, memory released)
+// copy the outgoing states to the host and publish those solves (done, memory released)
 static int complete_retiring(ts_batch* b) {
     if (b->retiring.empty()) return TS_OK;
-    BCHK(hipStreamSynchronize(b->cstream));
+    {
+        int r = fetch_results(b);
+        if (r) return r;
+    }
     std::lock_guard<std::mutex> lk(b->mu);
     for (Problem* p : b->retiring) {
-        std::vector<double>().swap(p->init);
         finish_retire(b, *p, p->final_ctl);
     }
     b->retiring.clear();
@@ -889,10 +950,8 @@ static int admit_queued(ts_batch* b) {
     std::vector<int> admitted(incoming.size(), 0);
     for (size_t i = 0; i < incoming.size(); i++) admitted[i] = admit(b, *incoming[i]) == TS_OK;
     BCHK(hipStreamSynchronize(b->cstream));
-    for (Problem* p : incoming) {
-        std::vector<double>().swap(p->init);
-        std::vector<double>().swap(p->geo_host);
-    }
+    b->staging.all_free();
+    for (Problem* p : incoming) p->init.release();
     // (3) under the lock again: attach them to their families (or fail them)
     std::lock_guard<std::mutex> lk(b->mu);
     for (size_t i = 0; i < incoming.size(); i++) {
@@ -1073,20 +1132,23 @@ int ts_batch_run(ts_batch* b, int n_steps, int* pending) {
 
 int ts_batch_poll(ts_batch* b, long long ticket, int* done, double* out_state, ts_step_info* info) {
     if (!b || !done) return TS_ERR_INVALID;
-    std::lock_guard<std::mutex> lk(b->mu);
-    auto it = b->probs.find(ticket);
-    if (it == b->probs.end()) return fail(b, TS_ERR_INVALID, "unknown ticket");
-    Problem& p = *it->second;
-    if (p.status != 2) {
-        *done = 0;
-        return TS_OK;
+    std::unique_ptr<Problem> p;
+    {
+        std::lock_guard<std::mutex> lk(b->mu);
+        auto it = b->probs.find(ticket);
+        if (it == b->probs.end()) return fail(b, TS_ERR_INVALID, "unknown ticket");
+        if (it->second->status != 2) {
+            *done = 0;
+            return TS_OK;
+        }
+        p = std::move(it->second);
+        b->probs.erase(it);
     }
+    // the copy without the lock: a pass does not wait for it
     *done = 1;
-    if (out_state) std::memcpy(out_state, p.result.data(), p.result.size() * sizeof(double));
-    if (info) *info = p.info;
-    int err = p.error;
-    b->probs.erase(it);
-    return err ? TS_ERR_UNPHYSICAL : TS_OK;
+    if (out_state && p->result.size()) tsr::host_copy(out_state, p->result.data(), p->result.size() * sizeof(double));
+    if (info) *info = p->info;
+    return p->error ? TS_ERR_UNPHYSICAL : TS_OK;
 }
 
 int ts_batch_start_server(ts_batch* b) {

@@ -8,6 +8,7 @@
 
 #include "../../include/ts_fvm.h"
 #include "fvm_dispatch.hpp"
+#include "ts_hostmem.hpp"
 
 struct ts_ctx {
     ts_config cfg;
@@ -85,6 +86,7 @@ struct ts_ctx {
     int graph_steps[2] = {0, 0};
     bool use_graphs = true;
 
+    tsr::Staging staging;     // of uploads and downloads
     double* d_aos = nullptr;  // device copy of the reference AoS state (uploads / downloads)
     size_t device_bytes = 0;
 

@@ -279,7 +279,7 @@ int ts_set_state(ts_ctx* c, const double* aos, size_t n) {
     int r = ensure_aos(c);
     if (r) return r;
     // the conversion also notes whether any momentum points out of the grid's axes
-    HIPCHK(c, hipMemcpyAsync(c->d_aos, aos, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, c->staging.to_device(c->d_aos, aos, n * sizeof(double), c->cfg.device, c->stream));
     HIPCHK(c, hipMemsetAsync(&c->dctl->out_of_grid, 0, sizeof(int), c->stream));
     HIPCHK(c, tsr::device_aos_to_soa(c->d_aos, (double*)c->dU[0], c->nd, c->n, c->stream, &c->dctl->out_of_grid));
     HIPCHK(c, hipMemcpyAsync(&c->hctl->out_of_grid, &c->dctl->out_of_grid, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -298,8 +298,7 @@ int ts_get_state(ts_ctx* c, double* aos, size_t n) {
     // ghost layers' images
     HIPCHK(c, hipMemsetAsync(c->d_aos, 0, n * sizeof(double), c->stream));
     HIPCHK(c, tsr::device_soa_to_aos((const double*)c->dU[c->cur], c->d_aos, c->nd, c->n, c->stream));
-    HIPCHK(c, hipMemcpyAsync(aos, c->d_aos, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, c->staging.to_host(aos, c->d_aos, n * sizeof(double), c->cfg.device, c->stream));
     fill_ghost_images(c, aos);
     return TS_OK;
 }

@@ -287,6 +287,7 @@ void destroy_device_ctx(ts_ctx* c) {
     if (c->d_cells) (void)hipFree(c->d_cells);
     if (c->d_cell_vals) (void)hipFree(c->d_cell_vals);
     if (c->d_aos) (void)hipFree(c->d_aos);
+    c->staging.release();
     if (c->hctl && c->hctl != &c->hctl_local) (void)hipHostFree(c->hctl);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
     if (c->stream && !c->arena) (void)hipStreamDestroy(c->stream);
