@@ -40,7 +40,7 @@ static void launch(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
     hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, R, TIn, TOut, N>), g, b, 0, s, a);
 #endif
     if constexpr (ModeTraits<MODE>::sr) {
-        if (!a.dt_minima) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, a.ntiles);
+        if (!a.dt_minima) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, int(g.x));
     }
 }
 
@@ -107,7 +107,7 @@ static void launch_vis(const KArgs& a, dim3 g, dim3 b, hipStream_t s) {
 #else
     hipLaunchKernelGGL((fvm_stage<TS_DIM, RC, LM, TS_FLUX, MODE, double, double, double, N, 1>), g, b, 0, s, a);
 #endif
-    if constexpr (ModeTraits<MODE>::sr) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, a.ntiles);
+    if constexpr (ModeTraits<MODE>::sr) hipLaunchKernelGGL(dt_finalize_kernel<0>, dim3(1), dim3(1024), 0, s, a.ctl, a.g.cfl, a.dt_part, int(g.x));
 }
 
 #if TS_DIM == 1

@@ -12,7 +12,7 @@
 //
 // Modes
 //   MODE_DT  spectral radius of every cell from the face eigenvalues, min(V/SR) over the grid
-//            (wave shuffle, one stored minimum per tile); a one-workgroup kernel launched
+//            (one stored minimum per workgroup); a one-workgroup kernel launched
 //            after it turns the minima into dt (ERK:1427-1437).  Used before forward Euler.
 //   MODE_S1  U1 = U + dt L(U)          forward Euler (kernel.h:319-331) / SSP stage 1
 //   MODE_S2  U2 = 3/4 Un + 1/4 (U1 + dt L(U1))
@@ -113,7 +113,7 @@ struct KArgs {
     int nstrips;       // strips along x
     int ntiles;        // strips * row blocks
     double* rn_part;   // per-block partial residual norms, 5 per block (MODE_RN)
-    double* dt_part;   // single solves: each tile's minimum of V/SR (dt passes, fused stage 1)
+    double* dt_part;   // single solves: each workgroup's minimum of V/SR (dt passes, fused stage 1)
     int dt_minima;     // fused stages 2 and 3: number of those minima where they apply the step's dt
                        // themselves (see step_dt); 0 where dt_finalize_kernel has done it
 };
@@ -313,8 +313,19 @@ __device__ inline double read_lane63(double v) {
 // what stage 3 reads, dt and go.  Time, the step count and the stop rule, which the other wavefronts
 // of stage 2 still read, are advanced by stage 3.  False where the step does not run.
 __device__ inline bool step_dt(StepCtl* ctl, double cfl, const double* part, int n, int lane, bool first, double& dt) {
-    double m = __builtin_inf();
-    for (int i = lane; i < n; i += 64) m = __builtin_fmin(m, part[i]);
+    // up to 640 minima in one round trip to memory, and 576 more in each further one: all loads of a trip
+    // are in flight together (one load at a time, 385 minima took most of what the launch does)
+    double m = part[lane < n ? lane : n - 1];
+    for (int i = 64; i < n; i += 576) {
+        double q[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            const int j = i + 64 * k + lane;
+            q[k] = part[j < n ? j : n - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < 9; k++) m = __builtin_fmin(m, q[k]);
+    }
     if (!ctl->active) return false;  // stage 1 has cleared go
     m = read_lane63(wave_min_lane63(m));
     const bool ok = dt_rule(ctl, cfl, m, dt);
@@ -329,7 +340,7 @@ __device__ inline bool step_dt(StepCtl* ctl, double cfl, const double* part, int
     return ok;
 }
 
-// Single solves: the step's dt from the `n` per-tile minima of V/SR that a dt pass or fused
+// Single solves: the step's dt from the `n` per-workgroup minima of V/SR that a dt pass or fused
 // stage 1 stored, launched right after it.  Plain stores and one workgroup's reduction instead of
 // one same-address atomic per wavefront: those serialise where the wavefronts finish together,
 // at the end of the launch (a 1-D stage 1 with 70k strips spent most of its time in them).  The
@@ -1043,8 +1054,8 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwaves = blockDim.x >> 6;
     const int tile = xcd_remap(blockIdx.x, gridDim.x) * nwaves + wave;
-    if constexpr (MODE != MODE_RN) {
-        if (tile >= a.ntiles) return;  // only the norms reduce across the block
+    if constexpr (MODE != MODE_RN && !MT::sr) {
+        if (tile >= a.ntiles) return;  // the norms and the minima are reduced across the block
     }
     double block_min = __builtin_inf();
     double rn[N] = {};
@@ -1056,17 +1067,24 @@ __global__ void __launch_bounds__(256) fvm_stage(KArgs a) {
             dt = ctl->dt;
         }
         stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, VIS, true>(a, tile, lane, block_min, rn, dt);
-    } else {
+    } else if (MODE == MODE_RN || tile < a.ntiles) {
         stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, VIS>(a, tile < a.ntiles ? tile : -1, lane, block_min, rn);
     }
     if constexpr (MODE == MODE_S3) {
         if (a.dt_minima && tile == 0 && lane == 0) step_advances(ctl, ctl->dt);
     }
     if constexpr (MT::sr) {
-        // store the wavefront's minimum; stage 2 or dt_finalize_kernel turns the tiles' minima into dt
-        // after this launch
-        block_min = wave_min_lane63(block_min);
-        if (lane == 63) st_plane(a.dt_part, 0, 0, unsigned(tile), block_min);
+        // store the workgroup's minimum; stage 2 or dt_finalize_kernel turns these into dt after this
+        // launch.  (One for each wavefront was four times as many: with the 1539 of a 512^2 grid stage 2
+        // lost more by reducing them itself than the launch between them takes.)
+        __shared__ double wave_min[4];
+        block_min = wave_min_lane63(block_min);  // +inf without a tile
+        if (lane == 63) wave_min[wave] = block_min;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const double m = __builtin_fmin(__builtin_fmin(wave_min[0], wave_min[1]), __builtin_fmin(wave_min[2], wave_min[3]));
+            st_plane(a.dt_part, 0, 0, blockIdx.x, m);
+        }
     }
     if constexpr (MODE == MODE_RN) {
         __shared__ double rred[4 * NV];

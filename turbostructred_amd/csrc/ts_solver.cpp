@@ -231,14 +231,12 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
     const bool sources_in_grid = !(k.external_force && k.sigma[2] != 0.0) && !(k.external_accel && k.accel[2] != 0.0);
     c->may_reduce = !c->arena && (c->vis ? c->nd == 2 && sources_in_grid : k.rk_stages == 1 || c->fused_dt) && tsr::boundaries_in_grid(k) &&
                     tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, true, &c->variant[1].ks);
-    size_t most_tiles = 0;
     for (int i = 0; i < (c->may_reduce ? 2 : 1); i++) {
         tile_variant(c, *cfg, c->variant[i]);
-        most_tiles = std::max(most_tiles, (size_t)c->variant[i].ntiles);
         c->most_blocks = std::max(c->most_blocks, (size_t)c->variant[i].grid_dim.x);
     }
-    // one minimum of V/SR per tile from every dt pass and fused stage 1
-    if ((r = dalloc(c, &c->dt_part, most_tiles))) return r;
+    // one minimum of V/SR per workgroup from every dt pass and fused stage 1
+    if ((r = dalloc(c, &c->dt_part, c->most_blocks))) return r;
     if ((r = use_variant(c, false))) return r;
     c->euler1d_wg = k.rk_stages == 1 && c->nd == 1 && k.precision == TS_FP64 && !c->vis && c->ks.euler1d_chunk &&
                     c->ntiles <= 64 && !(sep && sep[0] == '1');
@@ -407,11 +405,13 @@ void step_launches(const ts_ctx* c, int start_buf, int s, Launch (&L)[MAX_LAUNCH
         a.uout = c->dU[out];
         L[n++] = {c->ks.s1e, a, 1};
     } else if (c->fused_dt) {
-        // stages 2 and 3 apply dt themselves where stage 1 leaves few enough minima (10 loads a lane;
-        // with the 1539 of a 512^2 grid stage 2 lost more than the launch took: 51 against 54 us a step)
-        // and nothing else needs it in between
-        constexpr int most_minima = 640;
-        a.dt_minima = (c->nd < 3 && !c->norms && c->ntiles <= most_minima) ? c->ntiles : 0;
+        // stages 2 and 3 apply dt themselves where stage 1 leaves few enough minima and nothing else needs
+        // it in between.  The line lies at two round trips of step_dt: with 770 minima (1024^2 in float)
+        // a step takes 79.6 us against 81.9 with the launch, with 385 (512^2) 48.1 against 50.8; a larger
+        // grid's steps are long enough not to notice the launch.
+        constexpr int most_minima = 1216;
+        const int minima = (int)c->grid_dim.x;
+        a.dt_minima = (c->nd < 3 && !c->norms && minima <= most_minima) ? minima : 0;
         a.uin = c->dU[0];
         a.uout = c->dU[1];
         L[n++] = {c->ks.f1, a, 1};  // L(U^n) and dt
