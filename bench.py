@@ -21,6 +21,7 @@ sys.path.insert(0, os.path.join(ROOT, "tests"))
 from turbostructred_amd import capi  # noqa: E402
 
 HBM_PEAK = 8.0e12  # MI355X HBM3E, bytes/s
+PLANES_2D = 4 / 5  # a plane flow's kernels leave out one of the five variables that the library counts
 
 
 def lax_liu_state(cfg):
@@ -67,7 +68,7 @@ def gpu_run(n, steps, warmup, precision=capi.FP64, autotune=True):
         if cnt == 0:
             continue
         avg = ms / cnt * 1e-3
-        b = s.algorithmic_bytes_per_cell(kind) * ncell
+        b = PLANES_2D * s.algorithmic_bytes_per_cell(kind) * ncell
         kern[name] = dict(avg_us=avg * 1e6, launches=cnt, algorithmic_bytes=b, achieved_gbs=b / avg / 1e9,
                           frac=b / avg / HBM_PEAK)
     s.enable_kernel_timing(False)
@@ -167,15 +168,14 @@ def viscous_channel(n=2048, steps=40):
         s.enable_kernel_timing(True)
         s.step(min(steps, 10))
         kern = {}
-        for kind, name in ((capi.KIND_VISCOUS, "viscous_prepass"), (capi.KIND_DT, "dt_pass"),
-                           (capi.KIND_STAGE1, "stage1"), (capi.KIND_STAGE2, "stage2"), (capi.KIND_STAGE3, "stage3")):
+        for kind, name in ((capi.KIND_DT, "dt_pass"), (capi.KIND_STAGE1, "stage1"), (capi.KIND_STAGE2, "stage2"), (capi.KIND_STAGE3, "stage3")):
             ms, cnt = s.kernel_timing(kind)
             if cnt == 0:
                 continue
             avg = ms / cnt * 1e-3
-            b = s.algorithmic_bytes_per_cell(kind) * n * n
+            b = PLANES_2D * s.algorithmic_bytes_per_cell(kind) * n * n
             kern[name] = dict(avg_us=avg * 1e6, launches=cnt, achieved_gbs=b / avg / 1e9, frac=b / avg / HBM_PEAK)
-        bps = s.algorithmic_bytes_per_cell(capi.KIND_ALL)
+        bps = PLANES_2D * s.algorithmic_bytes_per_cell(capi.KIND_ALL)
         rate = n * n * steps / el
         out["euler" if rk == 1 else "ssp_rk3"] = {
             "cell_updates_per_s": rate, "ms_per_step": el / steps * 1e3, "algorithmic_bytes_per_cell_step": bps,
