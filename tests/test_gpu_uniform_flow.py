@@ -41,3 +41,14 @@ def after_steps(n, riemann, recon, stages, periodic, rho, p, velocity=VELOCITY):
 def test_lines_and_planes(n, stages, riemann, recon, periodic, rho, p):
     got, ref = after_steps(n, riemann, recon, stages, periodic, rho, p)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("rho,p", FLOWS)
+@pytest.mark.parametrize("periodic", [0, 1])
+@pytest.mark.parametrize("recon", [capi.RECON_PWC, capi.RECON_LINEAR_LIM])
+@pytest.mark.parametrize("riemann", [capi.RIEMANN_ROE, capi.RIEMANN_HLLC])
+@pytest.mark.parametrize("stages", [1, 3])
+@pytest.mark.parametrize("n", [(5, 3, 4), (61, 7, 15), (33, 21, 29)])
+def test_boxes(n, stages, riemann, recon, periodic, rho, p):
+    got, ref = after_steps(n, riemann, recon, stages, periodic, rho, p)
+    assert np.array_equal(got, ref)

@@ -10,16 +10,17 @@
 // evaluated once, by the wavefront above it.
 //
 // What bounds it is VALU issue and the latency of the row's serial chain, so registers and LDS are
-// spent to have wavefronts: 25 values per lane and wavefront in LDS (window 15, the residual
-// carried to the next row 5, z-flux 5), the face states as the cell and its offsets.  In float 16
-// wavefronts share a CU, four per SIMD, and 14 of 16 planes produce output (stage 2: 12, three,
-// 10 of 12).  In double 200 registers allow two per SIMD, 8 and 6 of 8; 12 wavefronts at 168
-// registers spilled (stage 2 of 256^3 3.0 ms).  With the window in registers and copies of the centre
+// spent to have wavefronts: 20 values per lane and wavefront in LDS (window 15, z-flux 5) and, where
+// they do not fit into registers, 10 that are carried to the next row; the face states as the cell and
+// its offsets.  In float 16 wavefronts share a CU, four per SIMD, and 14 of 16 planes produce output
+// (stage 2: 12, three, 10 of 12).  In double 220 to 250 registers allow two per SIMD, 8 and 6 of 8; 12 wavefronts
+// at 168 registers spilled (stage 2 of 256^3 3.0 ms).  With the window in registers and copies of the centre
 // row, the carried fluxes and both z exchanges in LDS (42 values) the float kernels ran at two per
-// SIMD: 150x141x133 step 507 us, now 361; 256^3 double step 3.37 ms, now 3.04.
+// SIMD: 150x141x133 step 507 us, now 363; 256^3 double step 3.37 ms, now 2.96.
 //
-// The residual of a cell is accumulated y-, z-, x, y+, z+ and its spectral radius x-, x+, y-, y+, z-,
-// z+ (ERK:1225-1248, 1305-1328, 1385-1408).  VIS instances add the viscous face fluxes of the
+// The residual of a cell is the sum of the flux differences of x, y and z, and its spectral radius that of
+// x-, x+, y-, y+, z-, z+ (ERK:1225-1248, 1305-1328, 1385-1408).  (Adding the fluxes one by one rounds
+// at the size of a flux, not of the difference: a uniform float flow drifted.)  VIS instances add the viscous face fluxes of the
 // pre-pass, the viscous spectral-radius term after each plus face (the z-face part travels through
 // LDS with the z eigenvalue) and the body-force sources.
 #pragma once
@@ -39,7 +40,15 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
     constexpr int ZW = z_waves<R, VIS, MODE>, ZOUT = ZW - 2;
     StepCtl* ctl = a.ctl;
     __shared__ R ring[ZW][3][NV][64];                  // [wavefront][slot][variable][lane]
-    __shared__ R carry[MT::flux ? ZW : 1][NV][64];     // residual of the pending row so far
+    // What is carried to the next row, of the row that is pending then: the x part of its residual and the
+    // fluxes through its faces below, in y and z.  In double all 15 values fit into the registers with the
+    // HLLC flux (247 of 256 at most; 256^3 step 2.96 ms, 3.04 with the x part in LDS, 3.16 with
+    // none) and with Roe's, whose stage 2 spills little (128^3 611 us, 637 with the x part in LDS) but for
+    // ENO2 (650 against 631); the exact solver and the float kernels would spill.
+    constexpr bool X_REGS = sizeof(R) == 8 && (FLUX == FX_HLLC || (FLUX == FX_ROE && RECON != RC_ENO2));
+    constexpr bool YZ_REGS = sizeof(R) == 8 && FLUX != FX_GODUNOV;
+    __shared__ R carry_x[MT::flux && !X_REGS ? ZW : 1][NV][64];
+    __shared__ R carry_y[MT::flux && !YZ_REGS ? ZW : 1][NV][64];
     __shared__ R lds_h[MT::flux ? ZW : 1][NV][64];     // flux through the z-face below every plane
     __shared__ R lds_l[MT::sr ? ZW : 1][64];           // eigenvalue of that face
     __shared__ double lds_vz[VIS && MT::sr ? ZW : 1][64];  // its viscous spectral-radius term before / V
@@ -175,7 +184,19 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
     double rn[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
     const int y0 = yb * a.ty;
     const int yend = (y0 + a.ty < ny) ? y0 + a.ty : ny;
-    R (&cy)[NV][64] = carry[MT::flux ? w : 0];
+    R Db[X_REGS ? NV : 1], Gb[YZ_REGS ? NV : 1], Hb[YZ_REGS ? NV : 1];
+    auto dfx = [&](int v) -> R& {
+        if constexpr (X_REGS) return Db[v];
+        else return carry_x[MT::flux ? w : 0][v][lane];
+    };
+    auto gbot = [&](int v) -> R& {
+        if constexpr (YZ_REGS) return Gb[v];
+        else return carry_y[MT::flux ? w : 0][v][lane];
+    };
+    auto hbot = [&](int v) -> R {
+        if constexpr (YZ_REGS) return Hb[v];
+        else return lds_h[w][v][lane];
+    };
     int sm = 0, s0 = 1, sp = 2;  // slots of rows rc-1, rc, rc+1
     RawCell Pn;                  // prefetched stencil row, completed one iteration later
     // The centre row of the z-neighbour that no wavefront holds (edge wavefronts, prefetched), or U^n
@@ -289,7 +310,6 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
             }
         };
         // y-face between rows rc-1 and rc
-        R acc[NV];  // residual of row rc: y-, then z-, then the x faces
         R G[NV], lamy = R(0), GL0 = R(0), GR0 = R(0);
         const R Sy = R(hx * hz);  // face area of a y-face (ERK:1269)
         if (out_plane && t >= 1) {
@@ -349,7 +369,8 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
                     R resv[NV], Um[NV];
 #pragma unroll
                     for (int v = 0; v < NV; v++) {
-                        resv[v] = (cy[v][lane] - G[v] * Sy) - lds_h[w + 1][v][lane] * Szb;
+                        resv[v] = (dfx(v) - flux_difference(G[v], gbot(v)) * Sy) -
+                                  flux_difference(lds_h[w + 1][v][lane], hbot(v)) * Szb;
                         Um[v] = ring[w][sm][v][lane];
                     }
                     if constexpr (VIS) add_sources(a.v, Um, hx * hyp * hz, resv);
@@ -380,7 +401,7 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
                     }
                 }
 #pragma unroll
-                for (int v = 0; v < NV; v++) acc[v] = G[v] * Sy;
+                for (int v = 0; v < NV; v++) gbot(v) = G[v];
             }
         }
         // the z+ face state goes up through the slot of the finalized row
@@ -427,7 +448,7 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
 #pragma unroll
                 for (int v = 0; v < NV; v++) {
                     lds_h[w][v][lane] = H[v];
-                    acc[v] += H[v] * Sz;
+                    if constexpr (YZ_REGS) Hb[v] = H[v];
                 }
             }
             if constexpr (MT::sr) {
@@ -487,7 +508,7 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
             }
             if constexpr (MT::flux) {
 #pragma unroll
-                for (int v = 0; v < NV; v++) cy[v][lane] = acc[v] - (dpp_from_right(F[v]) - F[v]) * Sx;
+                for (int v = 0; v < NV; v++) dfx(v) = -(flux_difference(dpp_from_right(F[v]), F[v]) * Sx);
             }
         }
         if (!EARLY && edge && t + 1 < nit) issue_cell(rc + 1, k + zoff, Zq);  // (these have no x-faces)
