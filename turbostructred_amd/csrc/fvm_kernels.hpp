@@ -362,9 +362,9 @@ __global__ void __launch_bounds__(1024) dt_finalize_kernel(StepCtl* ctl, double 
     }
 }
 
-// Batched 2-D solves: the dt of every resident solve from its work items' minima of V/SR, which
-// fused stage 1 stored by table entry (a solve's entries are contiguous: `ranges` holds the
-// descriptor slot, first entry and count of each member).  One wavefront per member, launched
+// Batched solves whose stage 2 does not do it (2-D, and 1-D of many work items): the dt of each from its
+// work items' minima of V/SR, which fused stage 1 stored by table entry (a solve's entries are
+// contiguous: `ranges` holds the descriptor slot, first entry and count of each such member).  One wavefront per member, launched
 // right after stage 1; skipped for a solve whose run has ended.  Per-item atomics on the solve's
 // control block serialised on a lone large solve (2 x 3000 same-address atomics per stage 1 at
 // 2048^2), and their ordering needed either a fence, which writes back the L2, or waiting for a
@@ -1355,14 +1355,16 @@ __global__ void __launch_bounds__(256) fvm_stage_batched(const KArgs* __restrict
                 continue;
             }
         } else {
-            if (!(DIM == 1 && MODE == MODE_F2) && !ctl->go) continue;
+            // (stage 2 that applies the step's dt itself is the one that sets go)
+            if (!(DIM == 1 && MODE == MODE_F2 && a.dt_minima) && !ctl->go) continue;
         }
         double m = __builtin_inf();
-        // 1-D solves have few entries: their stage 2 applies dt itself (see step_dt).  A solve's entries
-        // are contiguous, so its first one is this entry's index less its place in the solve.
+        // A 1-D solve of few entries applies dt itself in stage 2 (see step_dt).  A solve's entries are
+        // contiguous, so its first one is this entry's index less its place in the solve.
         double dt = 0.0;
         if constexpr (DIM == 1 && MODE == MODE_F2) {
-            if (!step_dt(ctl, a.g.cfl, part + (t - e.y), (a.ntiles + a.ty - 1) / a.ty, lane, e.y == 0, dt)) continue;
+            if (!a.dt_minima) dt = ctl->dt;
+            else if (!step_dt(ctl, a.g.cfl, part + (t - e.y), a.dt_minima, lane, e.y == 0, dt)) continue;
         }
         if constexpr (DIM == 1) {
             // a 1-D work item is a group of a.ty consecutive strips, walked by one wavefront
@@ -1377,7 +1379,7 @@ __global__ void __launch_bounds__(256) fvm_stage_batched(const KArgs* __restrict
             stage_tile<DIM, RECON, LIM, FLUX, MODE, R, TIn, TOut, N, 0, false, true>(a, e.y, lane, m);
         }
         if constexpr (DIM == 1 && MODE == MODE_S3) {
-            if (e.y == 0 && lane == 0) step_advances(ctl, ctl->dt);
+            if (a.dt_minima && e.y == 0 && lane == 0) step_advances(ctl, ctl->dt);
         }
         if constexpr (MT::sr) {
             // the entry's minimum; stage 2 or dt_finalize_batched reduces each solve's entries

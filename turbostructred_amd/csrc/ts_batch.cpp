@@ -181,6 +181,7 @@ struct Family {
     int slot_end = 0;        // slots handed out so far: [0, slot_end)
     int param = -1;          // tiling parameter chosen by the last retile (rows, or strips per item)
     int uploaded_param = -1; // the one the uploaded descriptors carry
+    bool in_stage = false;  // stage 2 applies the dt (see dt_in_stage); the descriptors and the graph say so too
     KArgs* d_fresh = nullptr;  // staging for new descriptors and their destination indices
     int* d_fresh_idx = nullptr;
     size_t cap_fresh = 0;
@@ -532,8 +533,33 @@ void retile(ts_batch* b, Family& f) {
     }
 }
 
+// 1-D: whether stage 2 applies the dt itself, each work item from all minima of its solve, instead of
+// dt_finalize_batched in a launch between the stages.  It does where an item reads them with one load (solves of
+// at most 64 items), or where no wavefront has more than a few items to do it for (some 4 us each round)
+// and all items together read little from the L2 (0.3 us per million).  us per step in FP64, with the
+// launch and without: HLLC 1 tube of 1000 cells 11.8 and 10.2, 1 x 400000 (6667 items) 55.5 and 50.6, 8 x 72000 55.6
+// and 54.5, 512 x 9000 (76800 items) 241 and 263, 64 x 72000 246 and 284, 1 x 1600000 190 and 418, 4096 x 1000
+// 217 and 219; exact solver 1 x 146000 41.0 and 35.8, 1 x 400000 84.0 and 80.1, 1 x 1600000 276 and 497.
+constexpr int kOneLoad = 64;
+constexpr long long kMostRounds = 4, kMostReads = 48ll << 20;
+
+bool dt_in_stage(const ts_batch* b, const Family& f) {
+    if (std::get<0>(f.key) != 1) return false;
+    long long items = 0, reads = 0, most = 0;
+    for (const Problem* q : f.members) {
+        items += q->ntiles;
+        reads += (long long)q->ntiles * q->ntiles;
+        most = std::max(most, (long long)q->ntiles);
+    }
+    return most <= kOneLoad || (items <= kMostRounds * b->ncu * f.occupancy * 4 && reads <= kMostReads);
+}
+
 int rebuild_tables(ts_batch* b, Family& f) {
     retile(b, f);
+    const bool in_stage = dt_in_stage(b, f);
+    const bool moved = in_stage != f.in_stage;
+    f.in_stage = in_stage;
+    for (Problem* q : f.members) q->desc.dt_minima = in_stage ? q->ntiles : 0;
     size_t nt = 0;
     for (const Problem* q : f.members) nt += q->ntiles;
     bool realloc = false;
@@ -566,14 +592,14 @@ int rebuild_tables(ts_batch* b, Family& f) {
         BCHK(hipMalloc(&f.d_nmem, sizeof(int)));
         realloc = true;
     }
-    if (realloc && f.graph) {
+    if ((realloc || moved) && f.graph) {
         (void)hipGraphExecDestroy(f.graph);
         f.graph = nullptr;
     }
     // descriptors: kernel k's block starts at k * cap_desc, so that the launch arguments stay
     // fixed while the resident set changes; only problems whose descriptors are not in place for
     // the current tiling are uploaded, contiguously, and scattered to their slots on the device
-    const bool all = realloc || f.param != f.uploaded_param;
+    const bool all = realloc || moved || f.param != f.uploaded_param;
     std::vector<KArgs> fresh;
     std::vector<int> fresh_idx;
     for (Problem* q : f.members) {
@@ -630,9 +656,10 @@ namespace {
 void issue_step(ts_batch* b, Family& f) {
     int nblk = b->ncu * f.occupancy;
     f.ks.bf1(f.d_desc, f.d_table, f.d_ntiles, f.d_part, nblk, b->stream);
-    // each member's dt from its entries' minima: one wavefront per member, 8 per CU (1-D: by stage 2)
-    if (std::get<0>(f.key) > 1) hipLaunchKernelGGL(tsd::dt_finalize_batched<0>, dim3(2 * b->ncu), dim3(256), 0, b->stream, f.d_desc, f.d_ranges,
-                       f.d_nmem, f.d_part);
+    // each member's dt from its entries' minima: one wavefront per member, 8 per CU
+    if (!f.in_stage)
+        hipLaunchKernelGGL(tsd::dt_finalize_batched<0>, dim3(2 * b->ncu), dim3(256), 0, b->stream, f.d_desc,
+                           f.d_ranges, f.d_nmem, f.d_part);
     f.ks.bf2(f.d_desc + f.cap_desc, f.d_table, f.d_ntiles, f.d_part, nblk, b->stream);
     f.ks.bs3(f.d_desc + 2 * f.cap_desc, f.d_table, f.d_ntiles, f.d_part, nblk, b->stream);
 }
