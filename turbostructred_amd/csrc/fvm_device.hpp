@@ -643,9 +643,9 @@ struct StarDev {
 //     not far below both: Newton takes no more steps from it than from the two-rarefaction formula,
 //     whose three powers every lane of the wavefront would wait for.
 __device__ inline StarDev star_state_dev(double g, double rl, double ul, double pl, double rr,
-                                         double ur, double pr, double irl, double irr) {
+                                         double ur, double pr, double al, double irl, double irr) {
     StarDev s;
-    const double al = fsqrt(g * pl * irl), ar = fsqrt(g * pr * irr);
+    const double ar = fsqrt(g * pr * irr);  // (and al, the left side's)
     const double du = ur - ul;
     const double ig = frcp(g), igp = frcp(g + 1.0), c2 = 2.0 * frcp(g - 1.0);
     s.vacuum = c2 * (al + ar) <= du;
@@ -768,63 +768,67 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
     double pR = eos.GetPressure(UR[0], UR[N - 1] * ir - kR / 2.0);
     double uL = vL[D], uR = vR[D];
     // Ahead of the waves a tube is constant, half of it on average over a run, and its faces have the
-    // same state on both sides: a wavefront of nothing else takes the flux of that state and skips
-    // the star state and the sampling, about 900 instructions.  (All lanes or none: with a single
-    // other face among them the wavefront runs the whole solver anyway.)  Batch of 1024 tubes 346 -> 304 ms,
-    // a 1000-cell tube 38 -> 32 ms.  The equality is bitwise, so
-    // a constant region stays one: every face in it gives the same flux.
+    // same state on both sides: a wavefront of nothing else skips the star state and the sampling, about 900
+    // instructions.  (All lanes or none: with a single other face among them the wavefront runs the
+    // whole solver anyway.)  Batch of 1024 tubes 346 -> 304 ms, a 1000-cell tube 38 -> 32 ms.  Such a face
+    // has the flux and the speed of its state in either case, lane by lane: the two cells beside a face may
+    // ask two wavefronts for it.
+    const double S = 0.0;
     bool same = UL[0] > 0.0 && pL > 0.0;
 #pragma unroll
     for (int i = 0; i < N; i++) same = same && UL[i] == UR[i];
-    if (__all(same)) {
-        const double a = fsqrt(g * pL * il);
-        F[0] = R(UL[0] * uL);
-#pragma unroll
-        for (int i = 0; i < NM; i++) F[1 + i] = R(UL[0] * uL * vL[i] + (i == D ? pL : 0.0));
-        F[N - 1] = R(uL * (UL[N - 1] + pL));
-        lam = R(__builtin_fabs(uL) + a);
-        return;
-    }
-    const StarDev st = star_state_dev(g, UL[0], uL, pL, UR[0], uR, pR, il, ir);
+    const double aL = fsqrt(g * pL * il);
     double ro, u, p;
-    const double S = 0.0;
-    bool left = st.vacuum ? (S <= 0.5 * (st.STL + st.STR)) : (st.u >= S);
-    // The side of the contact the sample lies on, then one of four cases for that side K:
-    // 0 its initial state, 1 its star state, 2 inside its rarefaction fan, 3 vacuum.  The
-    // conditions are the reference's with the right side mirrored by sgn = -1 (exact), so one
-    // fan evaluation serves both sides.
-    const double sgn = left ? 1.0 : -1.0;
-    const bool shockK = left ? st.shock_l : st.shock_r;
-    const double SK = left ? st.SL : st.SR, SHK = left ? st.SHL : st.SHR, STK = left ? st.STL : st.STR;
-    const double rK = left ? UL[0] : UR[0], uK = left ? uL : uR, pK = left ? pL : pR;
-    int cs;
-    if (shockK && !st.vacuum) cs = (sgn * (SK - S) >= 0.0) ? 0 : 1;
-    else if (sgn * (SHK - S) > 0.0) cs = 0;
-    else if (sgn * (S - STK) > 0.0) cs = st.vacuum ? 3 : 1;
-    else cs = 2;
-    if (cs == 0) { ro = rK; u = uK; p = pK; }
-    else if (cs == 1) {
-        // star density behind a shock (Toro eq. 4.50) or a rarefaction (eq. 4.53)
-        const double prK = fdiv(st.p, pK);
-        if (shockK) {
-            const double C = (g - 1.0) * frcp(g + 1.0);
-            ro = fdiv(prK + C, C * prK + 1.0) * rK;
-        } else {
-            ro = rK * dpow(prK, frcp(g));
+    bool left = true;
+    if (__all(same)) {
+        ro = UL[0];
+        u = uL;
+        p = pL;
+        lam = R(__builtin_fabs(uL) + aL);
+    } else {
+        const StarDev st = star_state_dev(g, UL[0], uL, pL, UR[0], uR, pR, aL, il, ir);
+        lam = R(same ? __builtin_fabs(uL) + aL : st.smax);
+        left = st.vacuum ? (S <= 0.5 * (st.STL + st.STR)) : (st.u >= S);
+        // The side of the contact the sample lies on, then one of four cases for that side K:
+        // 0 its initial state, 1 its star state, 2 inside its rarefaction fan, 3 vacuum.  The
+        // conditions are the reference's with the right side mirrored by sgn = -1 (exact), so one
+        // fan evaluation serves both sides.
+        const double sgn = left ? 1.0 : -1.0;
+        const bool shockK = left ? st.shock_l : st.shock_r;
+        const double SK = left ? st.SL : st.SR, SHK = left ? st.SHL : st.SHR, STK = left ? st.STL : st.STR;
+        const double rK = left ? UL[0] : UR[0], uK = left ? uL : uR, pK = left ? pL : pR;
+        int cs;
+        if (shockK && !st.vacuum) cs = (sgn * (SK - S) >= 0.0) ? 0 : 1;
+        else if (sgn * (SHK - S) > 0.0) cs = 0;
+        else if (sgn * (S - STK) > 0.0) cs = st.vacuum ? 3 : 1;
+        else cs = 2;
+        if (cs == 0) { ro = rK; u = uK; p = pK; }
+        else if (cs == 1) {
+            // star density behind a shock (Toro eq. 4.50) or a rarefaction (eq. 4.53)
+            const double prK = fdiv(st.p, pK);
+            if (shockK) {
+                const double C = (g - 1.0) * frcp(g + 1.0);
+                ro = fdiv(prK + C, C * prK + 1.0) * rK;
+            } else {
+                ro = rK * dpow(prK, frcp(g));
+            }
+            u = st.u;
+            p = st.p;
         }
-        u = st.u;
-        p = st.p;
-    }
-    else if (cs == 3) { ro = 0; u = 0; p = 0; }
-    else {
-        // inside the fan (Toro eq. 4.56): C^(2/(g-1)) scales the density, and the pressure by
-        // C^(2g/(g-1)) = C^(2/(g-1)) C^2
-        const double aK = fsqrt(fdiv(g * pK, rK)), igp = frcp(g + 1);
-        const double C = igp * (2.0 + sgn * (g - 1) * fdiv(uK - S, aK));
-        const double w = dpow(C, 2.0 * frcp(g - 1));
-        ro = w * rK;
-        u = (sgn * aK + 0.5 * (g - 1) * uK + S) * (2 * igp);
-        p = w * C * C * pK;
+        else if (cs == 3) { ro = 0; u = 0; p = 0; }
+        else {
+            // inside the fan (Toro eq. 4.56): C^(2/(g-1)) scales the density, and the pressure by
+            // C^(2g/(g-1)) = C^(2/(g-1)) C^2
+            const double aK = fsqrt(fdiv(g * pK, rK)), igp = frcp(g + 1);
+            const double C = igp * (2.0 + sgn * (g - 1) * fdiv(uK - S, aK));
+            const double w = dpow(C, 2.0 * frcp(g - 1));
+            ro = w * rK;
+            u = (sgn * aK + 0.5 * (g - 1) * uK + S) * (2 * igp);
+            p = w * C * C * pK;
+        }
+        ro = same ? UL[0] : ro;
+        u = same ? uL : u;
+        p = same ? pL : p;
     }
     double Vf[NM];
 #pragma unroll
@@ -835,20 +839,20 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
 #pragma unroll
         for (int i = 0; i < N; i++) Fd[i] = 0.0;
     } else {
-        // the flux of the sampled state (GodunovSolverPerfectGasEOS.h:416-427)
-        double k = 0.0;
+        // the flux of the sampled state (GodunovSolverPerfectGasEOS.h:416-427), with its fused operations
+        // written out: the compiler may form it once for each way here, and has to form the same bits
+#pragma clang fp contract(off)
+        double k = Vf[0] * Vf[0];
 #pragma unroll
-        for (int i = 0; i < NM; i++) k += Vf[i] * Vf[i];
+        for (int i = 1; i < NM; i++) k = __builtin_fma(Vf[i], Vf[i], k);
         const double un = Vf[D];
         Fd[0] = ro * un;
 #pragma unroll
-        for (int i = 0; i < NM; i++) Fd[1 + i] = Fd[0] * Vf[i];
-        Fd[1 + D] += p;
-        Fd[N - 1] = un * (p * frcp(g - 1.0) + 0.5 * ro * k + p);
+        for (int i = 0; i < NM; i++) Fd[1 + i] = i == D ? __builtin_fma(Fd[0], un, p) : Fd[0] * Vf[i];
+        Fd[N - 1] = un * __builtin_fma(0.5 * ro, k, __builtin_fma(p, frcp(g - 1.0), p));
     }
 #pragma unroll
     for (int i = 0; i < N; i++) F[i] = R(Fd[i]);
-    lam = R(st.smax);
 }
 
 // Face eigenvalue only (the dt pass needs no flux).
