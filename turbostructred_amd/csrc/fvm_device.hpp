@@ -464,6 +464,17 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[N], const R (&UR)[
     lam = eig;
 }
 
+// rho |u|^2 / 2 from the momenta, 1 / rho and the velocity along D.  Its range is that of the energy itself: the
+// momenta's squares leave a float's for densities of 1e-21 or 1e21.
+template <int D, typename R, int N>
+__device__ __forceinline__ R kinetic_energy(const R (&u)[N], R ir, R un) {
+    R s = un * u[1 + D];
+#pragma unroll
+    for (int i = 1; i < N - 1; i++)
+        if (i != 1 + D) s += (u[i] * ir) * u[i];
+    return R(0.5) * s;
+}
+
 // HLLC flux (Toro, Riemann Solvers and Numerical Methods for Fluid Dynamics, 3rd ed.,
 // sec. 10.4, eqs. 10.37-10.39) with Davis wave-speed bounds (eq. 10.48); lam = max(|SL|,|SR|).
 // Extension with no counterpart in the reference.  Branch-free: the upwind side K of the contact is
@@ -480,8 +491,7 @@ __device__ inline void hllc_flux(R gamma, const R (&UL)[N], const R (&UR)[N], R 
     const IdealGasEOS<R> eos(gamma);
     const R il = frcp(UL[0]), ir = frcp(UR[0]);
     const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-    const R kl = R(0.5) * il * momentum2(UL);
-    const R kr = R(0.5) * ir * momentum2(UR);
+    const R kl = kinetic_energy<D>(UL, il, ul), kr = kinetic_energy<D>(UR, ir, ur);
     const R pl = eos.PressureOfEnergyDensity(internal_energy(UL[N - 1], kl, UL));
     const R pr = eos.PressureOfEnergyDensity(internal_energy(UR[N - 1], kr, UR));
     const R al = eos.SoundSpeedOfPressure(pl, il), ar = eos.SoundSpeedOfPressure(pr, ir);
@@ -893,8 +903,7 @@ __device__ inline R face_eigen(R gamma, const R (&UL)[N], const R (&UR)[N]) {
         const IdealGasEOS<R> eos(gamma);
         const R il = frcp(UL[0]), ir = frcp(UR[0]);
         const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-        const R kl = R(0.5) * il * momentum2(UL);
-        const R kr = R(0.5) * ir * momentum2(UR);
+        const R kl = kinetic_energy<D>(UL, il, ul), kr = kinetic_energy<D>(UR, ir, ur);
         const R al = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UL[N - 1], kl, UL)), il);
         const R ar = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UR[N - 1], kr, UR)), ir);
         return vmax(vabs(vmin(ul - al, ur - ar)), vabs(vmax(ul + al, ur + ar)));
