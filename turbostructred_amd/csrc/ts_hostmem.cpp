@@ -100,7 +100,7 @@ hipError_t Staging::chunked(char* dst, const char* src, size_t bytes, int device
 }
 
 hipError_t Staging::to_device(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
-    if (bytes < kThreadedUpload || ensure() != hipSuccess) {
+    if (bytes < kThreadedUpload || copy_threads() == 1 || ensure() != hipSuccess) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
     }
@@ -110,7 +110,7 @@ hipError_t Staging::to_device(void* dst, const void* src, size_t bytes, int devi
 }
 
 hipError_t Staging::to_host(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
-    if (bytes < kThreadedCopy || ensure() != hipSuccess) {
+    if (bytes < kThreadedCopy || copy_threads() == 1 || ensure() != hipSuccess) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
     }

@@ -84,7 +84,9 @@ class Staging {
     static constexpr size_t kSlot = size_t(2) << 20;
     static constexpr size_t kBytes = kSlots * kSlot;
     static_assert(kBytes >= 2 * kSmallState);
-    // Both wait until the data are where they go.  On `device`, in the stream's order.
+    // Both wait until the data are where they go.  On `device`, in the stream's order.  Small copies, and all
+    // in a process with few CPUs, are left to the runtime: one thread would take turns with the bus, where the
+    // runtime's own copy of pageable memory overlaps the two.
     hipError_t to_device(void* dst, const void* src, size_t bytes, int device, hipStream_t stream);
     hipError_t to_host(void* dst, const void* src, size_t bytes, int device, hipStream_t stream);
     // `bytes` <= kBytes of the buffer for an asynchronous copy on `stream`: free again after the next wait
