@@ -1,6 +1,7 @@
 """Transfers of states through pinned memory (csrc/ts_hostmem.cpp), built against a stand-in for the HIP
-runtime whose device memory is the host's: every size arrives whole, with many CPUs and with few, where the
-runtime's own copy is used, which overlaps what one thread cannot."""
+runtime whose device memory is the host's: every size arrives whole, with and without pinned memory and with
+many CPUs or few.  Without pinned memory the transfers still work and leave no error behind for the next
+call, and a process with few CPUs uses the runtime's own copy, which overlaps what one thread cannot."""
 import os
 import subprocess
 import textwrap
@@ -101,7 +102,9 @@ def program(tmp_path_factory):
     return str(out)
 
 
+@pytest.mark.parametrize("lacking", ["nothing", "pinned memory", "events"])
 @pytest.mark.parametrize("cpus", [1, 4, 8, 64])
-def test_transfers(program, cpus):
-    r = subprocess.run([program, str(cpus), "0"], capture_output=True, text=True, timeout=120)
+def test_transfers(program, cpus, lacking):
+    which = {"nothing": 0, "pinned memory": 1, "events": 2}[lacking]
+    r = subprocess.run([program, str(cpus), str(which)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr

@@ -41,19 +41,19 @@ void HostArray::release() {
 }
 
 hipError_t Staging::ensure() {
-    if (pin_) return hipSuccess;
-    hipError_t e = hipHostMalloc((void**)&pin_, kBytes, hipHostMallocDefault);
-    if (e != hipSuccess) {
-        pin_ = nullptr;
-        return e;
-    }
-    for (hipEvent_t& ev : ev_)
-        if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) {
-            ev = nullptr;
+    if (buf_) return hipSuccess;
+    pinned_ = hipHostMalloc((void**)&buf_, kBytes, hipHostMallocDefault) == hipSuccess;
+    if (!pinned_) buf_ = nullptr;
+    for (int i = 0; pinned_ && i < kSlots; i++)
+        if (hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming) != hipSuccess) {
+            ev_[i] = nullptr;
             release();
-            return e;
         }
-    return hipSuccess;
+    if (!pinned_) {
+        (void)hipGetLastError();  // handled here: not the next launch's
+        buf_ = (char*)std::malloc(kBytes);
+    }
+    return buf_ ? hipSuccess : hipErrorOutOfMemory;
 }
 
 void Staging::release() {
@@ -61,8 +61,10 @@ void Staging::release() {
         if (ev) (void)hipEventDestroy(ev);
         ev = nullptr;
     }
-    if (pin_) (void)hipHostFree(pin_);
-    pin_ = nullptr;
+    if (buf_ && pinned_) (void)hipHostFree(buf_);
+    else std::free(buf_);
+    buf_ = nullptr;
+    pinned_ = false;
     used_ = 0;
 }
 
@@ -77,7 +79,7 @@ hipError_t Staging::chunked(char* dst, const char* src, size_t bytes, int device
     static_assert(kSlots == 4, "copy_threads gives at most one thread per slot");
     for_chunks(bytes, chunk, copy_threads(), [&](int w, size_t b, size_t e) {
         if (failed.load() != hipSuccess) return;
-        char* slot = pin_ + w * kSlot;
+        char* slot = buf_ + w * kSlot;
         hipError_t r = hipSetDevice(device);
         if (up) {
             if (r == hipSuccess && pending[w]) r = hipEventSynchronize(ev_[w]);
@@ -100,7 +102,7 @@ hipError_t Staging::chunked(char* dst, const char* src, size_t bytes, int device
 }
 
 hipError_t Staging::to_device(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
-    if (bytes < kThreadedUpload || copy_threads() == 1 || ensure() != hipSuccess) {
+    if (bytes < kThreadedUpload || copy_threads() == 1 || ensure() != hipSuccess || !pinned_) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
     }
@@ -110,7 +112,7 @@ hipError_t Staging::to_device(void* dst, const void* src, size_t bytes, int devi
 }
 
 hipError_t Staging::to_host(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
-    if (bytes < kThreadedCopy || copy_threads() == 1 || ensure() != hipSuccess) {
+    if (bytes < kThreadedCopy || copy_threads() == 1 || ensure() != hipSuccess || !pinned_) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
     }
@@ -128,7 +130,7 @@ char* Staging::take(size_t bytes, hipStream_t stream, hipError_t* e) {
         if (*e != hipSuccess) return nullptr;
         used_ = 0;
     }
-    char* p = pin_ + used_;
+    char* p = buf_ + used_;
     used_ += bytes;
     return p;
 }

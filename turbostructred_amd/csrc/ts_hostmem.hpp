@@ -77,7 +77,8 @@ class HostArray {
 };
 
 // A pinned buffer for the transfers of one context or batch, allocated at the first transfer that uses it and
-// freed with its owner.  One thread uses it at a time.
+// freed with its owner.  Where the system has no pinned memory to give, the buffer is an ordinary one: copies
+// through it are slower, and large ones go to the runtime as they are.  One thread uses it at a time.
 class Staging {
    public:
     static constexpr int kSlots = 4;  // one to a thread
@@ -98,7 +99,8 @@ class Staging {
    private:
     hipError_t ensure();
     hipError_t chunked(char* dst, const char* src, size_t bytes, int device, hipStream_t stream, bool up);
-    char* pin_ = nullptr;
+    char* buf_ = nullptr;
+    bool pinned_ = false;
     hipEvent_t ev_[kSlots] = {};
     size_t used_ = 0;
 };
