@@ -21,7 +21,6 @@ sys.path.insert(0, os.path.join(ROOT, "tests"))
 from turbostructred_amd import capi  # noqa: E402
 
 HBM_PEAK = 8.0e12  # MI355X HBM3E, bytes/s
-PLANES_2D = 4 / 5  # a plane flow's kernels leave out one of the five variables that the library counts
 
 
 def lax_liu_state(cfg):
@@ -68,7 +67,7 @@ def gpu_run(n, steps, warmup, precision=capi.FP64, autotune=True):
         if cnt == 0:
             continue
         avg = ms / cnt * 1e-3
-        b = PLANES_2D * s.algorithmic_bytes_per_cell(kind) * ncell
+        b = s.algorithmic_bytes_per_cell(kind) * ncell
         kern[name] = dict(avg_us=avg * 1e6, launches=cnt, algorithmic_bytes=b, achieved_gbs=b / avg / 1e9,
                           frac=b / avg / HBM_PEAK)
     s.enable_kernel_timing(False)
@@ -173,9 +172,9 @@ def viscous_channel(n=2048, steps=40):
             if cnt == 0:
                 continue
             avg = ms / cnt * 1e-3
-            b = PLANES_2D * s.algorithmic_bytes_per_cell(kind) * n * n
+            b = s.algorithmic_bytes_per_cell(kind) * n * n
             kern[name] = dict(avg_us=avg * 1e6, launches=cnt, achieved_gbs=b / avg / 1e9, frac=b / avg / HBM_PEAK)
-        bps = PLANES_2D * s.algorithmic_bytes_per_cell(capi.KIND_ALL)
+        bps = s.algorithmic_bytes_per_cell(capi.KIND_ALL)
         rate = n * n * steps / el
         out["euler" if rk == 1 else "ssp_rk3"] = {
             "cell_updates_per_s": rate, "ms_per_step": el / steps * 1e3, "algorithmic_bytes_per_cell_step": bps,

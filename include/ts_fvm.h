@@ -199,9 +199,12 @@ int ts_get_dt_log(ts_ctx* ctx, double* out, long long capacity, long long* n_out
 int ts_enable_kernel_timing(ts_ctx* ctx, int enable);
 int ts_get_kernel_timing(ts_ctx* ctx, int kind, double* total_ms, long long* launches);
 
-/* Device bytes held by the context and the algorithmic HBM bytes per cell of each kernel
-   kind of ts_get_kernel_timing except 5 (compulsory traffic: one state array = 5*sizeof(real)
-   per cell; with viscous fluxes, 3*ndims velocity gradients and 4 values per face). */
+/* Device bytes held by the context and the algorithmic HBM bytes per cell of one launch of each kernel
+   kind of ts_get_kernel_timing except 5 (4: of a whole step).  Compulsory traffic: one state array =
+   sizeof(real) per cell for each variable that the kernels in use carry, which are 5, or ndims + 2 after
+   ts_set_state has found a 1-D or 2-D flow without momentum out of the grid's axes.  With viscous
+   fluxes in 1-D and 3-D also 3*ndims velocity gradients and 4 values per face, which the pre-pass (kind 6)
+   writes; in 2-D kind 6 counts the stages, whose average it returns. */
 int ts_memory_footprint(const ts_ctx* ctx, size_t* device_bytes);
 int ts_algorithmic_bytes_per_cell(const ts_ctx* ctx, int kind, double* bytes);
 

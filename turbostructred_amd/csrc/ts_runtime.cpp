@@ -385,9 +385,11 @@ int ts_memory_footprint(const ts_ctx* c, size_t* bytes) {
 
 int ts_algorithmic_bytes_per_cell(const ts_ctx* c, int kind, double* bytes) {
     if (!c || !bytes || kind < 0 || kind > 6 || kind == 5) return TS_ERR_INVALID;
-    // one state array = 5 * sizeof(real) per cell; halo re-reads are not counted
-    const double d = 40.0;
-    const double s = c->cfg.precision == TS_FP32_RESIDUAL ? 20.0 : 40.0;
+    // one state array = sizeof(real) per cell and variable that the kernels in use carry; halo
+    // re-reads are not counted
+    const double nv = c->reduced ? c->nd + 2 : TS_NVAR;
+    const double d = 8.0 * nv;
+    const double s = c->cfg.precision == TS_FP32_RESIDUAL ? 4.0 * nv : d;
     double b[5];
     b[0] = d;  // dt pass reads U^n
     if (c->cfg.rk_stages == 1) {
@@ -417,7 +419,10 @@ int ts_algorithmic_bytes_per_cell(const ts_ctx* c, int kind, double* bytes) {
             if (b[k] > 0) b[k] += 32.0 * nd;
         pre = (d + 24.0 * nd) + (d + 24.0 * nd + 32.0 * nd);
     }
-    b[4] = b[0] + b[1] + b[2] + b[3] + pre * (c->cfg.rk_stages == 1 ? 1 : 3);
+    const int stages = c->cfg.rk_stages == 1 ? 1 : 3;
+    b[4] = b[0] + b[1] + b[2] + b[3] + pre * stages;
+    // kind 6 where the stages form the viscous fluxes: those stages, on average
+    if (c->vis && c->cfg.viscous && !c->ks.vpre) pre = (b[1] + b[2] + b[3]) / stages;
     *bytes = kind == 6 ? pre : b[kind];
     return TS_OK;
 }
