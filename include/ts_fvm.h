@@ -272,15 +272,17 @@ typedef struct ts_tile_trial {
 int ts_batch_tuning(ts_batch* b, ts_tile_trial* out, int cap, int* n);
 
 /* Autotuner: time the candidate tile heights for cfg's kernel family at cfg's size (the
-   occupancy-model choice, its neighbours and 4..64 rows) and store the winner in the
-   process-wide tuning table used by later ts_create calls.  Results never depend on it. */
+   occupancy-model choice, its neighbours and 1..64 rows) and store the winner in the
+   process-wide tuning table used by later ts_create calls.  The table is kept apart for the kernels with
+   every variable and those of 1-D and 2-D flows within the grid's axes; this call serves both, as far as
+   ts_autotune_state has not tuned them.  Results never depend on it. */
 int ts_autotune(const ts_config* cfg, int* chosen_rows_per_tile, double* best_ms);
 
 /* The same autotuner timed on the caller's own state (the reference AoS layout, n_doubles =
    ts_state_size of cfg's context; NULL = the quiescent state of ts_autotune) over `steps` steps
    per candidate, so that data-dependent cost (the exact solver's Newton iterations, limiter
    branches) counts.  Up to `cap` candidates are reported as (rows per tile, kernel ms per step);
-   the winner is stored in the table and returned in *chosen. */
+   the winner is stored in the table, for the kernels that this state runs, and returned in *chosen. */
 int ts_autotune_state(const ts_config* cfg, const double* aos_state, size_t n_doubles, int steps,
                       int* cand_rows_per_tile, double* cand_ms_per_step, int cap, int* n_cand,
                       int* chosen_rows_per_tile);

@@ -2,7 +2,8 @@
 //
 // The only free tiling parameter of the marching kernels is the number of output rows per tile
 // (cells per thread along the march).  Results never depend on it: every cell's arithmetic is
-// the same whatever the tiling, so the table may be keyed by problem size alone.
+// the same whatever the tiling, so the table may be keyed by problem size, and by which kernels run: those
+// with every variable or those of a flow within the grid's axes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -15,7 +16,8 @@
 #include "ts_internal.hpp"
 
 namespace {
-using Key = std::tuple<int, int, int, int, int, int>;  // nd, riemann, recon variant, precision, stages, size bucket
+// nd, riemann, recon variant, precision, stages, size bucket, reduced kernels
+using Key = std::tuple<int, int, int, int, int, int, bool>;
 std::mutex g_mu;
 std::map<Key, int> g_table;
 
@@ -26,8 +28,8 @@ int size_bucket(const ts_config& c) {
     return b;
 }
 
-Key key_of(const ts_config& c) {
-    return Key(c.ndims, c.riemann, tsr::recon_variant(c), c.precision, c.rk_stages, size_bucket(c));
+Key key_of(const ts_config& c, bool reduced) {
+    return Key(c.ndims, c.riemann, tsr::recon_variant(c), c.precision, c.rk_stages, size_bucket(c), reduced);
 }
 }  // namespace
 
@@ -45,11 +47,11 @@ double march_cost(long long tiles, int ty, long long units, int occ) {
     return c * (ty + 2);
 }
 
-int tuned_rows_per_tile(const ts_config& c, int zout, long long units, int occ) {
+int tuned_rows_per_tile(const ts_config& c, bool reduced, int zout, long long units, int occ) {
     if (c.ndims == 1) return 1;
     {
         std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_table.find(key_of(c));
+        auto it = g_table.find(key_of(c, reduced));
         if (it != g_table.end()) return it->second;
     }
     const long long strips = (c.nx + 59) / 60;
@@ -86,13 +88,8 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
         if (best_ms) *best_ms = 0;
         return TS_OK;
     }
-    // the occupancy model's choice (with no table entry) and its neighbours, the heights at which
-    // the tiles just fit one and two rounds of the resident slots, then fixed heights
-    {
-        std::lock_guard<std::mutex> lk(g_mu);
-        g_table.erase(key_of(*cfg));
-    }
     const size_t nst = ts_state_size_cfg(cfg);
+    const bool any_state = !aos;
     std::vector<double> quiet;
     if (!aos) {
         // a quiescent uniform state: the arithmetic of the flux kernels barely depends on the data
@@ -103,6 +100,23 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
         }
         aos = quiet.data();
     }
+    // the kernels that the state runs, and the table entry that is tuned
+    bool reduced = false;
+    {
+        ts_ctx* c = nullptr;
+        if (ts_create(cfg, &c) == TS_OK) {
+            (void)ts_set_state(c, aos, nst);
+            reduced = c->reduced;
+            ts_destroy(c);
+        }
+    }
+    const Key key = key_of(*cfg, reduced);
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_table.erase(key);
+    }
+    // the occupancy model's choice (with no table entry) and its neighbours, the heights at which
+    // the tiles just fit one and two rounds of the resident slots, then fixed heights
     std::vector<int> cands;
     {
         ts_ctx* c = nullptr;
@@ -135,7 +149,7 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
     for (int ty : uniq) {
         {
             std::lock_guard<std::mutex> lk(g_mu);
-            g_table[key_of(*cfg)] = ty;
+            g_table[key] = ty;
         }
         ts_ctx* c = nullptr;
         if (ts_create(cfg, &c) != TS_OK) continue;
@@ -166,10 +180,12 @@ int autotune_impl(const ts_config* cfg, const double* aos, size_t n_doubles, int
     if (n_cand) *n_cand = std::min(k, cap);
     std::lock_guard<std::mutex> lk(g_mu);
     if (best < 0) {
-        g_table.erase(key_of(*cfg));
+        g_table.erase(key);
         return TS_ERR_UNSUPPORTED;
     }
-    g_table[key_of(*cfg)] = best;
+    g_table[key] = best;
+    // without a state of the caller's, also for the other kernels, unless they have been tuned
+    if (any_state) g_table.emplace(key_of(*cfg, !reduced), best);
     if (chosen) *chosen = best;
     if (best_ms) *best_ms = bms;
     return TS_OK;

@@ -116,7 +116,7 @@ bool boundaries_in_grid(const ts_config& c);
 void host_bc_image(const ts_bc_config& bc, double g, int axis, const double* u, double* o);
 // output rows per tile of `zout` planes (1 below 3-D); the GPU holds `occ` tiles on each of `units`
 // SIMDs (3-D: CUs) at once (0: unknown)
-int tuned_rows_per_tile(const ts_config& c, int zout, long long units, int occ);
+int tuned_rows_per_tile(const ts_config& c, bool reduced, int zout, long long units, int occ);
 // modelled time of marching `tiles` tiles of ty rows
 double march_cost(long long tiles, int ty, long long units, int occ);
 // the calling thread's error text for entry points without a context (ts_last_error(NULL))

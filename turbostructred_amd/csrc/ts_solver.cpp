@@ -67,13 +67,13 @@ constexpr int CHUNK = 256;  // steps issued between host checks of the terminati
 
 // Tiling of one kernel variant: output rows per tile for the CUs of the device and the resident
 // workgroups per CU of its kernels, tiles and grid.
-void tile_variant(const ts_ctx* c, const ts_config& cfg, ts_ctx::Variant& v) {
+void tile_variant(const ts_ctx* c, const ts_config& cfg, bool reduced, ts_ctx::Variant& v) {
     const int per_block = c->nd == 3 ? 1 : 4;  // 1-D, 2-D: a tile (1-D: a strip) per wavefront, four to a block
     const int real = cfg.precision == TS_FP64 ? 8 : 4, zout = c->nd > 2 ? z_out_of(real, false) : 1;
     int cus = 0, occ = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device) == hipSuccess && v.ks.socc) occ = v.ks.socc();
-    v.ty = tsr::tuned_rows_per_tile(cfg, zout, (long long)cus * per_block, occ);
-    v.ty2 = c->nd > 2 ? tsr::tuned_rows_per_tile(cfg, z_out_of(real, true), cus, occ) : v.ty;
+    v.ty = tsr::tuned_rows_per_tile(cfg, reduced, zout, (long long)cus * per_block, occ);
+    v.ty2 = c->nd > 2 ? tsr::tuned_rows_per_tile(cfg, reduced, z_out_of(real, true), cus, occ) : v.ty;
     const int nyb = c->nd > 1 ? (c->n[1] + v.ty - 1) / v.ty : 1;
     const int nzb = (c->n[2] + zout - 1) / zout;
     v.ntiles = c->nstrips * nyb * nzb;
@@ -232,7 +232,7 @@ int init_device_ctx(ts_ctx* c, const ts_config* cfg) {
     c->may_reduce = !c->arena && (c->vis ? c->nd == 2 && sources_in_grid : k.rk_stages == 1 || c->fused_dt) && tsr::boundaries_in_grid(k) &&
                     tsr::lookup_kernels(c->nd, k.riemann, tsr::recon_variant(k), k.precision, true, &c->variant[1].ks);
     for (int i = 0; i < (c->may_reduce ? 2 : 1); i++) {
-        tile_variant(c, *cfg, c->variant[i]);
+        tile_variant(c, *cfg, i == 1, c->variant[i]);
         c->most_blocks = std::max(c->most_blocks, (size_t)c->variant[i].grid_dim.x);
     }
     // one minimum of V/SR per workgroup from every dt pass and fused stage 1
