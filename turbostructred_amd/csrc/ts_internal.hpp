@@ -52,6 +52,7 @@ struct ts_ctx {
     };
     Variant variant[2];
     bool may_reduce = false, reduced = false;
+    bool other_clear = false;  // the planes that the reduced kernels leave out are zero in dU[1]
     size_t most_blocks = 1;  // of the variants' grids
     tsd::KernelSet ks;
     int ty = 16, ty2 = 16;  // rows per tile (ty2: 3-D stage 2)
@@ -113,6 +114,8 @@ void venkat_axis_factors(int nd, int n, const double* h, std::vector<double>& ou
 bool lookup_kernels(int dim, int flux, int rv, int precision, bool in_grid, tsd::KernelSet* ks);
 // whether no boundary condition of the table can give momentum out of the grid's axes (1-D, 2-D)
 bool boundaries_in_grid(const ts_config& c);
+// whether no interior cell of a 1-D or 2-D state (the reference AoS layout) has such momentum
+bool state_in_grid(const double* aos, int nd, const int n[3]);
 void host_bc_image(const ts_bc_config& bc, double g, int axis, const double* u, double* o);
 // output rows per tile of `zout` planes (1 below 3-D); the GPU holds `occ` tiles on each of `units`
 // SIMDs (3-D: CUs) at once (0: unknown)

@@ -254,11 +254,13 @@ int drop_graphs(ts_ctx* c) {
 }
 
 int use_variant(ts_ctx* c, bool reduced) {
-    if (reduced && c->cfg.rk_stages == 1) {
+    if (!reduced) c->other_clear = false;
+    if (reduced && c->cfg.rk_stages == 1 && !c->other_clear) {
         // forward Euler ping-pongs: the planes that the kernels leave out are zero in the other
         // buffer too (SSP-RK3 updates U^n in place)
         const size_t first = 1 + c->nd;
         CHK(hipMemsetAsync((double*)c->dU[1] + first * c->ncell, 0, (4 - first) * c->ncell * sizeof(double), c->stream));
+        c->other_clear = true;
     }
     const ts_ctx::Variant& v = c->variant[reduced];
     if (reduced != c->reduced) {
