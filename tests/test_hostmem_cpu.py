@@ -23,7 +23,7 @@ enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
 enum { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2, hipHostMallocDefault = 0, hipEventDisableTiming = 2 };
 inline thread_local int last_error = 0;
 inline bool no_pinned = false, no_events = false;
-inline std::atomic<int> copies{0}, pinned{0};
+inline std::atomic<int> copies{0}, pinned{0}, waits{0};
 inline hipError_t done(int e) { if (e) last_error = e; return e; }
 inline hipError_t hipGetLastError() { int e = last_error; last_error = 0; return e; }
 inline hipError_t hipSetDevice(int) { return 0; }
@@ -39,7 +39,7 @@ inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
 inline hipError_t hipEventDestroy(hipEvent_t e) { std::free(e); return 0; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return 0; }
 inline hipError_t hipEventSynchronize(hipEvent_t) { return 0; }
-inline hipError_t hipStreamSynchronize(hipStream_t) { return 0; }
+inline hipError_t hipStreamSynchronize(hipStream_t) { waits++; return 0; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
     copies++; std::memcpy(d, s, n); return 0;
 }
@@ -62,9 +62,10 @@ int main(int, char** argv) {
         tsr::Staging st;
         std::vector<uint64_t> a(n / 8), b(n / 8), c(n / 8);
         for (size_t i = 0; i < a.size(); i++) a[i] = i * 0x9E3779B97F4A7C15u;
-        copies = 0;
+        copies = waits = 0;
         REQUIRE(st.to_device(b.data(), a.data(), n, 0, nullptr) == hipSuccess);
         const int up = copies.exchange(0);
+        REQUIRE(up > 1 || waits == 0);   // the caller waits, once, for what follows the copy
         REQUIRE(st.to_host(c.data(), b.data(), n, 0, nullptr) == hipSuccess);
         const int down = copies.exchange(0);
         REQUIRE(a == b && a == c);

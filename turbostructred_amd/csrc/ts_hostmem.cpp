@@ -103,8 +103,7 @@ hipError_t Staging::chunked(char* dst, const char* src, size_t bytes, int device
 
 hipError_t Staging::to_device(void* dst, const void* src, size_t bytes, int device, hipStream_t stream) {
     if (bytes < kThreadedUpload || copy_threads() == 1 || ensure() != hipSuccess || !pinned_) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
-        return e != hipSuccess ? e : hipStreamSynchronize(stream);
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
     }
     const hipError_t e = used_ ? hipStreamSynchronize(stream) : hipSuccess;  // what take() handed out
     used_ = 0;

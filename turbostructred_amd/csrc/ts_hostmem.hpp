@@ -85,7 +85,8 @@ class Staging {
     static constexpr size_t kSlot = size_t(2) << 20;
     static constexpr size_t kBytes = kSlots * kSlot;
     static_assert(kBytes >= 2 * kSmallState);
-    // Both wait until the data are where they go.  On `device`, in the stream's order.  Small copies, and all
+    // On `device`, in the stream's order.  to_host waits until the data are there; to_device may return before
+    // they are, and the caller keeps `src` until it has waited for the stream.  Small copies, and all
     // in a process with few CPUs, are left to the runtime: one thread would take turns with the bus, where the
     // runtime's own copy of pageable memory overlaps the two.
     hipError_t to_device(void* dst, const void* src, size_t bytes, int device, hipStream_t stream);
