@@ -22,12 +22,25 @@ constexpr int NV = 5;
 template <int N>
 __device__ __host__ constexpr int plane_of(int v) { return v == N - 1 ? NV - 1 : v; }
 
+// Sums over the components are written with explicit fused operations: left to itself the compiler chooses
+// which products of a sum it fuses, and chose differently for three components than for two.
+__device__ inline double madd(double a, double b, double s) { return __builtin_fma(a, b, s); }
+__device__ inline float madd(float a, float b, float s) { return __builtin_fmaf(a, b, s); }
+template <typename R, int M>
+__device__ __forceinline__ R dot(const R (&a)[M], const R (&b)[M]) {
+#pragma clang fp contract(off)
+    R s = a[0] * b[0];
+#pragma unroll
+    for (int i = 1; i < M; i++) s = madd(a[i], b[i], s);
+    return s;
+}
 // |momentum|^2
 template <typename R, int N>
 __device__ __forceinline__ R momentum2(const R (&u)[N]) {
+#pragma clang fp contract(off)
     R s = u[1] * u[1];
 #pragma unroll
-    for (int i = 2; i < N - 1; i++) s += u[i] * u[i];
+    for (int i = 2; i < N - 1; i++) s = madd(u[i], u[i], s);
     return s;
 }
 
@@ -367,22 +380,20 @@ enum : int { FX_GODUNOV = 0, FX_ROE = 1, FX_HLLC = 3 };
 // Internal energy density E - rho|v|^2/2 from the conserved state.  In the FP32 form the
 // difference is redone in double when it is a small part of E (near vacuum, where the float
 // subtraction loses most of its digits).
-__device__ inline double internal_energy(double E, double rho_ke) { return E - rho_ke; }
 template <int N>
-__device__ inline float internal_energy(float E, float rho_ke, const float (&U)[N]) {
-    float e = E - rho_ke;
-    if (e < 0.01f * E) {
+__device__ inline float checked_energy(float e, const float (&U)[N]) {
+    if (e < 0.01f * U[N - 1]) {
         double m2 = double(U[1]) * U[1];
 #pragma unroll
-        for (int i = 2; i < N - 1; i++) m2 += double(U[i]) * U[i];
+        for (int i = 2; i < N - 1; i++) m2 = __builtin_fma(double(U[i]), double(U[i]), m2);
         e = float(double(U[N - 1]) - 0.5 * m2 / double(U[0]));
     }
     return e;
 }
 template <int N>
-__device__ inline double internal_energy(double E, double rho_ke, const double (&)[N]) {
-    return E - rho_ke;
-}
+__device__ inline double checked_energy(double e, const double (&)[N]) { return e; }
+template <typename R, int N>
+__device__ inline R internal_energy(R E, R rho_ke, const R (&U)[N]) { return checked_energy(E - rho_ke, U); }
 
 // Roe-Pike flux with Harten's entropy fix (RoeSolverPerfectGasEOS.h:48-134) across a face with
 // normal +e_D.  lam receives |u.n| + c of the Roe average (RoeSolverPerfectGasEOS.h:88,128).
@@ -393,16 +404,12 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[N], const R (&UR)[
     const R gm1 = gamma - R(1);
     R il = frcp(UL[0]), ir = frcp(UR[0]);
     R vl[NM], vr[NM];
-    R kl = R(0), kr = R(0);
 #pragma unroll
     for (int i = 0; i < NM; i++) {
         vl[i] = UL[1 + i] * il;
         vr[i] = UR[1 + i] * ir;
-        kl += vl[i] * vl[i];
-        kr += vr[i] * vr[i];
     }
-    kl *= R(0.5);
-    kr *= R(0.5);
+    const R kl = R(0.5) * dot(vl, vl), kr = R(0.5) * dot(vr, vr);
     R el = UL[N - 1] * il, er = UR[N - 1] * ir;
     // physical fluxes (RoeSolverPerfectGasEOS.h:15-32)
     R pl = gm1 * internal_energy(UL[N - 1], UL[0] * kl, UL);
@@ -413,14 +420,9 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[N], const R (&UR)[
     R isum = frcp(sl + sr);
     R ql = sl * isum, qr = sr * isum;
     R v[NM];
-    R vv = R(0), vvl = R(0), vvr = R(0);
 #pragma unroll
-    for (int i = 0; i < NM; i++) {
-        v[i] = ql * vl[i] + qr * vr[i];
-        vv += v[i] * v[i];
-        vvl += v[i] * vl[i];
-        vvr += v[i] * vr[i];
-    }
+    for (int i = 0; i < NM; i++) v[i] = ql * vl[i] + qr * vr[i];
+    const R vv = dot(v, v), vvl = dot(v, vl), vvr = dot(v, vr);
     R h = ql * hl + qr * hr;
     R phi2 = R(0.5) * gm1 * vv;
     R c = fsqrt(gm1 * h - phi2);
@@ -464,15 +466,18 @@ __device__ inline void roe_flux(R gamma, R eps, const R (&UL)[N], const R (&UR)[
     lam = eig;
 }
 
-// rho |u|^2 / 2 from the momenta, 1 / rho and the velocity along D.  Its range is that of the energy itself: the
-// momenta's squares leave a float's for densities of 1e-21 or 1e21.
+// The same from the momenta, 1 / rho and the velocity along D, with rho |u|^2 formed as momentum times velocity:
+// its range is that of the energy itself, where the momenta's squares leave a float's for densities of
+// 1e-21 or 1e21.
 template <int D, typename R, int N>
-__device__ __forceinline__ R kinetic_energy(const R (&u)[N], R ir, R un) {
+__device__ __forceinline__ R internal_energy_along(const R (&u)[N], R ir, R un) {
+#pragma clang fp contract(off)
     R s = un * u[1 + D];
 #pragma unroll
     for (int i = 1; i < N - 1; i++)
-        if (i != 1 + D) s += (u[i] * ir) * u[i];
-    return R(0.5) * s;
+        if (i != 1 + D) s = madd(u[i] * ir, u[i], s);
+    const R e = madd(R(-0.5), s, u[N - 1]);
+    return checked_energy(e, u);
 }
 
 // HLLC flux (Toro, Riemann Solvers and Numerical Methods for Fluid Dynamics, 3rd ed.,
@@ -488,27 +493,29 @@ __device__ __forceinline__ R kinetic_energy(const R (&u)[N], R ir, R un) {
 template <int D, typename R, int N>
 __device__ inline void hllc_flux(R gamma, const R (&UL)[N], const R (&UR)[N], R (&F)[N],
                                  R& lam) {
+    // every fused operation is written out, so that a plane flow's kernels and those with all variables, and
+    // the dt pass, form the same bits
+#pragma clang fp contract(off)
     const IdealGasEOS<R> eos(gamma);
     const R il = frcp(UL[0]), ir = frcp(UR[0]);
     const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-    const R kl = kinetic_energy<D>(UL, il, ul), kr = kinetic_energy<D>(UR, ir, ur);
-    const R pl = eos.PressureOfEnergyDensity(internal_energy(UL[N - 1], kl, UL));
-    const R pr = eos.PressureOfEnergyDensity(internal_energy(UR[N - 1], kr, UR));
+    const R pl = eos.PressureOfEnergyDensity(internal_energy_along<D>(UL, il, ul));
+    const R pr = eos.PressureOfEnergyDensity(internal_energy_along<D>(UR, ir, ur));
     const R al = eos.SoundSpeedOfPressure(pl, il), ar = eos.SoundSpeedOfPressure(pr, ir);
     const R SL = vmin(ul - al, ur - ar);
     const R SR = vmax(ul + al, ur + ar);
     lam = vmax(vabs(SL), vabs(SR));
     const R wl = SL - ul, wr = SR - ur;
     const R ml = UL[0] * wl, mr = UR[0] * wr;
-    const R Ss = fdiv(pr - pl + ul * ml - ur * mr, ml - mr);
+    const R Ss = fdiv(madd(-ur, mr, madd(ul, ml, pr - pl)), ml - mr);
     const bool left = Ss >= R(0);
     const R S = left ? SL : SR, w = left ? wl : wr, m = left ? ml : mr;
     const R rho = left ? UL[0] : UR[0], un = left ? ul : ur, p = left ? pl : pr, E = left ? UL[N - 1] : UR[N - 1];
     const bool supersonic = left ? (S >= R(0)) : (S <= R(0));
     // on a subsonic side S - S* is not zero (S < 0 <= S*, or the mirror case)
     const R r = frcp(supersonic ? R(1) : S - Ss);
-    const R ps = p + m * (Ss - un);
-    const R Es = (w * E - p * un + ps * Ss) * r;
+    const R ps = madd(m, Ss - un, p);
+    const R Es = madd(ps, Ss, madd(w, E, -(p * un))) * r;
     const R c = supersonic ? R(1) : w * r;
     const R uf = supersonic ? un : Ss, pf = supersonic ? p : ps, Ef = supersonic ? E : Es;
     const R q = c * uf;
@@ -516,7 +523,7 @@ __device__ inline void hllc_flux(R gamma, const R (&UL)[N], const R (&UR)[N], R 
 #pragma unroll
     for (int i = 1; i < N - 1; i++)
         if (i != 1 + D) F[i] = (left ? UL[i] : UR[i]) * q;
-    F[1 + D] = F[0] * uf + pf;
+    F[1 + D] = madd(F[0], uf, pf);
     F[N - 1] = uf * (Ef + pf);
 }
 
@@ -766,14 +773,12 @@ __device__ inline void godunov_flux(R gammaR, const R (&ULr)[N], const R (&URr)[
     for (int i = 0; i < N; i++) { UL[i] = double(ULr[i]); UR[i] = double(URr[i]); }
     const double il = frcp(UL[0]), ir = frcp(UR[0]);
     double vL[NM], vR[NM];
-    double kL = 0.0, kR = 0.0;
 #pragma unroll
     for (int i = 0; i < NM; i++) {
         vL[i] = UL[1 + i] * il;
         vR[i] = UR[1 + i] * ir;
-        kL += vL[i] * vL[i];
-        kR += vR[i] * vR[i];
     }
+    const double kL = dot(vL, vL), kR = dot(vR, vR);
     double pL = eos.GetPressure(UL[0], UL[N - 1] * il - kL / 2.0);
     double pR = eos.GetPressure(UR[0], UR[N - 1] * ir - kR / 2.0);
     double uL = vL[D], uR = vR[D];
@@ -874,38 +879,31 @@ __device__ inline R face_eigen(R gamma, const R (&UL)[N], const R (&UR)[N]) {
         const R gm1 = gamma - R(1);
         R il = frcp(UL[0]), ir = frcp(UR[0]);
         R vl[NM], vr[NM];
-        R kl = R(0), kr = R(0);
 #pragma unroll
         for (int i = 0; i < NM; i++) {
             vl[i] = UL[1 + i] * il;
             vr[i] = UR[1 + i] * ir;
-            kl += vl[i] * vl[i];
-            kr += vr[i] * vr[i];
         }
-        kl *= R(0.5);
-        kr *= R(0.5);
+        const R kl = R(0.5) * dot(vl, vl), kr = R(0.5) * dot(vr, vr);
         R hl = (UL[N - 1] * il - kl) * gamma + kl;
         R hr = (UR[N - 1] * ir - kr) * gamma + kr;
         R sl = fsqrt(UL[0]), sr = fsqrt(UR[0]);
         R isum = frcp(sl + sr);
         R ql = sl * isum, qr = sr * isum;
-        R vv = R(0), vn = R(0);
+        R v[NM];
 #pragma unroll
-        for (int i = 0; i < NM; i++) {
-            const R v = ql * vl[i] + qr * vr[i];
-            vv += v * v;
-            if (i == D) vn = v;
-        }
+        for (int i = 0; i < NM; i++) v[i] = ql * vl[i] + qr * vr[i];
+        const R vv = dot(v, v), vn = v[D];
         R h = ql * hl + qr * hr;
         R phi2 = R(0.5) * gm1 * vv;
         return __builtin_fabs(vn) + fsqrt(gm1 * h - phi2);
     } else if constexpr (FLUX == FX_HLLC) {
+#pragma clang fp contract(off)
         const IdealGasEOS<R> eos(gamma);
         const R il = frcp(UL[0]), ir = frcp(UR[0]);
         const R ul = UL[1 + D] * il, ur = UR[1 + D] * ir;
-        const R kl = kinetic_energy<D>(UL, il, ul), kr = kinetic_energy<D>(UR, ir, ur);
-        const R al = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UL[N - 1], kl, UL)), il);
-        const R ar = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy(UR[N - 1], kr, UR)), ir);
+        const R al = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy_along<D>(UL, il, ul)), il);
+        const R ar = eos.SoundSpeedOfPressure(eos.PressureOfEnergyDensity(internal_energy_along<D>(UR, ir, ur)), ir);
         return vmax(vabs(vmin(ul - al, ur - ar)), vabs(vmax(ul + al, ur + ar)));
     } else {
         R F[N], lam;
