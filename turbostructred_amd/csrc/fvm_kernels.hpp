@@ -38,8 +38,10 @@ namespace tsd {
 enum : int { MODE_DT = 0, MODE_S1 = 1, MODE_S2 = 2, MODE_S3 = 3, MODE_F1 = 4, MODE_F2 = 5, MODE_RN = 6 };
 constexpr int STRIP = 60;   // output columns per wavefront
 // Wavefronts (z-planes) per 3-D workgroup; all but two produce output.  In double, whose kernels
-// hold about 200 registers, a SIMD takes two.  In float four fit, but stage 2 then spills 15 registers
-// of its two prefetched rows: three (256^3: 899 us against 1078 with four).
+// hold 200 to 250 registers, a SIMD takes two.  In float four fit, with a few registers spilled (HLLC: up to 4
+// of 128 with Barth-Jespersen and 20 with the other reconstructions; Roe: 25 and 37; the exact solver,
+// which works in double, more than a hundred), but stage 2 then spills 15 more of its two
+// prefetched rows: three (256^3: 899 us against 1078 with four).
 template <typename R, int VIS, int MODE>
 constexpr int z_waves = sizeof(R) == 8 ? 8 : (MODE == MODE_F2 ? 12 : 16);
 // output planes of stage 2 and of the others (which set the number of dt minima)
@@ -1329,8 +1331,8 @@ __global__ void __launch_bounds__(64 * wg1d_waves<FLUX>) fvm_euler1d_workgroup(K
 // no claim atomics, which serialise at one address at tens of ns each, and every wavefront's
 // loop ends after at most ceil(ntiles / W) tiles.  Neighbouring wavefront ids sit on one XCD, so
 // neighbouring tiles of a problem share an L2.  Stage 1 stores each table entry's wavefront-level
-// minimum of V/SR in `part` (by entry), and dt_finalize_batched turns each problem's entries into
-// its dt.  A cell's arithmetic depends only on its own problem, and the minimum is exact, so a
+// minimum of V/SR in `part` (by entry), and dt_finalize_batched or stage 2 turns each problem's entries
+// into its dt.  A cell's arithmetic depends only on its own problem, and the minimum is exact, so a
 // result is the same alone or in a mix.
 
 template <int DIM, int RECON, int LIM, int FLUX, int MODE, typename R, typename TIn, typename TOut, int N = NV>
