@@ -44,9 +44,10 @@ __global__ void __launch_bounds__(64 * (z_waves<R, VIS, MODE>)) fvm_stage3d(KArg
     // fluxes through its faces below, in y and z.  In double all 15 values fit into the registers with the
     // HLLC flux (247 of 256 at most; 256^3 step 2.96 ms, 3.04 with the x part in LDS, 3.16 with
     // none) and with Roe's, whose stage 2 spills little (128^3 611 us, 637 with the x part in LDS) but for
-    // ENO2 (650 against 631); the exact solver and the float kernels would spill.
-    constexpr bool X_REGS = sizeof(R) == 8 && (FLUX == FX_HLLC || (FLUX == FX_ROE && RECON != RC_ENO2));
-    constexpr bool YZ_REGS = sizeof(R) == 8 && FLUX != FX_GODUNOV;
+    // ENO2 (650 against 631), and in first order also with the exact solver (128^3 step 1137 us, 1189 in LDS);
+    // with a reconstruction that one and the float kernels would spill.
+    constexpr bool X_REGS = sizeof(R) == 8 && (FLUX == FX_HLLC || RECON == RC_PWC || (FLUX == FX_ROE && RECON != RC_ENO2));
+    constexpr bool YZ_REGS = sizeof(R) == 8 && (FLUX != FX_GODUNOV || RECON == RC_PWC);
     __shared__ R carry_x[MT::flux && !X_REGS ? ZW : 1][NV][64];
     __shared__ R carry_y[MT::flux && !YZ_REGS ? ZW : 1][NV][64];
     __shared__ R lds_h[MT::flux ? ZW : 1][NV][64];     // flux through the z-face below every plane
